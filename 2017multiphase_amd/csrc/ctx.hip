@@ -119,7 +119,7 @@ void free_all(Ctx& c) {
   dfree(c.phifluid); dfree(c.phiair); dfree(c.phisolid); dfree(c.ctmp); dfree(c.sf);
   dfree(c.div); dfree(c.press); dfree(c.tp); dfree(c.tpchange); dfree(c.tsave);
   dfree(c.vx); dfree(c.vr); dfree(c.vp); dfree(c.vq); dfree(c.vp2); dfree(c.vr2); dfree(c.vq2); dfree(c.vp3); dfree(c.nbm); dfree(c.dslow);
-  dfree(c.partials); dfree(c.scal); dfree(c.counters);
+  dfree(c.partials); dfree(c.scal); dfree(c.counters); dfree(c.res_buf);
   for (int a = 0; a < 3; ++a) {
     dfree(c.wu[a]); dfree(c.au[a]); dfree(c.wuo[a]); dfree(c.auo[a]); dfree(c.su[a]); dfree(c.ftmp[a]);
   }
@@ -192,6 +192,15 @@ bool alloc_all(Ctx& c) {
   ok = ok && dalloc(c, c.nbm, G) && dalloc(c, c.dslow, G);
   c.npart = 1024 * 48;  // solver partial sums (pcg.hip lays out regions of 1024-block slots)
   ok = ok && dalloc(c, c.partials, c.npart) && dalloc(c, c.scal, 1) && dalloc(c, c.counters, NCOUNTERS);
+  if (ok) {  // one block per CU
+    int cus = 0, coop = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device) == hipSuccess &&
+        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c.device) == hipSuccess && coop) {
+      c.res_blocks = cus < resident_most_blocks() ? cus : resident_most_blocks();
+      const int64_t words = resident_words(c.g, c.res_blocks, &c.res_cells);
+      if (words > 0) ok = dalloc(c, c.res_buf, (size_t)words);
+    }
+  }
   for (int a = 0; a < 3 && ok; ++a)
     ok = ok && dalloc(c, c.wu[a], fc[a]) && dalloc(c, c.au[a], fc[a]) && dalloc(c, c.wuo[a], fc[a]) &&
          dalloc(c, c.auo[a], fc[a]) && dalloc(c, c.su[a], fc[a]) && dalloc(c, c.ftmp[a], fc[a]);

@@ -115,6 +115,8 @@ struct SolveScalars {
   int last_true;  // MIXED: update index whose residual the last executed true-residual pass replaced (-1 none)
   int done_k;     // single-kernel iteration: the k of the launch that set done
   float alh[2];   // single-kernel iteration: the alpha launch k applied, in slot k&1
+  uint32_t res_seq;              // resident solve: number of the next meeting
+  int res_missed, res_restarts;  // resident solve: the true residual missed the tolerance; restarts from it
 };
 
 struct KernelStat {
@@ -182,6 +184,13 @@ struct Ctx {
   double* vx64 = nullptr;
   double* partials = nullptr;
   int npart = 0;
+  // resident solve (null when the grid does not fit): records, then six halo
+  // arrays of res_cells words; res_blocks blocks can be resident together;
+  // number of the next meeting (0: clear the words first)
+  uint64_t* res_buf = nullptr;
+  int64_t res_cells = 0;
+  int res_blocks = 0;
+  uint32_t res_seq = 0;
   SolveScalars* scal = nullptr;
   SolveScalars* scal_host = nullptr;  // pinned
   uint32_t* counters = nullptr;       // [0] reduction arrival, [1..63] misc counters, then spread counters
@@ -325,6 +334,8 @@ inline int64_t nbricks(const Grid& g) {
 // pcg.hip
 int run_pressure_solve(Ctx& c, mpf_solve_info* info);
 int run_heat_cg(Ctx& c, mpf_solve_info* info);
+int64_t resident_words(const Grid& g, int blocks, int64_t* cells);
+int resident_most_blocks();
 int run_adjoint_solve(Ctx& c, const double* rhs, double* sol, mpf_solve_info* info);
 // adjoint.hip
 bool adj_alloc_all(Ctx& c);

@@ -32,6 +32,7 @@
 // are dispatched round-robin over the 8 XCDs) walks one contiguous slab.
 #include "mpf_internal.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace mpf {
@@ -1981,6 +1982,8 @@ bool read_scalars(Ctx& c) {
   return hip_ok(c, hipStreamSynchronize(c.stream), "solver poll");
 }
 
+#include "cg_resident.inl"
+
 // Generic (P)CG driver.  V: vector type, Dacc: dot accumulation type.
 // b: right-hand side (type V), x: solution (type V; MIXED adds x64).
 // MIXED: after every refine_every iterations the FP64 true residual replaces
@@ -2001,6 +2004,51 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
   int check = mixed ? R : c.cfg.check_every;
   if (check <= 0) check = 16;
   launch(c, "pcg_nbm", dim3(nblocks(G, 256)), dim3(256), 0, k_nbm<OPk, V>, o, c.nbm, (V*)c.dslow);
+  auto report = [&](bool true_missed, int restarts) -> int {
+    const SolveScalars& s = *c.scal_host;
+    const bool converged = s.converged && !true_missed;
+    if (info) {
+      info->iterations = s.iter;
+      info->refinements = s.refinements;
+      info->converged = converged ? 1 : 0;
+      info->rel_residual = s.bb > 0 ? sqrt(s.rr_true) / sqrt(s.bb) : 0.0;
+      info->abs_rr = s.rr;
+    }
+    if (s.nonfinite) {
+      c.err = "non-finite value in the solver";
+      return MPF_NONFINITE;
+    }
+    if (true_missed)
+      c.note = "mixed-precision solve: the FP64 true residual missed the tolerance (" + std::to_string(restarts) +
+               " restarts, iteration " + std::to_string(s.iter) + ")";
+    return converged ? MPF_OK : MPF_NO_CONVERGENCE;
+  };
+  // |b - A x|^2 in FP64 for the report
+  auto true_rr = [&]() -> bool {
+    if (mixed)
+      launch(c, "pcg_true_resid", dim3(L.nblk), dim3(PB), 0, k_true_resid<OPk, V, double>, o, L, b,
+             (const double*)x64, P);
+    else
+      launch(c, "pcg_true_resid", dim3(L.nblk), dim3(PB), 0, k_true_resid<OPk, V, V>, o, L, b, (const V*)x, P);
+    launch(c, "pcg_collect", dim3(1), dim3(PB), 0, k_collect_rr, (const double*)P.S, L.nblk, c.scal);
+    return read_scalars(c);
+  };
+  if constexpr (OPk != OP_HEAT) {
+    bool queued = false;
+    const double bc = (OPk == OP_UNIT) ? 1.0 : o.il;
+    if (mixed) {
+      if constexpr (std::is_same<V, float>::value)
+        queued = !ref && !c.cfg.pcg_recompute_q && resident_launch<V, true>(c, o, b, x, x64, -1.0, tol, cap, R, bc);
+    } else {
+      queued = resident_launch<V, false>(c, o, b, x, nullptr, ref ? eps_abs : -1.0, tol, cap, R, bc);
+    }
+    if (queued) {
+      if (!true_rr()) return MPF_HIP_ERROR;
+      c.res_seq = c.scal_host->done ? c.scal_host->res_seq : 0;
+      if (c.scal_host->done) return report(c.scal_host->res_missed != 0, c.scal_host->res_restarts);
+      // a block waited too long for the others: the launch form solves it
+    }
+  }
   // slow rows: list in cell order (positions from a scan into the cell-count scratch)
   launch(c, "pcg_slow_flag", dim3(nblocks(G, 256)), dim3(256), 0, k_slow_flag, G, (const uint8_t*)c.nbm, c.ctmp_u32);
   const int64_t nslow = run_scan_u32(c, c.ctmp_u32, c.count, G, true);
@@ -2204,35 +2252,26 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
       k = kd;
     }
   }
-  if (mixed) {
+  if (mixed)
     launch(c, "pcg_fold", dim3(L.nblk), dim3(PB), 0, k_final_fold, L, G, (const uint8_t*)c.nbm, (float*)x, x64);
-    launch(c, "pcg_true_resid", dim3(L.nblk), dim3(PB), 0, k_true_resid<OPk, V, double>, o, L, b,
-           (const double*)x64, P);
-  } else {
-    launch(c, "pcg_true_resid", dim3(L.nblk), dim3(PB), 0, k_true_resid<OPk, V, V>, o, L, b, (const V*)x, P);
-  }
-  launch(c, "pcg_collect", dim3(1), dim3(PB), 0, k_collect_rr, (const double*)P.S, L.nblk, c.scal);
-  if (!read_scalars(c)) return MPF_HIP_ERROR;
-  const SolveScalars& s = *c.scal_host;
-  const bool converged = s.converged && !true_missed;
-  if (info) {
-    info->iterations = s.iter;
-    info->refinements = s.refinements;
-    info->converged = converged ? 1 : 0;
-    info->rel_residual = s.bb > 0 ? sqrt(s.rr_true) / sqrt(s.bb) : 0.0;
-    info->abs_rr = s.rr;
-  }
-  if (s.nonfinite) {
-    c.err = "non-finite value in the solver";
-    return MPF_NONFINITE;
-  }
-  if (true_missed)
-    c.note = "mixed-precision solve: the FP64 true residual missed the tolerance (" + std::to_string(restarts) +
-             " restarts, iteration " + std::to_string(s.iter) + ")";
-  return converged ? MPF_OK : MPF_NO_CONVERGENCE;
+  if (!true_rr()) return MPF_HIP_ERROR;
+  return report(true_missed, restarts);
 }
 
 }  // namespace
+
+// 8-byte words of the resident solve's buffer, and the cells of one of its
+// six halo arrays (0: no form of the solve fits the device).
+int64_t resident_words(const Grid& g, int blocks, int64_t* cells) {
+  int64_t n = 0;
+  ResTile t;
+  if (resident_tile(g, blocks, 4, false, t)) n = std::max<int64_t>(n, (int64_t)t.nblk * t.cells);
+  if (resident_tile(g, blocks, 4, true, t)) n = std::max<int64_t>(n, (int64_t)t.nblk * t.cells);
+  if (resident_tile(g, blocks, 8, false, t)) n = std::max<int64_t>(n, (int64_t)t.nblk * t.cells);
+  *cells = n;
+  return n > 0 ? 2 * RG * RWORDS + 16 + 6 * n : 0;
+}
+int resident_most_blocks() { return RG; }
 
 int run_pressure_solve(Ctx& c, mpf_solve_info* info) {
   const mpf_config& k = c.cfg;
