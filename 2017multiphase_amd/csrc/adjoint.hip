@@ -7,6 +7,8 @@
 #include "interp.h"
 #include "mpf_internal.h"
 
+#include <algorithm>
+
 namespace mpf {
 
 namespace {
@@ -130,44 +132,132 @@ __global__ void k_adj_divT(Grid g, const int8_t* __restrict__ mark, const float*
 //   g_v[p] += (w_pf / W_f) g_u[f]
 //   g_x[p] += (dw_pf/dx)(v_p - u_f) / W_f g_u[f]
 
-// W_f and u_f recomputed in FP64 (face gather with the forward's windows).
-template <int A, bool AIRPH>
-__global__ void k_adj_p2g_faces(Grid g, const f3* __restrict__ pos, const f3* __restrict__ vel,
-                                const float* __restrict__ mass, const int8_t* __restrict__ flag,
-                                const uint32_t* __restrict__ cstart, const uint32_t* __restrict__ cend,
-                                double* __restrict__ Wout, double* __restrict__ Uout, int64_t nf) {
-  int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nf) return;
+// The air window's rows are dealt to AIR_LANES lanes per face: few faces have
+// air near them, and one lane's walk over 25 rows is a chain of loads.
+constexpr int AIR_LANES = 8;
+// W_f and u_f recomputed in FP64 (face gather with the forward's windows, one
+// launch for the three axes).  Bound by FP64 arithmetic: about 30 operations
+// at half rate, a division among them, for each of a face's 144 particles.
+// The occupancy masks of the sort, which the forward call goes by too, leave
+// out the cells and bricks without a particle of the phase: the air window
+// (100 cells) was walked on every face before, 4.1 ms at 96^3 for the six
+// launches with 2.9M particles and 6 bubbles; 0.97 (liquid) + 0.64 ms (air) now.
+struct FaceOut {
+  double* W[3];
+  double* U[3];
+};
+template <int A, bool AIRPH, bool ROWS>
+__device__ __forceinline__ void adj_p2g_face(const Grid& g, const f3* __restrict__ pos, const f3* __restrict__ vel,
+                                             const float* __restrict__ mass, const int8_t* __restrict__ flag,
+                                             const uint32_t* __restrict__ cstart, const uint32_t* __restrict__ cend,
+                                             const uint8_t* __restrict__ cmask, const uint8_t* __restrict__ dm,
+                                             double* __restrict__ Wout, double* __restrict__ Uout, int64_t f, int sub) {
   int i, j, k;
   ijk_face<A>(g, f, i, j, k);
+  constexpr uint8_t need = AIRPH ? M_AIR : M_FLUIDSOLID;
+  {
+    // the bricks around the face's cell hold every cell of the window
+    const int by = (g.ny + 3) / 4, bz = (g.nz + 3) / 4;
+    const int64_t b = ((int64_t)(min(i, g.nx - 1) >> 2) * by + (min(j, g.ny - 1) >> 2)) * bz + (min(k, g.nz - 1) >> 2);
+    if (!(dm[b] & need)) {  // the same for all lanes of a face
+      if (sub == 0) {
+        Wout[f] = 0.0;
+        Uout[f] = 0.0;
+      }
+      return;
+    }
+  }
   const double gx = (double)i + (A == 0 ? 0.0 : 0.5), gy = (double)j + (A == 1 ? 0.0 : 0.5),
                gz = (double)k + (A == 2 ? 0.0 : 0.5);
   constexpr int lo = AIRPH ? -2 : -1, hin = AIRPH ? 1 : 0, lot = AIRPH ? -2 : -1, hit = AIRPH ? 2 : 1;
   const double RE2 = (double)1.4f * (double)1.4f, scale = 1.0 / (double)g.h;
+  constexpr int NP = AIRPH ? 8 : 4;  // particles whose loads are in flight together
   double W = 0, U = 0;
-  for (int di = (A == 0 ? lo : lot); di <= (A == 0 ? hin : hit); ++di)
-    for (int dj = (A == 1 ? lo : lot); dj <= (A == 1 ? hin : hit); ++dj)
-      for (int dk = (A == 2 ? lo : lot); dk <= (A == 2 ? hin : hit); ++dk) {
-        if (!valid(g, i + di, j + dj, k + dk)) continue;
-        int64_t c = cid(g, i + di, j + dj, k + dk);
-        uint32_t s = cstart[c];
-        if (s == MPF_CELL_UNDEF) continue;
-        for (uint32_t p = s; p < cend[c]; ++p) {
-          int8_t fl = flag[p];
-          bool take = AIRPH ? (fl == AIR) : (fl == FLUID || fl == SOLID);
-          if (!take) continue;
-          f3 x = pos[p];
-          double dx = ((double)x.x - g.gx0) * scale - gx, dy = ((double)x.y - g.gy0) * scale - gy,
-                 dz = ((double)x.z - g.gz0) * scale - gz;
-          double r2 = dx * dx + dy * dy + dz * dz;
-          double w = (double)mass[p] * fmax(RE2 / fmax(r2, (double)0.0001f) - 1.0, 0.0);
-          W += w;
-          const float* vp = &vel[p].x;
-          U += w * (double)vp[A];
+  auto visit = [&](uint32_t s, uint32_t e) {
+    for (uint32_t p0 = s; p0 < e; p0 += NP) {
+      int8_t fl[NP];
+      f3 x[NP];
+      float mp[NP], va[NP];
+#pragma unroll
+      for (int u = 0; u < NP; ++u) {
+        const uint32_t p = min(p0 + (uint32_t)u, e - 1u);
+        fl[u] = flag[p];
+        x[u] = pos[p];
+        mp[u] = mass[p];
+        va[u] = (&vel[p].x)[A];
+      }
+#pragma unroll
+      for (int u = 0; u < NP; ++u) {
+        const bool take = p0 + (uint32_t)u < e && (AIRPH ? (fl[u] == AIR) : (fl[u] == FLUID || fl[u] == SOLID));
+        if (!take) continue;
+        const double dx = ((double)x[u].x - g.gx0) * scale - gx, dy = ((double)x[u].y - g.gy0) * scale - gy,
+                     dz = ((double)x[u].z - g.gz0) * scale - gz;
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        double q = 0.0;  // not positive from the kernel's radius on: no division
+        if (!(r2 >= RE2)) q = fmax(RE2 / fmax(r2, (double)0.0001f) - 1.0, 0.0);
+        const double w = (double)mp[u] * q;
+        W += w;
+        U += w * (double)va[u];
+      }
+    }
+  };
+  constexpr int i0 = A == 0 ? lo : lot, j0 = A == 1 ? lo : lot;
+  constexpr int NJ = (A == 1 ? hin : hit) - j0 + 1, NR = ((A == 0 ? hin : hit) - i0 + 1) * NJ;
+  for (int r = sub; r < NR; r += AIRPH ? AIR_LANES : 1) {
+      const int di = i0 + r / NJ, dj = j0 + r % NJ;
+      if (i + di < 0 || i + di >= g.nx || j + dj < 0 || j + dj >= g.ny) continue;
+      // the row's masks and ranges together, then its particles (ROWS: one range)
+      constexpr int k0 = A == 2 ? lo : lot, NK = (A == 2 ? hin : hit) - k0 + 1;
+      uint32_t S[NK], E[NK];
+      bool take_cell[NK];
+#pragma unroll
+      for (int q = 0; q < NK; ++q) {
+        const int ck = k + k0 + q;
+        const bool in = ck >= 0 && ck < g.nz;
+        const int64_t c = cid(g, i + di, j + dj, in ? ck : min(max(ck, 0), g.nz - 1));
+        const uint8_t m = cmask[c];
+        S[q] = cstart[c];
+        E[q] = cend[c];
+        take_cell[q] = in && (m & need);
+      }
+      uint32_t s = MPF_CELL_UNDEF, e = 0;
+#pragma unroll
+      for (int q = 0; q < NK; ++q) {
+        if (!take_cell[q]) continue;
+        if (ROWS) {
+          s = min(s, S[q]);
+          e = max(e, E[q]);
+        } else {
+          visit(S[q], E[q]);
         }
       }
-  Wout[f] = W;
-  Uout[f] = (W > 0) ? U / W : 0.0;
+      if (ROWS && s < e) visit(s, e);
+    }
+  if (AIRPH) {
+#pragma unroll
+    for (int o = 1; o < AIR_LANES; o <<= 1) {
+      W += __shfl_xor(W, o);
+      U += __shfl_xor(U, o);
+    }
+  }
+  if (sub == 0) {
+    Wout[f] = W;
+    Uout[f] = (W > 0) ? U / W : 0.0;
+  }
+}
+template <bool AIRPH, bool ROWS>
+__global__ void __launch_bounds__(256) k_adj_p2g_faces(Grid g, const f3* __restrict__ pos, const f3* __restrict__ vel,
+                                const float* __restrict__ mass, const int8_t* __restrict__ flag,
+                                const uint32_t* __restrict__ cstart, const uint32_t* __restrict__ cend,
+                                const uint8_t* __restrict__ cmask, const uint8_t* __restrict__ dm, FaceOut out) {
+  const int64_t u = xcd_block() * blockDim.x + threadIdx.x;
+  const int64_t f = AIRPH ? u / AIR_LANES : u;
+  const int sub = AIRPH ? (int)(u % AIR_LANES) : 0;
+  const int A = blockIdx.y;
+  if (f >= (A == 0 ? g.FX : A == 1 ? g.FY : g.FZ)) return;
+  if (A == 0) adj_p2g_face<0, AIRPH, ROWS>(g, pos, vel, mass, flag, cstart, cend, cmask, dm, out.W[0], out.U[0], f, sub);
+  else if (A == 1) adj_p2g_face<1, AIRPH, ROWS>(g, pos, vel, mass, flag, cstart, cend, cmask, dm, out.W[1], out.U[1], f, sub);
+  else adj_p2g_face<2, AIRPH, ROWS>(g, pos, vel, mass, flag, cstart, cend, cmask, dm, out.W[2], out.U[2], f, sub);
 }
 
 struct P2GFaceData {
@@ -176,6 +266,7 @@ struct P2GFaceData {
   const double* gu[3];
 };
 
+// The liquid launch writes every particle (0 off its phase), the air launch adds.
 template <bool AIRPH>
 __global__ void k_adj_p2g_part(Grid g, int64_t P, const f3* __restrict__ pos, const f3* __restrict__ vel,
                                const float* __restrict__ mass, const int8_t* __restrict__ flag, P2GFaceData fd,
@@ -184,7 +275,11 @@ __global__ void k_adj_p2g_part(Grid g, int64_t P, const f3* __restrict__ pos, co
   if (p >= P) return;
   const int8_t fl = flag[p];
   const bool take = AIRPH ? (fl == AIR) : (fl == FLUID || fl == SOLID);
-  if (!take) return;
+  if (!take) {
+    if (!AIRPH)
+      for (int d = 0; d < 3; ++d) gv[3 * p + d] = gx[3 * p + d] = 0.0;
+    return;
+  }
   const f3 x = pos[p];
   const float* vp = &vel[p].x;
   // the particle's cell, as the hash assigns it (getijkfrompos)
@@ -231,8 +326,8 @@ __global__ void k_adj_p2g_part(Grid g, int64_t P, const f3* __restrict__ pos, co
   }
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    gv[3 * p + d] += av[d];
-    gx[3 * p + d] += ax[d];
+    gv[3 * p + d] = AIRPH ? gv[3 * p + d] + av[d] : av[d];
+    gx[3 * p + d] = AIRPH ? gx[3 * p + d] + ax[d] : ax[d];
   }
 }
 
@@ -241,29 +336,39 @@ __global__ void k_adj_p2g_part(Grid g, int64_t P, const f3* __restrict__ pos, co
 //   v' = (1 - alpha) T(x) u + alpha (v + T(x) du),  du = u - u_old (grid of the particle's phase)
 // Adjoint: g_v = alpha g_v';  g_u += T^T g_v' (both terms);  g_uold -= alpha T^T g_v';
 //   g_x += (1 - alpha) (dT u/dx)^T g_v' + alpha (dT du/dx)^T g_v'.
-// The grid scatter uses FP64 atomics (order-dependent rounding).
+// g_uold is -alpha times the scattered g_u, so only g_u is scattered (FP64
+// atomics, whose order sets the rounding).  Particles in the order of the
+// library's sort are scattered tile by tile (4x8x8 cells): a row of 8 cells is
+// one range of particles, a wave's lanes add them into the tile's faces in
+// LDS, and the tile adds its sums to the grid once.  48 grid atomics per
+// particle took 3.6 ms at 96^3 (2.9M particles), bound by the atomics; by tiles
+// 0.47 ms.
 struct G2PArgs {
   const float* u[6];   // water u, air u (current)
   const float* du[6];  // water du, air du (forward's u - u_old)
   double* gu[6];
-  double* guo[6];
 };
 
-__global__ void k_adj_g2p(Grid g, int64_t P, const f3* __restrict__ pos, const int8_t* __restrict__ flag,
-                          G2PArgs a, double alpha, const double* __restrict__ gvo, double* __restrict__ gvi,
-                          double* __restrict__ gx) {
-  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= P) return;
+// One particle's cotangents (gvi, gx written); scat(slot, axis, i, j, k, value)
+// takes the eight corner terms of each axis.
+template <class S>
+__device__ __forceinline__ void adj_g2p_particle(const Grid& g, int64_t p, const f3* __restrict__ pos,
+                                                 const int8_t* __restrict__ flag, const G2PArgs& a, double alpha,
+                                                 const double* __restrict__ gvo, double* __restrict__ gvi,
+                                                 double* __restrict__ gx, S scat) {
   const int8_t fl = flag[p];
   int ph = -1;
   if (fl == FLUID || fl == SOLID) ph = 0;
   else if (fl == AIR) ph = 1;
   const double gv[3] = {gvo[3 * p], gvo[3 * p + 1], gvo[3 * p + 2]};
   if (ph < 0) {
-    for (int d = 0; d < 3; ++d) gvi[3 * p + d] += gv[d];
+    for (int d = 0; d < 3; ++d) {
+      gvi[3 * p + d] = gv[d];
+      gx[3 * p + d] = 0.0;
+    }
     return;
   }
-  for (int d = 0; d < 3; ++d) gvi[3 * p + d] += alpha * gv[d];
+  for (int d = 0; d < 3; ++d) gvi[3 * p + d] = alpha * gv[d];
   const f3 x = pos[p];
   const double X = ((double)x.x - g.gx0) / g.h, Y = ((double)x.y - g.gy0) / g.h, Z = ((double)x.z - g.gz0) / g.h;
   double gpos[3] = {0, 0, 0};
@@ -274,16 +379,10 @@ __global__ void k_adj_g2p(Grid g, int64_t P, const f3* __restrict__ pos, const i
     int i, j, k;
     double wt[8];
     trilinear_weights(qx, qy, qz, w, hh, d, i, j, k, wt);
-    const int64_t sj = d, si = (int64_t)hh * d;
-    const int64_t base = i * si + j * sj + k;
-    const int64_t off[8] = {0, si, sj, si + sj, 1, si + 1, sj + 1, si + sj + 1};
-    double* gu = a.gu[3 * ph + A];
-    double* guo = a.guo[3 * ph + A];
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
       if (wt[c] == 0.0) continue;
-      atomicAdd(&gu[base + off[c]], wt[c] * gv[A]);
-      if (alpha != 0.0) atomicAdd(&guo[base + off[c]], -alpha * wt[c] * gv[A]);
+      scat(3 * ph + A, A, i + (c & 1), j + ((c >> 1) & 1), k + (c >> 2), wt[c] * gv[A]);
     }
     double g1x, g1y, g1z, g2x, g2y, g2z;
     trilinear_grad(a.u[3 * ph + A], qx, qy, qz, w, hh, d, g1x, g1y, g1z);
@@ -293,7 +392,86 @@ __global__ void k_adj_g2p(Grid g, int64_t P, const f3* __restrict__ pos, const i
     gpos[1] += (s1 * g1y + s2 * g2y) / (double)g.h;
     gpos[2] += (s1 * g1z + s2 * g2z) / (double)g.h;
   }
-  for (int d = 0; d < 3; ++d) gx[3 * p + d] += gpos[d];
+  for (int d = 0; d < 3; ++d) gx[3 * p + d] = gpos[d];
+}
+
+__global__ void __launch_bounds__(256) k_adj_g2p(Grid g, int64_t P, const f3* __restrict__ pos, const int8_t* __restrict__ flag,
+                          G2PArgs a, double alpha, const double* __restrict__ gvo, double* __restrict__ gvi,
+                          double* __restrict__ gx) {
+  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= P) return;
+  adj_g2p_particle(g, p, pos, flag, a, alpha, gvo, gvi, gx, [&](int slot, int A, int i, int j, int k, double v) {
+    unsafeAtomicAdd(&a.gu[slot][fid(g, A, i, j, k)], v);
+  });
+}
+
+// The tile's faces of axis a: [t0_d - (d != a), t0_d + T_d] along d, as in the liquid P2G.
+constexpr int GT_X = 4, GT_Y = 8, GT_Z = 8, GT = GT_X * GT_Y * GT_Z;
+__host__ __device__ constexpr int gt_t(int d) { return d == 0 ? GT_X : (d == 1 ? GT_Y : GT_Z); }
+__host__ __device__ constexpr int gt_r(int a, int d) { return gt_t(d) + (d == a ? 1 : 2); }
+__host__ __device__ constexpr int gt_sz(int a) { return gt_r(a, 0) * gt_r(a, 1) * gt_r(a, 2); }
+__host__ __device__ constexpr int gt_off(int a) { return a == 0 ? 0 : (a == 1 ? gt_sz(0) : gt_sz(0) + gt_sz(1)); }
+constexpr int GT_TOT = gt_sz(0) + gt_sz(1) + gt_sz(2);
+
+__global__ void __launch_bounds__(GT)
+    k_adj_g2p_tile(Grid g, const f3* __restrict__ pos, const int8_t* __restrict__ flag,
+                   const uint32_t* __restrict__ cstart, const uint32_t* __restrict__ cend, int nty, int ntz, G2PArgs a,
+                   double alpha, const double* __restrict__ gvo, double* __restrict__ gvi, double* __restrict__ gx) {
+  __shared__ double acc[2 * GT_TOT];  // liquid, then air
+  __shared__ uint32_t sS[GT], sE[GT];
+  int t = (int)xcd_block();
+  const int tz = t % ntz;
+  t /= ntz;
+  const int ty = t % nty, tx = t / nty;
+  const int x0 = tx * GT_X, y0 = ty * GT_Y, z0 = tz * GT_Z;
+  const int b = threadIdx.x, lane = b & 63;
+  for (int q = b; q < 2 * GT_TOT; q += GT) acc[q] = 0.0;
+  {
+    const int ci = x0 + b / (GT_Y * GT_Z), cj = y0 + (b / GT_Z) % GT_Y, ck = z0 + b % GT_Z;
+    uint32_t s = MPF_CELL_UNDEF, e = 0;
+    if (valid(g, ci, cj, ck)) {
+      const int64_t c = cid(g, ci, cj, ck);
+      s = cstart[c];
+      e = s == MPF_CELL_UNDEF ? 0 : cend[c];
+    }
+    sS[b] = s;
+    sE[b] = e;
+  }
+  __syncthreads();
+  for (int row = b >> 6; row < GT_X * GT_Y; row += GT / 64) {
+    uint32_t s = MPF_CELL_UNDEF, e = 0;
+#pragma unroll
+    for (int q = 0; q < GT_Z; ++q) {
+      s = min(s, sS[row * GT_Z + q]);
+      e = max(e, sE[row * GT_Z + q]);
+    }
+    for (uint32_t p = s + lane; s < e && p < e; p += 64)
+      adj_g2p_particle(g, p, pos, flag, a, alpha, gvo, gvi, gx, [&](int slot, int A, int i, int j, int k, double v) {
+        const int ri = i - (x0 - (A != 0)), rj = j - (y0 - (A != 1)), rk = k - (z0 - (A != 2));
+        // (a particle outside the domain lies in cell 0 whatever its position)
+        if ((unsigned)ri < (unsigned)gt_r(A, 0) && (unsigned)rj < (unsigned)gt_r(A, 1) &&
+            (unsigned)rk < (unsigned)gt_r(A, 2))
+          unsafeAtomicAdd(&acc[(slot >= 3 ? GT_TOT : 0) + gt_off(A) + (ri * gt_r(A, 1) + rj) * gt_r(A, 2) + rk], v);
+        else
+          unsafeAtomicAdd(&a.gu[slot][fid(g, A, i, j, k)], v);
+      });
+  }
+  __syncthreads();
+  for (int q = b; q < 2 * GT_TOT; q += GT) {
+    const double v = acc[q];
+    if (v == 0.0) continue;
+    const int ph = q >= GT_TOT, r = q - ph * GT_TOT;
+    const int A = r < gt_off(1) ? 0 : (r < gt_off(2) ? 1 : 2);
+    const int l = r - gt_off(A);
+    const int rk = l % gt_r(A, 2), rj = (l / gt_r(A, 2)) % gt_r(A, 1), ri = l / (gt_r(A, 2) * gt_r(A, 1));
+    unsafeAtomicAdd(&a.gu[3 * ph + A][fid(g, A, x0 - (A != 0) + ri, y0 - (A != 1) + rj, z0 - (A != 2) + rk)], v);
+  }
+}
+
+// g_uold = -alpha g_u
+__global__ void k_adj_uold(int64_t n, const double* __restrict__ gu, double alpha, double* __restrict__ guo) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) guo[i] = 0.0 - alpha * gu[i];
 }
 
 // ---------------- advection ----------------
@@ -337,7 +515,10 @@ __global__ void k_adj_advect(Grid g, int64_t P, const f3* __restrict__ pos, cons
 // diagonal direction; then the wall rule zeroes faces and sets the ceiling
 // uz(nz-1) to min(uz(nz-2), 0).  Linear in u for fixed level set and flags.
 
-// The forward's decision for face (i,j,k) of axis A: false = identity.
+// The forward's decision for face (i,j,k) of axis A: false = identity.  The
+// reference visits the 8 octants and the last one whose three weights are all
+// >= 0 decides; each weight depends on its own axis' sign only, so per axis +1
+// decides if its weight passes, else -1 (as in the forward's sweep).
 template <int A>
 __device__ __forceinline__ bool sweep_rule(const Grid& g, const float* __restrict__ ls,
                                            const int8_t* __restrict__ mark, int8_t sf, int i, int j, int k,
@@ -351,58 +532,96 @@ __device__ __forceinline__ bool sweep_rule(const Grid& g, const float* __restric
   constexpr int t1 = (A == 0) ? 1 : (A == 1) ? 0 : 1;
   constexpr int t2 = (A == 0) ? 2 : (A == 1) ? 2 : 0;
   const int lims[3] = {g.nx, g.ny, g.nz};
-  bool any = false;
-  for (int di = -1; di <= 1; di += 2)
-    for (int dj = -1; dj <= 1; dj += 2)
-      for (int dk = -1; dk <= 1; dk += 2) {
-        const int dd[3] = {di, dj, dk};
-        if (n[t1] + dd[t1] < 0 || n[t1] + dd[t1] > lims[t1] - 1) continue;
-        if (n[t2] + dd[t2] < 0 || n[t2] + dd[t2] > lims[t2] - 1) continue;
-        float wv[3];
-        wv[A] = (float)(-dd[A]) * (lsc - lsb);
-        if (wv[A] < 0) continue;
-        int o1[3] = {0, 0, 0};
-        o1[t1] = dd[t1];
-        wv[t1] = (lsc + lsb - ls[cid(g, i + o1[0], j + o1[1], k + o1[2])] - ls[cid(g, bi + o1[0], bj + o1[1], bk + o1[2])]) * 0.5f;
-        if (wv[t1] < 0) continue;
-        int o2[3] = {0, 0, 0};
-        o2[t2] = dd[t2];
-        wv[t2] = (lsc + lsb - ls[cid(g, i + o2[0], j + o2[1], k + o2[2])] - ls[cid(g, bi + o2[0], bj + o2[1], bk + o2[2])]) * 0.5f;
-        if (wv[t2] < 0) continue;
-        float wx = wv[0], wy = wv[1], wz = wv[2];
-        const float wsum = wx + wy + wz;
-        if (wsum == 0) wx = wy = wz = 1.0f / 3;
-        else { wx /= wsum; wy /= wsum; wz /= wsum; }
-        dsel[0] = di; dsel[1] = dj; dsel[2] = dk;
-        wsel[0] = wx; wsel[1] = wy; wsel[2] = wz;
-        any = true;
-      }
-  return any;
+  float wv[3][2];
+  bool ok[3][2];
+#pragma unroll
+  for (int sg = 0; sg < 2; ++sg) {
+    const int dd = sg ? 1 : -1;
+    wv[A][sg] = (float)(-dd) * (lsc - lsb);
+    ok[A][sg] = !(wv[A][sg] < 0);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int ax = t == 0 ? t1 : t2;
+      const bool in = n[ax] + dd >= 0 && n[ax] + dd <= lims[ax] - 1;
+      int o[3] = {0, 0, 0};
+      o[ax] = in ? dd : 0;
+      const float lc = ls[cid(g, i + o[0], j + o[1], k + o[2])], lb = ls[cid(g, bi + o[0], bj + o[1], bk + o[2])];
+      wv[ax][sg] = (lsc + lsb - lc - lb) * 0.5f;
+      ok[ax][sg] = in && !(wv[ax][sg] < 0);
+    }
+  }
+  if (!((ok[0][0] || ok[0][1]) && (ok[1][0] || ok[1][1]) && (ok[2][0] || ok[2][1]))) return false;
+  float wx[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    dsel[d] = ok[d][1] ? 1 : -1;
+    wx[d] = ok[d][1] ? wv[d][1] : wv[d][0];
+  }
+  const float wsum = wx[0] + wx[1] + wx[2];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) wsel[d] = wsum == 0 ? 1.0f / 3 : wx[d] / wsum;
+  return true;
+}
+
+// The decisions of every face of axis A, for both transposed passes: code bit
+// 3: blended, bits 0-2: the direction along x, y, z is +1; the three weights.
+// (A pass that evaluates the rules of a face and its six readers itself took
+// 87 us a launch at 96^3, 12 launches; now 12 us, and 11 us for an axis' rules.)
+struct SweepRules {
+  float* w[3];
+  uint8_t* code;
+};
+template <int A>
+__global__ void k_adj_sweep_rules(Grid g, const float* __restrict__ ls, const int8_t* __restrict__ mark, int8_t sf,
+                                  SweepRules r, int64_t nf) {
+  int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (f >= nf) return;
+  int i, j, k;
+  ijk_face<A>(g, f, i, j, k);
+  int dsel[3];
+  float wsel[3];
+  if (!sweep_rule<A>(g, ls, mark, sf, i, j, k, dsel, wsel)) {
+    r.code[f] = 0;
+    return;
+  }
+  uint8_t c = 8;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    c |= dsel[d] > 0 ? (uint8_t)(1u << d) : (uint8_t)0;
+    r.w[d][f] = wsel[d];
+  }
+  r.code[f] = c;
 }
 
 // One transposed pass, as a gather: face n collects its identity term and the
 // weights of the (at most 6) faces whose chosen blend reads it.
 template <int A>
-__global__ void k_adj_sweep_u(Grid g, const double* __restrict__ gout, double* __restrict__ gin,
-                              const float* __restrict__ ls, const int8_t* __restrict__ mark, int8_t sf, int64_t nf) {
+__global__ void k_adj_sweep_u(Grid g, const double* __restrict__ gout, double* __restrict__ gin, SweepRules r,
+                              int64_t nf) {
   int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= nf) return;
   int i, j, k;
   ijk_face<A>(g, f, i, j, k);
   const int dims[3] = {g.nx + (A == 0), g.ny + (A == 1), g.nz + (A == 2)};
-  int dsel[3];
-  float wsel[3];
-  double acc = sweep_rule<A>(g, ls, mark, sf, i, j, k, dsel, wsel) ? 0.0 : gout[f];
+  const int n[3] = {i, j, k};
+  const int64_t st[3] = {(int64_t)dims[1] * dims[2], dims[2], 1};
+  uint8_t c[3][2];
 #pragma unroll
   for (int d = 0; d < 3; ++d)
 #pragma unroll
-    for (int s = -1; s <= 1; s += 2) {
-      int q[3] = {i, j, k};
-      q[d] -= s;  // candidate reader: its blend along d with direction s lands on f
-      if (q[d] < 0 || q[d] >= dims[d]) continue;
-      if (!sweep_rule<A>(g, ls, mark, sf, q[0], q[1], q[2], dsel, wsel)) continue;
-      if (dsel[d] != s) continue;
-      acc += (double)wsel[d] * gout[fid(g, A, q[0], q[1], q[2])];
+    for (int s = 0; s < 2; ++s) {
+      // candidate reader: its blend along d with direction s lands on f
+      const bool in = s ? n[d] > 0 : n[d] + 1 < dims[d];
+      c[d][s] = in ? r.code[s ? f - st[d] : f + st[d]] : (uint8_t)0;
+    }
+  double acc = r.code[f] ? 0.0 : gout[f];
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      if (!c[d][s] || ((c[d][s] >> d) & 1) != s) continue;
+      const int64_t q = s ? f - st[d] : f + st[d];
+      acc += (double)r.w[d][q] * gout[q];
     }
   gin[f] = acc;
 }
@@ -545,6 +764,16 @@ int run_extrapolate_adjoint(Ctx& c, const double* const* gout, double* const* gi
   if (!adj_alloc(c)) return MPF_INVALID_ARG;
   for (int q = 0; q < 6; ++q) copy_in(c, c.adj_fin[q], gout ? gout[q] : nullptr, face_count(c, q), where);
   const int64_t fc[3] = {c.g.FX, c.g.FY, c.g.FZ};
+  // the decisions of one axis at a time, in the P2G's tile buffer (over 12
+  // floats per cell; they take 13 bytes per face)
+  SweepRules rules;
+  const int64_t fmax_ = std::max(fc[0], std::max(fc[1], fc[2]));
+  for (int d = 0; d < 3; ++d) rules.w[d] = c.p2g_parts + d * fmax_;
+  rules.code = (uint8_t*)(c.p2g_parts + 3 * fmax_);
+  if (3 * fmax_ + (fmax_ + 3) / 4 > p2g_parts_floats(c.g)) {
+    c.err = "extrapolation adjoint: scratch too small";
+    return MPF_INVALID_ARG;
+  }
   for (int ph = 0; ph < 2; ++ph) {
     float* const* u = ph == 0 ? c.wu : c.au;
     const float* phi = ph == 0 ? c.phifluid : c.phiair;
@@ -560,12 +789,16 @@ int run_extrapolate_adjoint(Ctx& c, const double* const* gout, double* const* gi
       if (A == 0) launch(c, "adj_bc", dim3(nb), dim3(256), 0, k_adj_bc<0>, c.g, (const double*)a, b, mk, (const float*)u[0], fc[0]);
       if (A == 1) launch(c, "adj_bc", dim3(nb), dim3(256), 0, k_adj_bc<1>, c.g, (const double*)a, b, mk, (const float*)u[1], fc[1]);
       if (A == 2) launch(c, "adj_bc", dim3(nb), dim3(256), 0, k_adj_bc<2>, c.g, (const double*)a, b, mk, (const float*)u[2], fc[2]);
+      const char* rn = "adj_sweep_rules";
+      if (A == 0) launch(c, rn, dim3(nb), dim3(256), 0, k_adj_sweep_rules<0>, c.g, phi, mk, sf, rules, fc[0]);
+      if (A == 1) launch(c, rn, dim3(nb), dim3(256), 0, k_adj_sweep_rules<1>, c.g, phi, mk, sf, rules, fc[1]);
+      if (A == 2) launch(c, rn, dim3(nb), dim3(256), 0, k_adj_sweep_rules<2>, c.g, phi, mk, sf, rules, fc[2]);
       for (int pass = 0; pass < 2; ++pass) {
         const double* src = pass == 0 ? b : a;
         double* dst = pass == 0 ? a : b;
-        if (A == 0) launch(c, "adj_sweep_u", dim3(nb), dim3(256), 0, k_adj_sweep_u<0>, c.g, src, dst, phi, mk, sf, fc[0]);
-        if (A == 1) launch(c, "adj_sweep_u", dim3(nb), dim3(256), 0, k_adj_sweep_u<1>, c.g, src, dst, phi, mk, sf, fc[1]);
-        if (A == 2) launch(c, "adj_sweep_u", dim3(nb), dim3(256), 0, k_adj_sweep_u<2>, c.g, src, dst, phi, mk, sf, fc[2]);
+        if (A == 0) launch(c, "adj_sweep_u", dim3(nb), dim3(256), 0, k_adj_sweep_u<0>, c.g, src, dst, rules, fc[0]);
+        if (A == 1) launch(c, "adj_sweep_u", dim3(nb), dim3(256), 0, k_adj_sweep_u<1>, c.g, src, dst, rules, fc[1]);
+        if (A == 2) launch(c, "adj_sweep_u", dim3(nb), dim3(256), 0, k_adj_sweep_u<2>, c.g, src, dst, rules, fc[2]);
       }
     }
   }
@@ -578,27 +811,23 @@ int run_p2g_adjoint(Ctx& c, const double* const* gfaces, double* gvel, double* g
   const int cur = c.cur;
   const int64_t P = c.P;
   for (int q = 0; q < 6; ++q) copy_in(c, c.adj_fin[q], gfaces ? gfaces[q] : nullptr, face_count(c, q), where);
-  zero(c, c.adj_part[0], 3 * P);
-  zero(c, c.adj_part[2], 3 * P);
+  const int64_t fc[3] = {c.g.FX, c.g.FY, c.g.FZ};
+  const int64_t fm = std::max(fc[0], std::max(fc[1], fc[2]));
   for (int ph = 0; ph < 2; ++ph) {
     // W in adj_fout[0..2], U in adj_fout[3..5]
-    const int64_t fc[3] = {c.g.FX, c.g.FY, c.g.FZ};
+    FaceOut fo;
     for (int A = 0; A < 3; ++A) {
-      auto args = [&](auto kern) {
-        launch(c, "adj_p2g_faces", dim3(nblocks(fc[A], 256)), dim3(256), 0, kern, c.g, (const f3*)c.pos[cur],
-               (const f3*)c.vel[cur], (const float*)c.mass[cur], (const int8_t*)c.flag[cur],
-               (const uint32_t*)c.cstart, (const uint32_t*)c.cend, c.adj_fout[A], c.adj_fout[3 + A], fc[A]);
-      };
-      if (ph == 0) {
-        if (A == 0) args(k_adj_p2g_faces<0, false>);
-        if (A == 1) args(k_adj_p2g_faces<1, false>);
-        if (A == 2) args(k_adj_p2g_faces<2, false>);
-      } else {
-        if (A == 0) args(k_adj_p2g_faces<0, true>);
-        if (A == 1) args(k_adj_p2g_faces<1, true>);
-        if (A == 2) args(k_adj_p2g_faces<2, true>);
-      }
+      fo.W[A] = c.adj_fout[A];
+      fo.U[A] = c.adj_fout[3 + A];
     }
+    // with the library's own sort a row's cells are one range of particles
+    auto kern = ph == 0 ? (c.own_sort ? k_adj_p2g_faces<false, true> : k_adj_p2g_faces<false, false>)
+                        : (c.own_sort ? k_adj_p2g_faces<true, true> : k_adj_p2g_faces<true, false>);
+    launch(c, ph == 0 ? "adj_p2g_faces" : "adj_p2g_faces_air",
+           dim3(nblocks(ph == 0 ? fm : fm * AIR_LANES, 256), 3), dim3(256), 0, kern, c.g,
+           (const f3*)c.pos[cur], (const f3*)c.vel[cur], (const float*)c.mass[cur], (const int8_t*)c.flag[cur],
+           (const uint32_t*)c.cstart, (const uint32_t*)c.cend, (const uint8_t*)c.cmask,
+           (const uint8_t*)(c.bmask + nbricks(c.g)), fo);
     P2GFaceData fd;
     for (int A = 0; A < 3; ++A) {
       fd.W[A] = c.adj_fout[A];
@@ -610,7 +839,7 @@ int run_p2g_adjoint(Ctx& c, const double* const* gfaces, double* gvel, double* g
              (const f3*)c.pos[cur], (const f3*)c.vel[cur], (const float*)c.mass[cur], (const int8_t*)c.flag[cur], fd,
              c.adj_part[0], c.adj_part[2]);
     else
-      launch(c, "adj_p2g_part", dim3(nblocks(P, 256)), dim3(256), 0, k_adj_p2g_part<true>, c.g, P,
+      launch(c, "adj_p2g_part_air", dim3(nblocks(P, 256)), dim3(256), 0, k_adj_p2g_part<true>, c.g, P,
              (const f3*)c.pos[cur], (const f3*)c.vel[cur], (const float*)c.mass[cur], (const int8_t*)c.flag[cur], fd,
              c.adj_part[0], c.adj_part[2]);
   }
@@ -625,12 +854,7 @@ int run_g2p_adjoint(Ctx& c, const double* gvel_out, double* gvel_in, double* con
   const int cur = c.cur;
   const int64_t P = c.P;
   copy_in(c, c.adj_part[0], gvel_out, 3 * P, where);
-  zero(c, c.adj_part[1], 3 * P);
-  zero(c, c.adj_part[2], 3 * P);
-  for (int q = 0; q < 6; ++q) {
-    zero(c, c.adj_fin[q], face_count(c, q));
-    zero(c, c.adj_fout[q], face_count(c, q));
-  }
+  for (int q = 0; q < 6; ++q) zero(c, c.adj_fin[q], face_count(c, q));
   G2PArgs a;
   for (int A = 0; A < 3; ++A) {
     a.u[A] = c.wu[A];
@@ -638,13 +862,24 @@ int run_g2p_adjoint(Ctx& c, const double* gvel_out, double* gvel_in, double* con
     a.du[A] = c.wuo[A];
     a.du[3 + A] = c.auo[A];
   }
-  for (int q = 0; q < 6; ++q) {
-    a.gu[q] = c.adj_fin[q];
-    a.guo[q] = c.adj_fout[q];
+  for (int q = 0; q < 6; ++q) a.gu[q] = c.adj_fin[q];
+  const double alpha = (double)c.cfg.flip_alpha;
+  // tile by tile when the particles lie in the order of this library's sort
+  // (lists given by the caller need not be the particles' order)
+  if (c.own_sort) {
+    const int ntx = (c.g.nx + GT_X - 1) / GT_X, nty = (c.g.ny + GT_Y - 1) / GT_Y, ntz = (c.g.nz + GT_Z - 1) / GT_Z;
+    launch(c, "adj_g2p_tile", dim3((unsigned)(ntx * nty * ntz)), dim3(GT), 0, k_adj_g2p_tile, c.g,
+           (const f3*)c.pos[cur], (const int8_t*)c.flag[cur], (const uint32_t*)c.cstart, (const uint32_t*)c.cend, nty,
+           ntz, a, alpha, (const double*)c.adj_part[0], c.adj_part[1], c.adj_part[2]);
+  } else {
+    launch(c, "adj_g2p", dim3(nblocks(P, 256)), dim3(256), 0, k_adj_g2p, c.g, P, (const f3*)c.pos[cur],
+           (const int8_t*)c.flag[cur], a, alpha, (const double*)c.adj_part[0], c.adj_part[1], c.adj_part[2]);
   }
-  launch(c, "adj_g2p", dim3(nblocks(P, 256)), dim3(256), 0, k_adj_g2p, c.g, P, (const f3*)c.pos[cur],
-         (const int8_t*)c.flag[cur], a, (double)c.cfg.flip_alpha, (const double*)c.adj_part[0], c.adj_part[1],
-         c.adj_part[2]);
+  if (guo)
+    for (int q = 0; q < 6; ++q)
+      if (guo[q])
+        launch(c, "adj_uold", dim3(nblocks(face_count(c, q), 256)), dim3(256), 0, k_adj_uold, face_count(c, q),
+               (const double*)c.adj_fin[q], alpha, c.adj_fout[q]);
   copy_out(c, gvel_in, c.adj_part[1], 3 * P, where);
   copy_out(c, gpos, c.adj_part[2], 3 * P, where);
   for (int q = 0; q < 6; ++q) {

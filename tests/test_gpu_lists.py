@@ -1,0 +1,66 @@
+"""Gathers and scatters over rows of cells against their forms for caller-given
+cell lists.
+
+With the library's own sort a row of cells along k is one range of particles,
+which the air P2G, the P2G adjoint and the G2P adjoint read as such; cell lists
+set by the caller take the same kernels cell by cell (the G2P adjoint: particle
+by particle).  Both forms add the same terms: the air P2G in the same order
+(equal bits), the adjoints in FP64 in another order.  A sum of at most
+n = 4000 FP64 terms differs between two orders by at most n * 2^-53 times the
+sum of the terms' magnitudes, so 1e-12 of the largest value bounds every
+element; the cotangents of P2G divide by the weights' sum, whose relative
+change is as small.
+"""
+import numpy as np
+import pytest
+
+from helpers import say
+
+pytestmark = pytest.mark.gpu
+
+FACE = ["WATER_UX", "WATER_UY", "WATER_UZ", "AIR_UX", "AIR_UY", "AIR_UZ"]
+
+
+@pytest.mark.parametrize("dims", [(4, 4, 12), (5, 9, 7), (8, 16, 8), (13, 17, 23), (33, 31, 10)])
+def test_row_ranges(pkg, dims):
+    say("row ranges", dims)
+    nx, ny, nz = dims
+    cfg = pkg.default_config(nx, ny, nz, particle_capacity=nx * ny * nz * 6 + 64, adjoint_enabled=1, flip_alpha=0.95,
+                             heat_enabled=0, gas_enabled=0, mc_enabled=0)
+    rng = np.random.default_rng(nx * 1000 + ny * 10 + nz)
+    n = nx * ny * nz * 6
+    h = float(cfg.dx)
+    # some particles on cell borders and some outside the domain (cell 0);
+    # liquid, air and solids mixed, whole bricks without air
+    pos = (rng.uniform(0.0, 1.0, (n, 3)) * np.array(dims) * h).astype(np.float32)
+    pos[::17] = (np.round(pos[::17] / h) * h).astype(np.float32)
+    pos[::101] -= np.float32(3 * h * nx)
+    flag = np.where(rng.uniform(size=n) < 0.2, pkg.TYPESOLID, pkg.TYPEFLUID).astype(np.int8)
+    air = (pos[:, 2] > 0.5 * nz * h) & (rng.uniform(size=n) < 0.5)
+    flag[air] = pkg.TYPEAIR
+    vel = rng.standard_normal((n, 3)).astype(np.float32)
+    own = pkg.Simulator(cfg)
+    own.set_particles(n, pos=pos, vel=vel, flag=flag, mass=rng.uniform(0.5, 2.0, n).astype(np.float32))
+    own.hash_sort()
+    p = own.get_particles()
+    given = pkg.Simulator(cfg)
+    given.set_particles(n, **p)
+    for nm in ("CELL_START", "CELL_END"):
+        given.set_field(nm, own.get_field(nm))
+    gf = [rng.standard_normal(m) for m in own.face_sizes()]
+    gv = rng.standard_normal((n, 3))
+    out = []
+    for sim in (own, given):
+        sim.p2g()
+        faces = [sim.get_field(f) for f in FACE]
+        pv, px = sim.p2g_adjoint(gf)
+        r = sim.g2p_adjoint(gv)
+        out.append((faces, [pv, px, r["vel"], r["pos"]] + list(r["u"]) + list(r["u_old"])))
+    for f, a, b in zip(FACE, out[0][0], out[1][0]):
+        if f.startswith("AIR"):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), f
+    assert np.any(out[0][0][3]) and np.any(out[0][0][0])
+    for q, (a, b) in enumerate(zip(out[0][1], out[1][1])):
+        err = np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300)
+        say("  adjoint output %d: %.2e" % (q, err))
+        assert np.any(b) and err <= 1e-12
