@@ -1684,6 +1684,7 @@ static void p2g_liquid(Ctx& c, float* const* out, float* const* out2 = nullptr, 
          ntz, out[2], out2 ? out2[2] : (float*)nullptr, fc[2], band, big);
 }
 
+static_assert(2 * ST_RTOT >= 12 * ST_CELLS, "the solver's slow-row weights (six FP64 values a cell) fit as well");
 int64_t p2g_parts_floats(const Grid& g) {
   const int64_t nt = (int64_t)((g.nx + ST_X - 1) / ST_X) * ((g.ny + ST_Y - 1) / ST_Y) * ((g.nz + ST_Z - 1) / ST_Z);
   return nt * 2 * ST_RTOT;

@@ -392,16 +392,18 @@ __global__ void __launch_bounds__(PB) k_init(OpArgs o, Launch L, const V* __rest
 }
 
 // ---- spmv tiling ----
-constexpr int TJ = 8, TK = 128;               // (j, k) column tile
+// (j, k) column tiles of TCELLS / TK rows of TK cells, TK = 128 or 64 by the
+// grid (make_tiling), with a one-cell ring in LDS.
+constexpr int TCELLS = 1024;                  // cells of a tile's plane
+constexpr int TK_WIDE = 128, TK_NARROW = 64;
 constexpr int ST = 512;                       // threads per spmv block
-constexpr int RPT = TJ * TK / ST;             // tile rows per thread (2)
-constexpr int LJ = TJ + 2, LK = TK + 2;       // LDS plane with a one-cell ring
-constexpr int NRING = 2 * TK + 2 * TJ;        // ring cells per plane
-static_assert(NRING <= ST, "one ring cell per thread");
-static_assert((TK & (TK - 1)) == 0 && (ST / TK) * RPT == TJ, "threads cover the tile in rows of TK");
+constexpr int RPT = TCELLS / ST;              // tile rows per thread (2)
+static_assert(2 * TK_WIDE + 2 * (TCELLS / TK_WIDE) <= ST && 2 * TK_NARROW + 2 * (TCELLS / TK_NARROW) <= ST,
+              "one ring cell per thread");
 
 struct Tiling {
   int ntj, ntk, seg, nblk;
+  int tk;   // cells of a tile along k (TK)
   int ns5;  // single-kernel iteration: blocks of slow-row partials after the nblk tile blocks
 };
 // Block -> tile run.  Blocks are dispatched round-robin over the 8 XCDs, so
@@ -496,14 +498,71 @@ __device__ __forceinline__ V slow_row(const OpArgs& o, int i, int j, int k, int6
   return (OPk == OP_HEAT) ? s : s / ((V)g.h * (V)g.h);
 }
 
+// The six face weights of the slow rows in list order, weight f of row t at
+// sb[f n + t] (0: no flow through the face).  Computed once per solve: a row
+// that read the flags and the level set of its neighbours in every iteration
+// waited for one memory round trip per face (13 us an iteration at 192^3 with
+// a bubble, 8 with the weights stored, 5 of them an empty launch's).
+template <class V, int OPk>
+__global__ void k_slow_beta(OpArgs o, const uint32_t* __restrict__ list, int64_t n, V* __restrict__ sb) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const Grid& g = o.g;
+  const int64_t idx = list[t];
+  int i, j, k;
+  ijk_of(g, idx, i, j, k);
+  const int8_t m = o.mark[idx];
+#pragma unroll
+  for (int f = 0; f < 6; ++f) {
+    const int ii = i + c_off[f][0], jj = j + c_off[f][1], kk = k + c_off[f][2];
+    const int8_t mn = mark_at(g, o.mark, ii, jj, kk);
+    V be = V(0);
+    if (!neumann(o, OPk, mn)) be = (OPk == OP_UNIT) ? V(1) : face_beta<V>(o, idx, cid(g, ii, jj, kk), m, mn);
+    sb[f * n + t] = be;
+  }
+}
+
+// slow_row from the stored weights (p is 0 off the unknowns in every buffer
+// of a solve); the heat operator's rows read the flags.
+template <class V, int OPk>
+__device__ __forceinline__ V slow_row_at(const OpArgs& o, int64_t idx, const V* __restrict__ sb, int64_t n, int64_t t,
+                                         const V* __restrict__ pc, V pcv) {
+  V pn[6];
+  if constexpr (OPk == OP_HEAT) {
+    int i, j, k;
+    ijk_of(o.g, idx, i, j, k);
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+      const int ii = i + c_off[f][0], jj = j + c_off[f][1], kk = k + c_off[f][2];
+      pn[f] = valid(o.g, ii, jj, kk) ? pc[cid(o.g, ii, jj, kk)] : V(0);
+    }
+    return slow_row<V, OPk>(o, i, j, k, idx, pcv, pn[0], pn[1], pn[2], pn[3], pn[4], pn[5]);
+  } else {
+    int64_t st[6];
+    nb_strides(o.g, st);
+    V be[6];
+    // (a neighbour outside the array has weight 0: clamped into it)
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+      be[f] = sb[f * n + t];
+      pn[f] = pc[min(max(idx + st[f], (int64_t)0), o.g.G - 1)];
+    }
+    V s = V(0);
+#pragma unroll
+    for (int f = 0; f < 6; ++f) s = (be[f] != V(0)) ? s + be[f] * (pn[f] - pcv) : s;
+    return s / ((V)o.g.h * (V)o.g.h);
+  }
+}
+
 // Iteration k.  From update(k-1): rz_k, rr_k (slot (k-1)&1) and rz_{k-1}
 // (slot k&1) -> convergence, beta.  Then p_k = r*dinv + beta p_{k-1} for the
 // block's tile (plus its ring), stored; q = A p_k; partial p.q.
-template <class V, class Dacc, int OPk, bool SLOW>
+template <class V, class Dacc, int OPk, bool SLOW, int TK>
 __global__ void __launch_bounds__(ST, (sizeof(V) == 4 && !SLOW) ? 6 : 4) k_spmv(OpArgs o, Tiling T, int nbu, const V* __restrict__ r,
                                              const V* __restrict__ pp, V* __restrict__ pc, V* __restrict__ q,
                                              Parts P, SolveScalars* sc, int k, int ref, double eps_abs, double tol,
                                              int cap) {
+  constexpr int TJ = TCELLS / TK, LJ = TJ + 2, LK = TK + 2, NRING = 2 * TK + 2 * TJ;
   if (sc->done) return;
   __shared__ V dtab[8];  // 1/diag of the fast rows by open-face count (ordered by read_partials' barriers)
   if (threadIdx.x < 8) dtab[threadIdx.x] = (threadIdx.x < 7) ? dinv_tab<V>(o, threadIdx.x) : V(1);
@@ -717,23 +776,14 @@ __global__ void k_slow_list(int64_t G, const uint8_t* __restrict__ nbm, const ui
 // into S2.  A fixed grid walks the list, so the sums are deterministic.
 template <class V, class Dacc, int OPk>
 __global__ void __launch_bounds__(PB) k_slow_q(OpArgs o, const uint32_t* __restrict__ list, int64_t n,
-                                               const V* __restrict__ pc, V* __restrict__ q, double* __restrict__ S2,
-                                               SolveScalars* sc) {
+                                               const V* __restrict__ sb, const V* __restrict__ pc,
+                                               V* __restrict__ q, double* __restrict__ S2, SolveScalars* sc) {
   if (sc->done) return;
-  const Grid& g = o.g;
   Dacc a_pq = 0;
   for (int64_t t = (int64_t)blockIdx.x * PB + threadIdx.x; t < n; t += (int64_t)gridDim.x * PB) {
     const int64_t idx = list[t];
-    int i, j, k;
-    ijk_of(g, idx, i, j, k);
-    V pn[6];
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {
-      const int ii = i + c_off[f][0], jj = j + c_off[f][1], kk = k + c_off[f][2];
-      pn[f] = valid(g, ii, jj, kk) ? pc[cid(g, ii, jj, kk)] : V(0);
-    }
     const V pcv = pc[idx];
-    const V qv = slow_row<V, OPk>(o, i, j, k, idx, pcv, pn[0], pn[1], pn[2], pn[3], pn[4], pn[5]);
+    const V qv = slow_row_at<V, OPk>(o, idx, sb, n, t, pc, pcv);
     q[idx] = qv;
     a_pq += (Dacc)pcv * (Dacc)qv;
   }
@@ -910,11 +960,12 @@ __global__ void __launch_bounds__(PB) k_update(OpArgs o, Launch L, V* __restrict
 // MODE 0: no slow rows; 1: slow rows inline (flags and level set read per
 // row); 2: slow rows skipped (their residual and sums come from
 // k_slow_resid64, whose partials follow this kernel's T.nblk blocks).
-template <int OPk, int MODE>
+template <int OPk, int MODE, int TK>
 __global__ void __launch_bounds__(ST, MODE == 1 ? 2 : 4) k_resid64(OpArgs o, Tiling T, const float* __restrict__ b,
                                                 const double* __restrict__ x64, const float* __restrict__ x,
                                                 float* __restrict__ r, Parts P, SolveScalars* sc, int k, int npad,
                                                 const float* __restrict__ qf, double* __restrict__ Pf) {
+  constexpr int TJ = TCELLS / TK, LJ = TJ + 2, LK = TK + 2, NRING = 2 * TK + 2 * TJ;
   if (sc->done) return;
   __shared__ float dtab[8];
   if (threadIdx.x < 8) dtab[threadIdx.x] = (threadIdx.x < 7) ? dinv_tab<float>(o, threadIdx.x) : 1.0f;
@@ -1204,7 +1255,7 @@ __device__ __forceinline__ CgScalars cg_scalars(const Tiling& T, int nres, int f
 // in one fixed order (likewise the true-residual sums of k_slow_resid64).
 // STEADY: a launch with first = 0 and fold = 0 (all but one launch in
 // refine_every), compiled with both as constants so the plane loop carries
-// no branch on them.  XM (steady launches without slow rows): how x advances,
+// no branch on them.  XM (steady launches): how x advances,
 // 1: x += alpha_k-1 p_k-1; 2: not at all (that term stays pending, x is
 // neither read nor written); 3: x = (x + alpha_k-2 p_k-2) + alpha_k-1 p_k-1,
 // the pending term first (p2in = p_k-2, alpha_k-2 as launch k-1 applied it),
@@ -1212,7 +1263,7 @@ __device__ __forceinline__ CgScalars cg_scalars(const Tiling& T, int nres, int f
 // launch after a true-residual pass (first = 0, fold = 1 as constants), whose
 // x64 += x + alpha p reads x64 in the plane pipeline with the vectors.  A
 // launch that stops the solve advances x by all it owes.
-template <int OPk, bool SLOW, bool STEADY, int XM>
+template <int OPk, bool SLOW, bool STEADY, int XM, int TK>
 __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, int nbu, const double* __restrict__ Pprev,
                                                const double* __restrict__ Pres, double* __restrict__ Pout,
                                                const float* __restrict__ rin, const float* __restrict__ qin,
@@ -1221,7 +1272,8 @@ __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, in
                                                float* __restrict__ x, double* __restrict__ x64, int fold,
                                                SolveScalars* sc, int k, double tol, int cap,
                                                const float* __restrict__ p2in) {
-  static_assert(XM == 1 || (STEADY && !SLOW && (XM == 2 || XM == 3)) || (XM == 4 && !STEADY && !SLOW),
+  constexpr int TJ = TCELLS / TK, LJ = TJ + 2, LK = TK + 2, NRING = 2 * TK + 2 * TJ;
+  static_assert(XM == 1 || (STEADY && (XM == 2 || XM == 3)) || (XM == 4 && !STEADY),
                 "x modes 2 and 3 are steady launches, mode 4 the fold launch");
   using V = float;
   // a launch after the one that stopped the solve does nothing (the
@@ -1326,7 +1378,7 @@ __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, in
   // (the slow-row diagonal exists only in the SLOW form: a field that is
   // constant there still shifts the register allocation of the fast form)
   struct RwS {
-    V r, q, p, x, ds;
+    V r, q, p, x, p2, ds;
     uint8_t nb;
   };
   struct RwF {
@@ -1345,7 +1397,7 @@ __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, in
     w.p = (pin + pb)[cv];
     w.x = (with_x && XM != 2) ? (x + pb)[cv] : V(0);
     if constexpr (SLOW) w.ds = ((const V*)o.dslow + pb)[(un && (nb & NB_SLOW) && o.precond) ? c : 0u];
-    else w.p2 = (with_x && XM == 3) ? (p2in + pb)[cv] : V(0);
+    w.p2 = (with_x && XM == 3) ? (p2in + pb)[cv] : V(0);
   };
   // r_k, and p_k = z_k + beta p_{k-1} (0 off the unknowns)
   auto r_of = [&](const Rw& w) -> V { return first ? w.r : w.r - al * w.q; };
@@ -1513,6 +1565,7 @@ __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, in
 // registers) and p_k goes to LDS; q_k of plane i is formed on the tile from
 // the p_k plane.  Loads run two planes ahead of their use (masks three).
 constexpr int SQ = 1024;                     // threads per block
+constexpr int TK = TK_WIDE, TJ = TCELLS / TK, LJ = TJ + 2, LK = TK + 2, NRING = 2 * TK + 2 * TJ;
 constexpr int LJ2 = TJ + 4, LK2 = TK + 4;    // LDS plane with two rings
 constexpr int NRING2 = 2 * TK + 2 * TJ + 4;  // second ring + the first ring's corners
 static_assert(TJ * TK == SQ, "one tile cell per thread");
@@ -1779,26 +1832,17 @@ __global__ void __launch_bounds__(SQ, 4) k_cgq(OpArgs o, Tiling T, int nres, int
 // deterministic.
 template <int OPk>
 __global__ void __launch_bounds__(PB) k_slow_q5(OpArgs o, const uint32_t* __restrict__ list, int64_t n,
-                                                const float* __restrict__ pc, const float* __restrict__ rk,
+                                                const float* __restrict__ sb, const float* __restrict__ pc, const float* __restrict__ rk,
                                                 float* __restrict__ q, double* __restrict__ S7, SolveScalars* sc,
                                                 int k) {
   using V = float;
   if (sc->done) return;  // the solve stopped at launch k: no later launch reads these sums
   double a[FDOT] = {0, 0, 0, 0, 0, 0, 0};  // r.z, r.r are k_cgf's
   {
-    const Grid& g = o.g;
     for (int64_t t = (int64_t)blockIdx.x * PB + threadIdx.x; t < n; t += (int64_t)gridDim.x * PB) {
       const int64_t idx = list[t];
-      int i, j, kk;
-      ijk_of(g, idx, i, j, kk);
-      V pn[6];
-#pragma unroll
-      for (int f = 0; f < 6; ++f) {
-        const int ii = i + c_off[f][0], jj = j + c_off[f][1], k2 = kk + c_off[f][2];
-        pn[f] = valid(g, ii, jj, k2) ? pc[cid(g, ii, jj, k2)] : V(0);
-      }
       const V pcv = pc[idx];
-      const V qv = slow_row<V, OPk>(o, i, j, kk, idx, pcv, pn[0], pn[1], pn[2], pn[3], pn[4], pn[5]);
+      const V qv = slow_row_at<V, OPk>(o, idx, sb, n, t, pc, pcv);
       q[idx] = qv;
       const V r = rk[idx];
       const V dv = o.precond ? dslow_at<V>(o, idx) : V(1);
@@ -1934,10 +1978,13 @@ Launch make_launch(int64_t G) {
 // launch has about `blocks` blocks: one resident round on 256 CUs, i.e. as
 // many 512-thread blocks as fit a CU at the kernel's register use (three for
 // FP32 vectors without slow rows, two otherwise).
-Tiling make_tiling(const Grid& g, int blocks) {
+Tiling make_tiling(const Grid& g, int blocks, int tk) {
   Tiling t;
-  t.ntj = (g.ny + TJ - 1) / TJ;
-  t.ntk = (g.nz + TK - 1) / TK;
+  t.tk = tk;
+  t.ns5 = 0;
+  const int tj = TCELLS / tk;
+  t.ntj = (g.ny + tj - 1) / tj;
+  t.ntk = (g.nz + tk - 1) / tk;
   const int tiles = t.ntj * t.ntk;
   int nseg = blocks / tiles;
   if (nseg < 1) nseg = 1;
@@ -1946,6 +1993,16 @@ Tiling make_tiling(const Grid& g, int blocks) {
   nseg = (g.nx + t.seg - 1) / t.seg;
   t.nblk = tiles * nseg;
   return t;
+}
+
+// Wide tiles read whole 512-byte rows and fewer ring cells per plane; narrow
+// ones pad less where nz ends early in the last wide tile.  A launch costs
+// about (seg + 3) plane steps (three fill the pipeline), a narrow step up to
+// 8/7 of a wide one: 105 us a narrow launch against 94 at 256^3, where both
+// run 32 planes; 56 against 64 at 192^3, 14 planes against 20.
+Tiling make_tiling(const Grid& g, int blocks) {
+  const Tiling w = make_tiling(g, blocks, TK_WIDE), n = make_tiling(g, blocks, TK_NARROW);
+  return 8 * (n.seg + 3) < 7 * (w.seg + 3) ? n : w;
 }
 
 OpArgs make_op(Ctx& c, int precond, int opk) {
@@ -2057,23 +2114,32 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
   if (nslow > 0)
     launch(c, "pcg_slow_list", dim3(nblocks(G, 256)), dim3(256), 0, k_slow_list, G, (const uint8_t*)c.nbm,
            (const uint32_t*)c.count, slow_list);
+  // their face weights in the scratch of the liquid P2G (free during a solve;
+  // 12 floats per cell or more, six values of V are at most 12)
+  V* slow_b = (V*)c.p2g_parts;
+  if (nslow > 0 && OPk != OP_HEAT)
+    launch(c, "pcg_slow_beta", dim3(nblocks(nslow, 256)), dim3(256), 0, k_slow_beta<V, OPk>, o,
+           (const uint32_t*)slow_list, nslow, slow_b);
   // slow-row blocks: grid-stride over the list, at most MAX_BLK of them (the
   // single-kernel iteration sums their partials after its tile blocks, in a
   // region that holds 2 * MAX_BLK blocks)
   int nsb = (int)((nslow + PB - 1) / PB);
   if (nsb > MAX_BLK) nsb = MAX_BLK;
-  auto spmv = nslow > 0 ? k_spmv<V, Dacc, OPk, true> : k_spmv<V, Dacc, OPk, false>;
-  auto resid64 = nslow > 0 ? k_resid64<OPk, 1> : k_resid64<OPk, 0>;
-  // the MIXED form without slow rows runs one kernel per iteration (k_cgf)
-  const bool fused = std::is_same<V, float>::value && mixed && !ref;
+    // the MIXED form without slow rows runs one kernel per iteration (k_cgf)
+  const bool fused = std::is_same<V, float>::value && OPk != OP_HEAT && mixed && !ref;
   // without slow rows the fused iteration can form q_{k-1} again instead of
   // storing q (k_cgq, one 1024-thread block per CU; cfg.pcg_recompute_q)
   const bool qfree = fused && nslow == 0 && c.cfg.pcg_recompute_q;
-  Tiling T = make_tiling(c.g, qfree ? 256 : fused ? 512 : ((sizeof(V) == 4 && nslow == 0) ? 768 : 512));
+  Tiling T = qfree ? make_tiling(c.g, 256, TK_WIDE) : make_tiling(c.g, fused ? 512 : ((sizeof(V) == 4 && nslow == 0) ? 768 : 512));
   T.ns5 = fused ? nsb : 0;
+  const bool wide = T.tk == TK_WIDE;
+  auto spmv = nslow > 0 ? (wide ? k_spmv<V, Dacc, OPk, true, TK_WIDE> : k_spmv<V, Dacc, OPk, true, TK_NARROW>)
+                        : (wide ? k_spmv<V, Dacc, OPk, false, TK_WIDE> : k_spmv<V, Dacc, OPk, false, TK_NARROW>);
+  auto resid64 = nslow > 0 ? (wide ? k_resid64<OPk, 1, TK_WIDE> : k_resid64<OPk, 1, TK_NARROW>)
+                           : (wide ? k_resid64<OPk, 0, TK_WIDE> : k_resid64<OPk, 0, TK_NARROW>);
   // the true-residual pass keeps two 512-thread blocks per CU (its own
   // tiling when k_cgq runs one block per CU); its partial count is Tr.nblk
-  Tiling Tr = qfree ? make_tiling(c.g, 512) : T;
+  Tiling Tr = qfree ? make_tiling(c.g, 512, TK_WIDE) : T;
   Tr.ns5 = T.ns5;
   // U-slot partials: update and init write L.nblk, the residual pass T.nblk;
   // both pad to npad, the count the spmv sums
@@ -2093,7 +2159,7 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
   int restarts = 0;
   bool true_missed = false;
   double prev_true_rr = -1.0;  // FP64 true r.r at the last restart (stagnation test)
-  if constexpr (std::is_same<V, float>::value) {
+  if constexpr (std::is_same<V, float>::value && OPk != OP_HEAT) {
     if (fused) {
       float* rb[2] = {(float*)c.vr, (float*)c.vr2};
       float* qb[2] = {(float*)c.vq, (float*)c.vq2};
@@ -2102,15 +2168,30 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
       // partial sums: per launch T.nblk tile blocks then T.ns5 slow-row blocks
       double* S7[2] = {c.partials + 8 * MAX_BLK, c.partials + 22 * MAX_BLK};
       double* Rs = c.partials + 36 * MAX_BLK;
-      auto cg_iter = nslow > 0 ? k_cgf<OPk, true, false, 1> : k_cgf<OPk, false, false, 1>;
-      auto cg_steady = nslow > 0 ? k_cgf<OPk, true, true, 1> : k_cgf<OPk, false, true, 1>;
-      // without slow rows x advances every other launch (modes 2 and 3 of
-      // k_cgf), and fully before each true-residual pass
-      auto cg_skip = k_cgf<OPk, false, true, 2>;
-      auto cg_double = k_cgf<OPk, false, true, 3>;
-      auto cg_fold = k_cgf<OPk, false, false, 4>;  // x64 += x + alpha p after a true residual
+      // x advances every other launch (modes 2 and 3 of k_cgf), and fully
+      // before each true-residual pass; not with slow rows on wide tiles,
+      // whose mode 3 spills (89 and 124 us a launch in turn against 105 at
+      // 256^3; on narrow tiles 46 and 58 against 55 at 192^3)
+      struct Iter {
+        decltype(&k_cgf<OPk, false, false, 1, TK_WIDE>) any, steady, skip, twice, fold;
+      };
+#define MPF_ITER(SL, W) \
+  Iter { k_cgf<OPk, SL, false, 1, W>, k_cgf<OPk, SL, true, 1, W>, k_cgf<OPk, SL, true, 2, W>, \
+         k_cgf<OPk, SL, true, 3, W>, k_cgf<OPk, SL, false, 4, W> }
+      Iter it = wide ? MPF_ITER(false, TK_WIDE) : MPF_ITER(false, TK_NARROW);
+      bool halves = true;
+      if constexpr (OPk == OP_VARDENS) {
+        if (nslow > 0 && wide) {
+          it.any = it.fold = k_cgf<OPk, true, false, 1, TK_WIDE>;
+          it.steady = k_cgf<OPk, true, true, 1, TK_WIDE>;
+          halves = false;
+        } else if (nslow > 0) {
+          it = MPF_ITER(true, TK_NARROW);
+        }
+      }
+#undef MPF_ITER
       bool pending = false;  // the last launch left alpha p in x's debt
-      auto res_tiles = nslow > 0 ? k_resid64<OPk, 2> : k_resid64<OPk, 0>;
+      auto res_tiles = nslow > 0 ? (wide ? k_resid64<OPk, 2, TK_WIDE> : k_resid64<OPk, 2, TK_NARROW>) : resid64;
       // FP64 true residual: the tile pass, then the slow rows' list pass
       auto true_resid = [&](int kk, float* rr_, const float* qq_) {
         launch(c, "pcg_resid64", dim3(Tr.nblk), dim3(ST), 0, res_tiles, o, Tr, (const float*)b, (const double*)x64,
@@ -2134,21 +2215,19 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
                    rb[(k + 1) & 1], p_next, (k + 1) % R == 0 ? qb[(k + 1) & 1] : (float*)nullptr, (float*)x, x64,
                    fold, c.scal, k, tol, cap);
           } else {
-            auto kern = cg_iter;
+            auto kern = it.any;
             if (first == 0 && fold == 0) {
-              kern = cg_steady;
-              if (nslow == 0) {
-                if (pending) {
-                  kern = cg_double;
-                  pending = false;
-                } else if ((k + 1) % R != 0 && k < cap) {
-                  kern = cg_skip;
-                  pending = true;
-                }
+              kern = it.steady;
+              if (pending) {
+                kern = it.twice;
+                pending = false;
+              } else if (halves && (k + 1) % R != 0 && k < cap) {
+                kern = it.skip;
+                pending = true;
               }
             } else {
               pending = false;
-              if (first == 0 && nslow == 0) kern = cg_fold;
+              if (first == 0) kern = it.fold;
             }
             launch(c, "pcg_cg_iter", dim3(T.nblk), dim3(ST), 0, kern, o, T, first, npad,
                    (const double*)S7[(k + 1) & 1], pres, S7[k & 1], (const float*)rb[k & 1],
@@ -2157,7 +2236,7 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
           }
           if (nslow > 0)
             launch(c, "pcg_slow_q5", dim3(nsb), dim3(PB), 0, k_slow_q5<OPk>, o, (const uint32_t*)slow_list, nslow,
-                   (const float*)p_next, (const float*)rb[(k + 1) & 1], qb[(k + 1) & 1], S7[k & 1] + FDOT * T.nblk,
+                   (const float*)slow_b, (const float*)p_next, (const float*)rb[(k + 1) & 1], qb[(k + 1) & 1], S7[k & 1] + FDOT * T.nblk,
                    c.scal, k);
           first = 0;
           fold = 0;
@@ -2212,7 +2291,7 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
                pbuf[(k + 1) & 1], q, P, c.scal, k, (int)ref, eps_abs, tol, cap);
         if (nsb > 0)
           launch(c, "pcg_slow_q", dim3(nsb), dim3(PB), 0, k_slow_q<V, Dacc, OPk>, o, (const uint32_t*)slow_list, nslow,
-                 (const V*)pbuf[(k + 1) & 1], q, P.S2, c.scal);
+                 (const V*)slow_b, (const V*)pbuf[(k + 1) & 1], q, P.S2, c.scal);
         const bool resid_next = mixed && (k + 1) % R == 0;
         const bool h = (k % 2 == 0) && !resid_next && !fold_next;
         const int mode = h ? 0 : ((k > 0 && half[k - 1]) ? 2 : 1);
