@@ -58,8 +58,9 @@ __device__ __forceinline__ void wave_runs(bool act, uint32_t k, bool& head, int&
   headlane = below ? (63 - __clzll((long long)below)) : 0;
 }
 
+// rank: the particle's place among its cell's, in the order the atomics came.
 __global__ void k_hash_count(Grid g, const f3* __restrict__ pos, int64_t P, uint32_t* __restrict__ key,
-                             uint32_t* __restrict__ count) {
+                             uint32_t* __restrict__ rank, uint32_t* __restrict__ count) {
   int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   bool act = p < P;
   uint32_t k = 0xffffffffu;
@@ -70,25 +71,22 @@ __global__ void k_hash_count(Grid g, const f3* __restrict__ pos, int64_t P, uint
   bool head;
   int runlen, headlane;
   wave_runs(act, k, head, runlen, headlane);
-  if (head) atomicAdd(&count[k], (uint32_t)runlen);
+  uint32_t base = 0;
+  if (head) base = atomicAdd(&count[k], (uint32_t)runlen);
+  base = __shfl(base, headlane);
+  if (act) rank[p] = base + (uint32_t)(lane_id() - headlane);
 }
 
-__global__ void k_scatter(int64_t P, const uint32_t* __restrict__ key, uint32_t* __restrict__ cursor,
-                          uint32_t* __restrict__ perm, uint32_t* __restrict__ skey) {
+// Every particle's cell has a start, so no atomics here.
+__global__ void k_scatter(int64_t P, const uint32_t* __restrict__ key, const uint32_t* __restrict__ rank,
+                          const uint32_t* __restrict__ cstart, uint32_t* __restrict__ perm,
+                          uint32_t* __restrict__ skey) {
   int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  bool act = p < P;
-  uint32_t k = act ? key[p] : 0xffffffffu;
-  bool head;
-  int runlen, headlane;
-  wave_runs(act, k, head, runlen, headlane);
-  uint32_t base = 0;
-  if (head) base = atomicAdd(&cursor[k], (uint32_t)runlen);
-  base = __shfl(base, headlane);
-  if (act) {
-    uint32_t slot = base + (uint32_t)(lane_id() - headlane);
-    perm[slot] = (uint32_t)p;
-    skey[slot] = k;
-  }
+  if (p >= P) return;
+  const uint32_t k = key[p];
+  const uint32_t slot = cstart[k] + rank[p];
+  perm[slot] = (uint32_t)p;
+  skey[slot] = k;
 }
 
 // Keyless variants for mpf_hash_sort_noalloc: the count goes straight into
@@ -125,17 +123,6 @@ __global__ void k_scatter_rehash(Grid g, const f3* __restrict__ pos, int64_t P, 
 __global__ void k_fill_u32(int64_t n, uint32_t* __restrict__ v, uint32_t x) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) v[i] = x;
-}
-
-// counts (in cend) + exclusive scan (in cstart) -> cstart = start or UNDEF,
-// cend = start as the scatter cursor (UNDEF when empty); the scatter then
-// advances each non-empty cell's cursor to its end.
-__global__ void k_cells_cursor(int64_t G, uint32_t* __restrict__ cstart, uint32_t* __restrict__ cend) {
-  int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= G) return;
-  const uint32_t n = cend[c], s = cstart[c];
-  cstart[c] = n ? s : MPF_CELL_UNDEF;
-  cend[c] = n ? s : MPF_CELL_UNDEF;
 }
 
 template <int N>
@@ -221,17 +208,6 @@ __global__ void k_reorder(int64_t P, const uint32_t* __restrict__ perm,
   olheat[s] = ilheat[p];
   osolub[s] = isolub[p];
   ogas[s] = igas[p];
-}
-
-// counts -> cell_start / cell_end (UNDEF when empty) and scatter cursors.
-__global__ void k_cells_from_scan(int64_t G, uint32_t* __restrict__ count, uint32_t* __restrict__ cstart,
-                                  uint32_t* __restrict__ cend) {
-  int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= G) return;
-  uint32_t n = count[c], s = cstart[c];
-  count[c] = s;
-  cstart[c] = n ? s : MPF_CELL_UNDEF;
-  cend[c] = n ? s + n : MPF_CELL_UNDEF;
 }
 
 __global__ void k_cell_mask(int64_t G, const uint32_t* __restrict__ cstart, const uint32_t* __restrict__ cend,
@@ -328,15 +304,36 @@ __global__ void k_scan_blocks(uint32_t* blk, int64_t nb) {
   if (threadIdx.x == 0) blk[nb] = carry;
 }
 
-__global__ void k_scan_apply(const uint32_t* __restrict__ in, int64_t n, const uint32_t* __restrict__ blk,
-                             uint32_t* __restrict__ out) {
+// The exclusive scan of in, tile by tile.  blk: the tiles' exclusive prefixes
+// (own = false), or their sums, of which each block adds up those before it
+// (own = true: one launch less; the last block then leaves the total at
+// blk[nb], as k_scan_blocks does).  What is written (in and end may be one):
+enum { SCAN_PLAIN, SCAN_CELLS, SCAN_CURSORS };
+// SCAN_PLAIN    out = prefix
+// SCAN_CELLS    counts -> out = start, end = end of each cell's particles
+// SCAN_CURSORS  counts -> out = start, end = start (a scatter's cursor)
+// (cells without particles: MPF_CELL_UNDEF in both)
+template <int KIND>
+__global__ void k_scan_apply(const uint32_t* in, int64_t n, uint32_t* blk, bool own, uint32_t* __restrict__ out,
+                             uint32_t* end) {
   __shared__ uint32_t tile[SCAN_TILE + SCAN_TILE / 16];
   __shared__ uint32_t wsum[SCAN_THREADS / 64];
   int64_t base = (int64_t)blockIdx.x * SCAN_TILE;
+  uint32_t cnt[SCAN_PER_THREAD];
+#pragma unroll
   for (int q = 0; q < SCAN_PER_THREAD; ++q) {
     int e = q * SCAN_THREADS + threadIdx.x;
     int64_t ge = base + e;
-    tile[e + (e >> 4)] = (ge < n) ? in[ge] : 0u;
+    cnt[q] = (ge < n) ? in[ge] : 0u;
+    tile[e + (e >> 4)] = cnt[q];
+  }
+  uint32_t before;
+  if (own) {
+    uint32_t s = 0;
+    for (uint32_t e = threadIdx.x; e < blockIdx.x; e += SCAN_THREADS) s += blk[e];
+    block_excl_scan(s, wsum, before);
+  } else {
+    before = blk[blockIdx.x];
   }
   __syncthreads();
   uint32_t loc[SCAN_PER_THREAD];
@@ -349,19 +346,32 @@ __global__ void k_scan_apply(const uint32_t* __restrict__ in, int64_t n, const u
     run += tile[e + (e >> 4)];
   }
   uint32_t total;
-  uint32_t off = block_excl_scan(run, wsum, total) + blk[blockIdx.x];
+  uint32_t off = block_excl_scan(run, wsum, total) + before;
 #pragma unroll
   for (int q = 0; q < SCAN_PER_THREAD; ++q) {
     int e = t0 + q;
     tile[e + (e >> 4)] = loc[q] + off;
   }
+  if (own && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) blk[gridDim.x] = before + total;
   __syncthreads();
+#pragma unroll
   for (int q = 0; q < SCAN_PER_THREAD; ++q) {
     int e = q * SCAN_THREADS + threadIdx.x;
     int64_t ge = base + e;
-    if (ge < n) out[ge] = tile[e + (e >> 4)];
+    if (ge >= n) continue;
+    const uint32_t s = tile[e + (e >> 4)];
+    if (KIND == SCAN_PLAIN) {
+      out[ge] = s;
+    } else {
+      out[ge] = cnt[q] ? s : MPF_CELL_UNDEF;
+      end[ge] = !cnt[q] ? MPF_CELL_UNDEF : (KIND == SCAN_CELLS) ? s + cnt[q] : s;
+    }
   }
 }
+
+// A grid's tiles up to which each block adds the sums before its own itself:
+// one block's scan of 4096 sums takes 12 us, their reads by all blocks less.
+constexpr int64_t SCAN_OWN_TILES = 4096;
 
 }  // namespace
 
@@ -370,7 +380,8 @@ __global__ void k_iota(int64_t n, uint32_t* __restrict__ v) {
   if (i < n) v[i] = (uint32_t)i;
 }
 
-int64_t run_scan_u32(Ctx& c, const uint32_t* in, uint32_t* out, int64_t n, bool want_total) {
+template <int KIND>
+static int64_t scan(Ctx& c, const uint32_t* in, uint32_t* out, uint32_t* end, int64_t n, bool want_total) {
   if (n <= 0) return 0;
   int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
   if (nb + 1 > c.scan_blk_n) {
@@ -378,15 +389,20 @@ int64_t run_scan_u32(Ctx& c, const uint32_t* in, uint32_t* out, int64_t n, bool 
     return -1;
   }
   launch(c, "scan_reduce", dim3((unsigned)nb), dim3(SCAN_THREADS), 0, k_scan_reduce, in, n, c.scan_blk);
-  launch(c, "scan_blocks", dim3(1), dim3(SCAN_THREADS), 0, k_scan_blocks, c.scan_blk, nb);
-  launch(c, "scan_apply", dim3((unsigned)nb), dim3(SCAN_THREADS), 0, k_scan_apply, in, n,
-         (const uint32_t*)c.scan_blk, out);
+  const bool own = nb <= SCAN_OWN_TILES;
+  if (!own) launch(c, "scan_blocks", dim3(1), dim3(SCAN_THREADS), 0, k_scan_blocks, c.scan_blk, nb);
+  launch(c, KIND == SCAN_PLAIN ? "scan_apply" : "cells_from_scan", dim3((unsigned)nb), dim3(SCAN_THREADS), 0,
+         k_scan_apply<KIND>, in, n, c.scan_blk, own, out, end);
   if (!want_total) return 0;
   uint32_t tot = 0;
   hipMemcpyAsync(c.counters_host + 15, c.scan_blk + nb, 4, hipMemcpyDeviceToHost, c.stream);
   hipStreamSynchronize(c.stream);
   tot = c.counters_host[15];
   return (int64_t)tot;
+}
+
+int64_t run_scan_u32(Ctx& c, const uint32_t* in, uint32_t* out, int64_t n, bool want_total) {
+  return scan<SCAN_PLAIN>(c, in, out, nullptr, n, want_total);
 }
 
 int64_t run_check_cells(Ctx& c) {
@@ -416,14 +432,13 @@ void run_hash_sort(Ctx& c) {
     run_cell_mask(c);
     return;
   }
+  uint32_t* rank = (uint32_t*)c.temp[nxt];  // the reorder's output, free until then
   hipMemsetAsync(c.count, 0, (size_t)G * 4, c.stream);
   launch(c, "hash_count", dim3(nblocks(P, 256)), dim3(256), 0, k_hash_count, c.g, (const f3*)c.pos[cur], P,
-         c.key, c.count);
-  run_scan_u32(c, c.count, c.cstart, G, false);
-  launch(c, "cells_from_scan", dim3(nblocks(G, 256)), dim3(256), 0, k_cells_from_scan, G, c.count, c.cstart,
-         c.cend);
-  launch(c, "scatter", dim3(nblocks(P, 256)), dim3(256), 0, k_scatter, P, (const uint32_t*)c.key, c.count,
-         c.perm, c.ghash);
+         c.key, rank, c.count);
+  scan<SCAN_CELLS>(c, c.count, c.cstart, c.cend, G, false);
+  launch(c, "scatter", dim3(nblocks(P, 256)), dim3(256), 0, k_scatter, P, (const uint32_t*)c.key,
+         (const uint32_t*)rank, (const uint32_t*)c.cstart, c.perm, c.ghash);
   launch(c, "segsort", dim3(nblocks(G, 256)), dim3(256), 0, k_segsort, G, (const uint32_t*)c.cstart,
          (const uint32_t*)c.cend, c.perm);
   launch(c, "reorder", dim3(nblocks(P, 256)), dim3(256), 0, k_reorder, P, (const uint32_t*)c.perm,
@@ -446,14 +461,13 @@ void run_hash_sort(Ctx& c) {
 void run_hash_sort_mc(Ctx& c) {
   const int64_t P = c.P, G2 = c.g2.G;
   const int cur = c.cur, nxt = 1 - c.cur;
+  uint32_t* rank = (uint32_t*)c.temp[nxt];
   hipMemsetAsync(c.mc_count, 0, (size_t)G2 * 4, c.stream);
   launch(c, "mc_hash_count", dim3(nblocks(P, 256)), dim3(256), 0, k_hash_count, c.g2, (const f3*)c.pos[cur], P,
-         c.key, c.mc_count);
-  run_scan_u32(c, c.mc_count, c.mc_cstart, G2, false);
-  launch(c, "mc_cells_from_scan", dim3(nblocks(G2, 256)), dim3(256), 0, k_cells_from_scan, G2, c.mc_count,
-         c.mc_cstart, c.mc_cend);
-  launch(c, "mc_scatter", dim3(nblocks(P, 256)), dim3(256), 0, k_scatter, P, (const uint32_t*)c.key, c.mc_count,
-         c.perm, c.ghash);
+         c.key, rank, c.mc_count);
+  scan<SCAN_CELLS>(c, c.mc_count, c.mc_cstart, c.mc_cend, G2, false);
+  launch(c, "mc_scatter", dim3(nblocks(P, 256)), dim3(256), 0, k_scatter, P, (const uint32_t*)c.key,
+         (const uint32_t*)rank, (const uint32_t*)c.mc_cstart, c.perm, c.ghash);
   launch(c, "mc_segsort", dim3(nblocks(G2, 256)), dim3(256), 0, k_segsort, G2, (const uint32_t*)c.mc_cstart,
          (const uint32_t*)c.mc_cend, c.perm);
   launch(c, "mc_reorder", dim3(nblocks(P, 256)), dim3(256), 0, k_reorder, P, (const uint32_t*)c.perm,
@@ -546,10 +560,10 @@ extern "C" mpf_status mpf_hash_sort_noalloc(const mpf_config* cfg, int64_t n, co
     hipLaunchKernelGGL(k_hash_count_nokey, dim3(nblocks(n, 256)), dim3(256), 0, st, g, p3, n, cell_end);
     hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SCAN_THREADS), 0, st, (const uint32_t*)cell_end, G,
                        blk);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(SCAN_THREADS), 0, st, blk, nb);
-    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(SCAN_THREADS), 0, st, (const uint32_t*)cell_end, G,
-                       (const uint32_t*)blk, cell_start);
-    hipLaunchKernelGGL(k_cells_cursor, dim3(nblocks(G, 256)), dim3(256), 0, st, G, cell_start, cell_end);
+    const bool own = nb <= SCAN_OWN_TILES;
+    if (!own) hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(SCAN_THREADS), 0, st, blk, nb);
+    hipLaunchKernelGGL(k_scan_apply<SCAN_CURSORS>, dim3((unsigned)nb), dim3(SCAN_THREADS), 0, st,
+                       (const uint32_t*)cell_end, G, blk, own, cell_start, cell_end);
     hipLaunchKernelGGL(k_scatter_rehash, dim3(nblocks(n, 256)), dim3(256), 0, st, g, p3, n, cell_end, grid_index,
                        grid_hash);
     hipLaunchKernelGGL(k_segsort, dim3(nblocks(G, 256)), dim3(256), 0, st, G, (const uint32_t*)cell_start,
