@@ -323,14 +323,34 @@ __global__ void k_sph_force(Grid g, int64_t P, const f3* __restrict__ pos, const
 // (the bound keeps a margin against the rounding of the cell boundaries), and
 // a pair is evaluated only when its squared distance is below re^2 (1 + 2^-19),
 // a bound under which the rounded quotient d^2/re^2 is always >= 1.
-constexpr int CP_LIST = 16;  // in-range neighbours listed per thread before a drain
+//
+// Two passes.  The first reads distances only, row by row of the reachable
+// cells: with the library's own sort the cells (k-1, k, k+1) of a row are one
+// range of particles (ROWS; lists given by the caller: a cell at a time).  The
+// in-range ones of up to 32 particles are bits of a word; a cell's non-empty
+// word goes to the thread's list in LDS (first particle, bits), the first of
+// each cell marked.  The second pass takes the bits in the reference's order
+// (cells by offset, particles by index) and evaluates the spring terms, adding
+// the running cell subtotal to the spring at each mark (sumcellspring returns
+// one subtotal per cell; cells without an in-range neighbour add +-0).  A wave
+// then pays the spring arithmetic for its lane with the most in-range
+// neighbours, not for every candidate any lane has in range.  A full list is
+// drained and refilled.  The particle itself adds nothing and is not listed.
+// Bound by issuing vector instructions: about 11 per candidate here, 27 when
+// each candidate was bounds-checked, listed and counted by itself (9.1M
+// particles 0.97 -> 0.75 ms, 89.6M 9.2 -> 7.4 ms).
+constexpr int CP_LIST = 12;  // words listed per thread before a drain (three a row at most)
+__device__ __forceinline__ uint32_t low_bits(uint32_t n) { return n >= 32u ? 0xffffffffu : (1u << n) - 1u; }
+
+template <bool ROWS>
 __global__ void __launch_bounds__(256) k_correct_pos(Grid g, int64_t P, const f3* __restrict__ pin, f3* __restrict__ pout,
                               const float* __restrict__ mass, const int8_t* __restrict__ flag,
                               const uint32_t* __restrict__ cstart, const uint32_t* __restrict__ cend, float spring_k,
                               float radius, float ss, float dt) {
-  __shared__ uint32_t lds_hits[CP_LIST][256];  // blockDim.x == 256
-  const int64_t p = xcd_block() * blockDim.x + threadIdx.x;
-  if (p >= P) return;
+  __shared__ uint32_t hit_q[CP_LIST][256], hit_m[CP_LIST][256];  // blockDim.x == 256
+  const int64_t pp = xcd_block() * blockDim.x + threadIdx.x;
+  if (pp >= P) return;
+  const uint32_t p = (uint32_t)pp;
   const int8_t fl = flag[p];
   f3 x = pin[p];
   if (fl == SOLID || fl == AIRSOLO) {
@@ -352,102 +372,137 @@ __global__ void __launch_bounds__(256) k_correct_pos(Grid g, int64_t P, const f3
   // when that gap is below re
   const float mg = 1e-3f * hh;
   const float lx = (x.x - g.gx0) - (float)i * hh, ly = (x.y - g.gy0) - (float)j * hh, lz = (x.z - g.gz0) - (float)k * hh;
-  const float gl[3] = {lx - mg, ly - mg, lz - mg};
-  const float gh[3] = {hh - lx - mg, hh - ly - mg, hh - lz - mg};
-  auto gap = [&](int a, int d) -> float {
-    const float v = d < 0 ? gl[a] : (d > 0 ? gh[a] : 0.0f);
-    return v > 0.0f ? v : 0.0f;
+  // squared gaps of the sides -1, 0, +1 (off the grid: NaN, never reachable)
+  auto gaps = [&](float l, int c, int n, float (&sq)[3]) {
+    const float lo = l - mg, hi = hh - l - mg;
+    const float a = lo > 0.0f ? lo : 0.0f, b = hi > 0.0f ? hi : 0.0f;
+    sq[0] = c > 0 ? a * a : __builtin_nanf("");
+    sq[1] = 0.0f;
+    sq[2] = c + 1 < n ? b * b : __builtin_nanf("");
   };
+  float gx[3], gy[3], gz[3];
+  gaps(lx, i, g.nx, gx);
+  gaps(ly, j, g.ny, gy);
+  gaps(lz, k, g.nz, gz);
   // the reachable cells, as bits of the 27 offsets in the reference's order
   uint32_t cand = 0;
-  for (int o = 0; o < 27; ++o) {
-    const int di = o / 9 - 1, dj = (o / 3) % 3 - 1, dk = o % 3 - 1;
-    if (!valid(g, i + di, j + dj, k + dk)) continue;
-    const float gx = gap(0, di), gy = gap(1, dj), gz = gap(2, dk);
-    if (gx * gx + gy * gy + gz * gz <= cut) cand |= 1u << o;
-  }
-  // Two passes.  The first reads distances only: the in-range neighbours of
-  // the reachable cells (cells by offset, particles by index, the reference's
-  // order) go to this thread's list in LDS, the first of each cell marked.
-  // The second evaluates the spring terms of the list, adding the running
-  // cell subtotal to the spring at each mark (sumcellspring returns one
-  // subtotal per cell; cells without an in-range neighbour add +-0).  A wave
-  // then pays the spring arithmetic for its lane with the most in-range
-  // neighbours, not for every candidate any lane has in range.  A full list
-  // is drained and refilled.  The particle itself (d = 0) adds nothing and
-  // is not listed.
-  uint32_t(*hits)[256] = lds_hits;
+#pragma unroll
+  for (int o = 0; o < 27; ++o)
+    cand |= (gx[o / 9] + gy[(o / 3) % 3] + gz[o % 3] <= cut) ? 1u << o : 0u;
   const int tid = threadIdx.x;
-  int nh = 0;
+  int ne = 0;
   f3 sc = mk3(0.0f, 0.0f, 0.0f);
   auto drain = [&]() {
-    if (nh == 0) return;
-    uint32_t e = hits[0][tid];
-    f3 y = pin[e & 0x7fffffffu];
-    float m = mass[e & 0x7fffffffu];
-    for (int h = 0; h < nh; ++h) {
-      const uint32_t ec = e;
-      const f3 yc = y;
-      const float mc = m;
-      if (h + 1 < nh) {  // next entry's loads in flight during this one
-        e = hits[h + 1][tid];
-        y = pin[e & 0x7fffffffu];
-        m = mass[e & 0x7fffffffu];
+    int ei = 0;
+    uint32_t b = 0, w = 0;
+    auto next = [&](uint32_t& q) -> bool {
+      if (w == 0) {
+        if (ei == ne) return false;
+        b = hit_q[ei][tid];
+        w = hit_m[ei][tid];
+        ++ei;
       }
-      if (ec >> 31) {
+      q = b + (uint32_t)(__ffs(w) - 1);
+      b &= 0x7fffffffu;
+      w &= w - 1u;
+      return true;
+    };
+    uint32_t q = 0;
+    bool more = next(q);
+    f3 y = pin[q & 0x7fffffffu];
+    float my = mass[q & 0x7fffffffu];
+    while (more) {
+      const uint32_t qc = q;
+      const f3 yc = y;
+      const float mc = my;
+      more = next(q);  // the next one's loads in flight during this one
+      y = pin[q & 0x7fffffffu];
+      my = mass[q & 0x7fffffffu];
+      if (qc >> 31) {
         spring = add3(spring, sc);
         sc = mk3(0.0f, 0.0f, 0.0f);
       }
       const f3 dd = sub3(yc, x);
       const float d2 = dot3(dd, dd);
       const float dist = sqrtf(d2);
-      const float w = mc * fmaxf(1.0f - (dist * dist) / (re * re), 0.0f);
-      if (dist > 0.1f * re) sc = add3(sc, div3(smul3(w, sub3(x, yc)), dist));
+      const float wt = mc * fmaxf(1.0f - (dist * dist) / (re * re), 0.0f);
+      if (dist > 0.1f * re) sc = add3(sc, div3(smul3(wt, sub3(x, yc)), dist));
     }
-    nh = 0;
+    ne = 0;
   };
-  // up to 8 cells at a time: their ranges read together, then each cell's
-  // particles four at a time (positions in flight together)
-  constexpr int NCB = 8;
-  while (cand) {
-    uint32_t cs[NCB], ce[NCB];
-    int nc = 0;
-#pragma unroll
-    for (int t = 0; t < NCB; ++t) {
-      int64_t c = 0;
-      if (cand) {
-        const int o = __ffs(cand) - 1;
-        cand &= cand - 1u;
-        c = cid(g, i + o / 9 - 1, j + (o / 3) % 3 - 1, k + o % 3 - 1);
-        nc = t + 1;
-      }
-      cs[t] = cstart[c];
-      ce[t] = cend[c];
-    }
-#pragma unroll
-    for (int t = 0; t < NCB; ++t) {
-      if (t >= nc) break;
-      const uint32_t s0 = cs[t];
-      if (s0 == MPF_CELL_UNDEF) continue;
-      const uint32_t e0 = ce[t];
-      uint32_t mark = 0x80000000u;
-      for (uint32_t q0 = s0; q0 < e0; q0 += 4) {
+  // particles [s, e): those of the first cell below ea, of the second below
+  // eb.  Reads up to three positions past e (the array is that much longer).
+  auto visit = [&](uint32_t s, uint32_t ea, uint32_t eb, uint32_t e) {
+    uint32_t ma = 0x80000000u, mb = 0x80000000u, mc = 0x80000000u;  // marks: first word of each cell
+    for (uint32_t c0 = s; c0 < e; c0 += 32) {
+      const uint32_t n = e - c0;
+      const f3* __restrict__ yp = pin + c0;
+      uint32_t w = 0;
+      for (uint32_t u0 = 0; u0 < 32 && u0 < n; u0 += 4) {
         f3 y4[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) y4[u] = pin[min(q0 + (uint32_t)u, e0 - 1u)];
+        for (int u = 0; u < 4; ++u) y4[u] = yp[u0 + u];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const uint32_t q = q0 + (uint32_t)u;
-          if (q >= e0) break;
           const f3 dd = sub3(y4[u], x);
-          const float d2 = dot3(dd, dd);
-          if (!(d2 < cut) || (int64_t)q == p) continue;
-          if (nh == CP_LIST) drain();
-          hits[nh][tid] = q | mark;
-          mark = 0;
-          ++nh;
+          w |= dot3(dd, dd) < cut ? 1u << (u0 + u) : 0u;
         }
       }
+      w &= low_bits(n);
+      if (p - c0 < 32u) w &= ~(1u << (p - c0));
+      if (ne > CP_LIST - 3) drain();
+      auto push = [&](uint32_t bits, uint32_t& mark) {
+        if (!bits) return;
+        hit_q[ne][tid] = c0 | mark;
+        hit_m[ne][tid] = bits;
+        mark = 0;
+        ++ne;
+      };
+      if (ROWS) {
+        const uint32_t la = low_bits(ea > c0 ? ea - c0 : 0u), lb = low_bits(eb > c0 ? eb - c0 : 0u);
+        push(w & la, ma);
+        push(w & lb & ~la, mb);
+        push(w & ~lb, mc);
+      } else {
+        push(w, ma);
+      }
+    }
+  };
+  // a few rows (cells) at a time: their ranges read together
+  const uint32_t cell = (uint32_t)cid(g, i, j, k);
+  const int sx = g.ny * g.nz, sy = g.nz;
+  if (ROWS) {
+    constexpr int NR = 4;
+    while (cand) {
+      uint32_t S[NR], EA[NR], EB[NR], E[NR];
+#pragma unroll
+      for (int t = 0; t < NR; ++t) {
+        const int r = cand ? (__ffs(cand) - 1) / 3 : 4;
+        const uint32_t bits = (cand >> (3 * r)) & 7u;
+        cand &= ~(7u << (3 * r));
+        const uint32_t c = cell + (uint32_t)((r / 3 - 1) * sx + (r % 3 - 1) * sy);
+        const uint32_t cl = (bits & 1u) ? c - 1u : cell, cm = (bits & 2u) ? c : cell, cr = (bits & 4u) ? c + 1u : cell;
+        const uint32_t s0 = cstart[cl], s1 = cstart[cm], s2 = cstart[cr];
+        const uint32_t e0 = cend[cl], e1 = cend[cm], e2 = cend[cr];
+        const bool h0 = (bits & 1u) && s0 != MPF_CELL_UNDEF, h1 = (bits & 2u) && s1 != MPF_CELL_UNDEF,
+                   h2 = (bits & 4u) && s2 != MPF_CELL_UNDEF;
+        S[t] = h0 ? s0 : (h1 ? s1 : (h2 ? s2 : 0u));
+        EA[t] = h0 ? e0 : S[t];
+        EB[t] = h1 ? e1 : EA[t];
+        E[t] = h2 ? e2 : EB[t];
+      }
+#pragma unroll
+      for (int t = 0; t < NR; ++t) visit(S[t], EA[t], EB[t], E[t]);
+    }
+  } else {
+    while (cand) {
+      const int o = __ffs(cand) - 1;
+      cand &= cand - 1u;
+      const uint32_t c = cell + (uint32_t)((o / 9 - 1) * sx + ((o / 3) % 3 - 1) * sy + (o % 3 - 1));
+      const uint32_t s = cstart[c];
+      if (s == MPF_CELL_UNDEF) continue;
+      const uint32_t e = cend[c];
+      visit(s, e, e, e);
     }
   }
   drain();
@@ -603,7 +658,8 @@ void run_solo_air_sph(Ctx& c) {
 
 void run_correct_pos(Ctx& c) {
   const int cur = c.cur, nxt = 1 - c.cur;
-  launch(c, "correct_pos", dim3(nblocks(c.P, 256)), dim3(256), 0, k_correct_pos, c.g, c.P, (const f3*)c.pos[cur],
+  auto kern = c.own_sort ? k_correct_pos<true> : k_correct_pos<false>;
+  launch(c, "correct_pos", dim3(nblocks(c.P, 256)), dim3(256), 0, kern, c.g, c.P, (const f3*)c.pos[cur],
          c.pos[nxt], (const float*)c.mass[cur], (const int8_t*)c.flag[cur], (const uint32_t*)c.cstart,
          (const uint32_t*)c.cend, c.cfg.correction_spring, c.cfg.correction_radius, c.cfg.samplespace, c.cfg.dt);
   std::swap(c.pos[cur], c.pos[nxt]);

@@ -163,7 +163,9 @@ bool alloc_all(Ctx& c) {
   const int64_t fc[3] = {c.g.FX, c.g.FY, c.g.FZ};
   bool ok = true;
   for (int b = 0; b < 2 && ok; ++b) {
-    ok = ok && dalloc(c, c.pos[b], cap) && dalloc(c, c.vel[b], cap) && dalloc(c, c.flag[b], cap) &&
+    // (+8: the level set and the position correction read positions and flags
+    // up to eight at a time from the first of a cell)
+    ok = ok && dalloc(c, c.pos[b], cap + 8) && dalloc(c, c.vel[b], cap) && dalloc(c, c.flag[b], cap + 8) &&
          dalloc(c, c.mass[b], cap) && dalloc(c, c.temp[b], cap) && dalloc(c, c.lheat[b], cap) &&
          dalloc(c, c.solub[b], cap) && dalloc(c, c.gas[b], cap);
   }
