@@ -5,6 +5,7 @@
 // order, positions) and holds every discrete decision of that call fixed.
 // Cotangents are FP64.
 #include "interp.h"
+#include "row_bits.h"
 #include "mpf_internal.h"
 
 #include <algorithm>
@@ -141,7 +142,8 @@ constexpr int AIR_LANES = 8;
 // The occupancy masks of the sort, which the forward call goes by too, leave
 // out the cells and bricks without a particle of the phase: the air window
 // (100 cells) was walked on every face before, 4.1 ms at 96^3 for the six
-// launches with 2.9M particles and 6 bubbles; 0.97 (liquid) + 0.64 ms (air) now.
+// launches with 2.9M particles and 6 bubbles; 0.97 (liquid) + 0.36 ms (air: row
+// bits, the 36 cells within the radius) now.
 struct FaceOut {
   double* W[3];
   double* U[3];
@@ -150,8 +152,8 @@ template <int A, bool AIRPH, bool ROWS>
 __device__ __forceinline__ void adj_p2g_face(const Grid& g, const f3* __restrict__ pos, const f3* __restrict__ vel,
                                              const float* __restrict__ mass, const int8_t* __restrict__ flag,
                                              const uint32_t* __restrict__ cstart, const uint32_t* __restrict__ cend,
-                                             const uint8_t* __restrict__ cmask, const uint8_t* __restrict__ dm,
-                                             double* __restrict__ Wout, double* __restrict__ Uout, int64_t f, int sub) {
+                                             const uint8_t* __restrict__ cmask, const RowBits& rb,
+                                             const uint8_t* __restrict__ dm, double* __restrict__ Wout, double* __restrict__ Uout, int64_t f, int sub) {
   int i, j, k;
   ijk_face<A>(g, f, i, j, k);
   constexpr uint8_t need = AIRPH ? M_AIR : M_FLUIDSOLID;
@@ -203,18 +205,29 @@ __device__ __forceinline__ void adj_p2g_face(const Grid& g, const f3* __restrict
   };
   constexpr int i0 = A == 0 ? lo : lot, j0 = A == 1 ? lo : lot;
   constexpr int NJ = (A == 1 ? hin : hit) - j0 + 1, NR = ((A == 0 ? hin : hit) - i0 + 1) * NJ;
+  constexpr int k0 = A == 2 ? lo : lot, NK = (A == 2 ? hin : hit) - k0 + 1;
   for (int r = sub; r < NR; r += AIRPH ? AIR_LANES : 1) {
-      const int di = i0 + r / NJ, dj = j0 + r % NJ;
-      if (i + di < 0 || i + di >= g.nx || j + dj < 0 || j + dj >= g.ny) continue;
+    const int ci = i + i0 + r / NJ, cj = j + j0 + r % NJ;
+    if (AIRPH) {  // the row's cells that hold air, from their bits
+      using AW = AirWindow<A>;
+      const bool near = ROWS && *rb.odd == 0;
+      if (near && !AW::row_near(r)) continue;
+      uint32_t bits = row_window(rb.a, rb, ci + 2, cj + 2, k) & (near ? AW::bits_near : AW::ROW);
+      if (!bits) continue;
+      const int64_t c0 = cid(g, ci, cj, k + k0);
+      if (ROWS) visit(cstart[c0 + __ffs(bits) - 1], cend[c0 + 31 - __clz(bits)]);
+      else
+        for (; bits; bits &= bits - 1u) visit(cstart[c0 + __ffs(bits) - 1], cend[c0 + __ffs(bits) - 1]);
+    } else {
+      if (ci < 0 || ci >= g.nx || cj < 0 || cj >= g.ny) continue;
       // the row's masks and ranges together, then its particles (ROWS: one range)
-      constexpr int k0 = A == 2 ? lo : lot, NK = (A == 2 ? hin : hit) - k0 + 1;
       uint32_t S[NK], E[NK];
       bool take_cell[NK];
 #pragma unroll
       for (int q = 0; q < NK; ++q) {
         const int ck = k + k0 + q;
         const bool in = ck >= 0 && ck < g.nz;
-        const int64_t c = cid(g, i + di, j + dj, in ? ck : min(max(ck, 0), g.nz - 1));
+        const int64_t c = cid(g, ci, cj, in ? ck : min(max(ck, 0), g.nz - 1));
         const uint8_t m = cmask[c];
         S[q] = cstart[c];
         E[q] = cend[c];
@@ -233,6 +246,7 @@ __device__ __forceinline__ void adj_p2g_face(const Grid& g, const f3* __restrict
       }
       if (ROWS && s < e) visit(s, e);
     }
+  }
   if (AIRPH) {
 #pragma unroll
     for (int o = 1; o < AIR_LANES; o <<= 1) {
@@ -249,15 +263,15 @@ template <bool AIRPH, bool ROWS>
 __global__ void __launch_bounds__(256) k_adj_p2g_faces(Grid g, const f3* __restrict__ pos, const f3* __restrict__ vel,
                                 const float* __restrict__ mass, const int8_t* __restrict__ flag,
                                 const uint32_t* __restrict__ cstart, const uint32_t* __restrict__ cend,
-                                const uint8_t* __restrict__ cmask, const uint8_t* __restrict__ dm, FaceOut out) {
+                                const uint8_t* __restrict__ cmask, RowBits rb, const uint8_t* __restrict__ dm, FaceOut out) {
   const int64_t u = xcd_block() * blockDim.x + threadIdx.x;
   const int64_t f = AIRPH ? u / AIR_LANES : u;
   const int sub = AIRPH ? (int)(u % AIR_LANES) : 0;
   const int A = blockIdx.y;
   if (f >= (A == 0 ? g.FX : A == 1 ? g.FY : g.FZ)) return;
-  if (A == 0) adj_p2g_face<0, AIRPH, ROWS>(g, pos, vel, mass, flag, cstart, cend, cmask, dm, out.W[0], out.U[0], f, sub);
-  else if (A == 1) adj_p2g_face<1, AIRPH, ROWS>(g, pos, vel, mass, flag, cstart, cend, cmask, dm, out.W[1], out.U[1], f, sub);
-  else adj_p2g_face<2, AIRPH, ROWS>(g, pos, vel, mass, flag, cstart, cend, cmask, dm, out.W[2], out.U[2], f, sub);
+  if (A == 0) adj_p2g_face<0, AIRPH, ROWS>(g, pos, vel, mass, flag, cstart, cend, cmask, rb, dm, out.W[0], out.U[0], f, sub);
+  else if (A == 1) adj_p2g_face<1, AIRPH, ROWS>(g, pos, vel, mass, flag, cstart, cend, cmask, rb, dm, out.W[1], out.U[1], f, sub);
+  else adj_p2g_face<2, AIRPH, ROWS>(g, pos, vel, mass, flag, cstart, cend, cmask, rb, dm, out.W[2], out.U[2], f, sub);
 }
 
 struct P2GFaceData {
@@ -813,6 +827,8 @@ int run_p2g_adjoint(Ctx& c, const double* const* gfaces, double* gvel, double* g
   for (int q = 0; q < 6; ++q) copy_in(c, c.adj_fin[q], gfaces ? gfaces[q] : nullptr, face_count(c, q), where);
   const int64_t fc[3] = {c.g.FX, c.g.FY, c.g.FZ};
   const int64_t fm = std::max(fc[0], std::max(fc[1], fc[2]));
+  const RowBits rb = run_row_bits(c);
+  if (c.own_sort) run_air_regular(c, rb);
   for (int ph = 0; ph < 2; ++ph) {
     // W in adj_fout[0..2], U in adj_fout[3..5]
     FaceOut fo;
@@ -826,7 +842,7 @@ int run_p2g_adjoint(Ctx& c, const double* const* gfaces, double* gvel, double* g
     launch(c, ph == 0 ? "adj_p2g_faces" : "adj_p2g_faces_air",
            dim3(nblocks(ph == 0 ? fm : fm * AIR_LANES, 256), 3), dim3(256), 0, kern, c.g,
            (const f3*)c.pos[cur], (const f3*)c.vel[cur], (const float*)c.mass[cur], (const int8_t*)c.flag[cur],
-           (const uint32_t*)c.cstart, (const uint32_t*)c.cend, (const uint8_t*)c.cmask,
+           (const uint32_t*)c.cstart, (const uint32_t*)c.cend, (const uint8_t*)c.cmask, rb,
            (const uint8_t*)(c.bmask + nbricks(c.g)), fo);
     P2GFaceData fd;
     for (int A = 0; A < 3; ++A) {

@@ -4,6 +4,7 @@
 // the solid distance/velocity fields used by the collision advection (a15).
 #include "mpf_internal.h"
 #include "interp.h"
+#include "row_bits.h"
 
 #include <algorithm>
 #include <cmath>
@@ -68,17 +69,10 @@ constexpr Rings make_rings() {
 }
 __constant__ Rings c_rings = make_rings();
 
-// The phases of the cells as bits, row by row along k, in words of 64: cell
-// (i, j, k) at bit k + 2 of row (i + 2, j + 2), with empty rows and bits around
-// the grid, so that every row of a window is five bits of one unaligned read.
-struct RowBits {
-  const uint64_t* f;  // liquid or solid
-  const uint64_t* a;  // air
-  int nw;             // words a row
-};
 __global__ void k_row_bits(Grid g, const uint8_t* __restrict__ cmask, uint64_t* __restrict__ fb,
-                           uint64_t* __restrict__ ab, int nw) {
+                           uint64_t* __restrict__ ab, int nw, uint32_t* __restrict__ odd) {
   const int64_t w = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;  // a wave per word
+  if (blockIdx.x == 0 && threadIdx.x == 0) *odd = 0;
   if (w >= (int64_t)(g.nx + 4) * (g.ny + 4) * nw) return;
   const int64_t row = w / nw;
   const int i = (int)(row / (g.ny + 4)) - 2, j = (int)(row % (g.ny + 4)) - 2;
@@ -90,21 +84,45 @@ __global__ void k_row_bits(Grid g, const uint8_t* __restrict__ cmask, uint64_t* 
     ab[w] = a;
   }
 }
+// *odd = 1 if an air particle's position, velocity or mass is not finite or its
+// position lies off the grid (it is then listed in a cell it is not in).
+__global__ void k_air_regular(Grid g, int64_t P, const f3* __restrict__ pos, const f3* __restrict__ vel,
+                              const float* __restrict__ mass, const int8_t* __restrict__ flag,
+                              uint32_t* __restrict__ odd) {
+  const int64_t p0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 16;
+  if (p0 >= P) return;
+  int8_t fl[16];
+  if (p0 + 16 <= P) __builtin_memcpy(fl, __builtin_assume_aligned(flag + p0, 16), 16);
+  else
+    for (int u = 0; u < 16; ++u) fl[u] = p0 + u < P ? flag[p0 + u] : (int8_t)-1;
+  bool air = false;
+#pragma unroll
+  for (int u = 0; u < 16; ++u) air = air || fl[u] == AIR;
+  if (!air) return;
+  const float lim = 3.4e38f;
+  bool bad = false;
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    if (fl[u] != AIR) continue;
+    const f3 x = pos[p0 + u], v = vel[p0 + u];
+    const float qx = (x.x - g.gx0) / g.h, qy = (x.y - g.gy0) / g.h, qz = (x.z - g.gz0) / g.h;
+    const bool in = qx >= 0 && qx < (float)g.nx && qy >= 0 && qy < (float)g.ny && qz >= 0 && qz < (float)g.nz;
+    const bool fin = fabsf(v.x) < lim && fabsf(v.y) < lim && fabsf(v.z) < lim && fabsf(mass[p0 + u]) < lim;
+    bad = bad || !in || !fin;
+  }
+  if (bad) *odd = 1;
+}
+
 // The 125 bits of the window around (i, j, k).
-__device__ __forceinline__ void window_bits(const uint64_t* __restrict__ rows, int nw, int ny4, int i, int j, int k,
+__device__ __forceinline__ void window_bits(const uint64_t* __restrict__ rows, const RowBits& rb, int i, int j, int k,
                                             uint64_t& lo, uint64_t& hi) {
-  const uint8_t* base = (const uint8_t*)(rows + ((int64_t)i * ny4 + j) * nw) + (k >> 3);
   uint32_t w[5];
 #pragma unroll
   for (int di = 0; di < 5; ++di) {
     w[di] = 0;
-    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_sched_barrier(0);  // five reads in flight, not 25 addresses in registers
 #pragma unroll
-    for (int dj = 0; dj < 5; ++dj) {
-      uint16_t v;  // bits k & 7 .. (k & 7) + 4 of two bytes
-      __builtin_memcpy(&v, base + ((int64_t)di * ny4 + dj) * nw * 8, 2);
-      w[di] |= (((uint32_t)v >> (k & 7)) & 31u) << (5 * dj);
-    }
+    for (int dj = 0; dj < 5; ++dj) w[di] |= row_window(rows, rb, i + di, j + dj, k) << (5 * dj);
   }
   lo = (uint64_t)w[0] | (uint64_t)w[1] << 25 | (uint64_t)w[2] << 50;
   hi = (uint64_t)(w[2] >> 14) | (uint64_t)w[3] << 11 | (uint64_t)w[4] << 36;
@@ -229,8 +247,8 @@ __global__ void __launch_bounds__(256, 8) k_genlevelset(Grid g, const f3* __rest
   uint64_t fw[2] = {0, 0}, aw[2] = {0, 0};
   {
     const float lb = 0.999f * c_rings.lb[2] * h2;
-    if (has_f && mf2 > lb) window_bits(rb.f, rb.nw, g.ny + 4, i, j, k, fw[0], fw[1]);
-    if (has_a && ma2 > lb) window_bits(rb.a, rb.nw, g.ny + 4, i, j, k, aw[0], aw[1]);
+    if (has_f && mf2 > lb) window_bits(rb.f, rb, i, j, k, fw[0], fw[1]);
+    if (has_a && ma2 > lb) window_bits(rb.a, rb, i, j, k, aw[0], aw[1]);
   }
   for (int ring = 2; ring < 9; ++ring) {
     const float lb = 0.999f * c_rings.lb[ring] * h2;
@@ -484,16 +502,19 @@ __global__ void k_mark_solid(Grid g, const uint32_t* __restrict__ cstart, const 
 // 2809-2937.  One thread per face, the three axes in one launch; window normal
 // [-2,1] x transverse [-2,2], in the reference's order.  Faces without air in
 // the bricks around them are done at once; the others are few (bubbles) and
-// walk up to 100 cells, so the kernel is bound by the latency of that chain:
-// a row's masks and ranges are read together, and with the library's own sort
-// a row's cells (consecutive along k) are one range of particles, read eight
-// at a time.  At 128^3 with 8 bubbles 1.38 ms as three launches that walked
-// cell by cell and particle by particle, 0.61 ms now.
+// walk many particles in a fixed order, so the kernel is bound by the latency
+// of that chain.  The rows that hold air come from the row bits; of the 100
+// cells only the 36 within the kernel's radius are visited when that changes
+// nothing (AirWindow); with the library's own sort a row's cells (consecutive
+// along k) are one range of particles, read eight at a time, and the next
+// row's range is fetched meanwhile.  At 128^3 with 8 bubbles 1.38 ms as three
+// launches that walked 100 cells, particle by particle; 0.56 with rows and
+// bits; 0.23 with the near cells alone.
 template <int A, bool ROWS>
 __device__ __forceinline__ void p2g_air_face(const Grid& g, const f3* __restrict__ pos, const f3* __restrict__ vel,
                                              const float* __restrict__ mass, const int8_t* __restrict__ flag,
                                              const uint32_t* __restrict__ cstart, const uint32_t* __restrict__ cend,
-                                             const uint8_t* __restrict__ cmask, const uint8_t* __restrict__ dm,
+                                             const RowBits& rb, const uint8_t* __restrict__ dm,
                                              float* __restrict__ out, float* __restrict__ out2, int64_t f) {
   int i, j, k;
   ijk_face<A>(g, f, i, j, k);
@@ -510,7 +531,6 @@ __device__ __forceinline__ void p2g_air_face(const Grid& g, const f3* __restrict
   }
   const float scale = 1.0f / g.h;
   const f3 gp = mk3((float)i + (A == 0 ? 0.0f : 0.5f), (float)j + (A == 1 ? 0.0f : 0.5f), (float)k + (A == 2 ? 0.0f : 0.5f));
-  constexpr int k0 = -2, NK = A == 2 ? 4 : 5;
   constexpr int NB = 8;
   float weight = 0, usum = 0;
   const float RE = 1.4f;
@@ -544,44 +564,60 @@ __device__ __forceinline__ void p2g_air_face(const Grid& g, const f3* __restrict
       }
     }
   };
-  // rows in the reference's order, the next row's masks and ranges in flight
-  constexpr int NJ = A == 1 ? 4 : 5, NR = (A == 0 ? 4 : 5) * NJ;
-  uint32_t S[NK], E[NK];
-  uint8_t m[NK];
-  auto row = [&](int r, uint32_t (&rs)[NK], uint32_t (&re)[NK], uint8_t (&rm)[NK]) {
-    const int ci = i + r / NJ - 2, cj = j + r % NJ - 2;
-    const bool rin = ci >= 0 && ci < g.nx && cj >= 0 && cj < g.ny;
+  // the window's rows that hold air, NK bits each, in the reference's order
+  using AW = AirWindow<A>;
+  constexpr int NJ = AW::NJ, NK = AW::NK, RW = AW::RW;
+  uint64_t w[2] = {0, 0};
 #pragma unroll
-    for (int q = 0; q < NK; ++q) {
-      const int ck = k + k0 + q;
-      const int64_t c = cid(g, min(max(ci, 0), g.nx - 1), min(max(cj, 0), g.ny - 1), min(max(ck, 0), g.nz - 1));
-      rm[q] = (rin && ck >= 0 && ck < g.nz) ? cmask[c] : (uint8_t)0;
-      rs[q] = cstart[c];
-      re[q] = cend[c];
+  for (int di = 0; di < AW::NI; ++di) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int dj = 0; dj < NJ; ++dj) {
+      const int r = di * NJ + dj;
+      w[r / RW] |= (uint64_t)(row_window(rb.a, rb, i + di, j + dj, k) & AW::ROW) << (NK * (r % RW));
     }
+  }
+  if (ROWS && *rb.odd == 0) {  // the library's own sort, every air particle finite and on the grid
+    w[0] &= AW::near_word(0);
+    w[1] &= AW::near_word(1);
+  }
+  // the next row's range (ROWS) or cells: offset of its cell k - 2, its bits
+  auto pop = [&](int64_t& c0, uint32_t& bits) {
+    const bool lo = w[0] != 0;
+    const uint64_t v = lo ? w[0] : w[1];
+    const int q = (__ffsll((unsigned long long)v) - 1) / NK, r = q + (lo ? 0 : RW);
+    bits = (uint32_t)(v >> (NK * q)) & AW::ROW;
+    const uint64_t keep = ~((uint64_t)AW::ROW << (NK * q));
+    if (lo) w[0] &= keep;
+    else w[1] &= keep;
+    c0 = cid(g, i + r / NJ - 2, j + r % NJ - 2, k - 2);
   };
-  row(0, S, E, m);
-  for (int r = 0; r < NR; ++r) {
-    uint32_t Sn[NK], En[NK];
-    uint8_t mn[NK];
-    row(r + 1 < NR ? r + 1 : r, Sn, En, mn);
-    uint32_t s = MPF_CELL_UNDEF, e = 0;
-#pragma unroll
-    for (int q = 0; q < NK; ++q) {
-      if (!(m[q] & M_AIR)) continue;
-      if (ROWS) {
-        s = min(s, S[q]);
-        e = max(e, E[q]);
-      } else {
-        visit(S[q], E[q]);
-      }
+  if (ROWS) {
+    uint32_t s = 0, e = 0;
+    auto next = [&]() {
+      s = e = 0;
+      if (!(w[0] | w[1])) return;
+      int64_t c0;
+      uint32_t bits;
+      pop(c0, bits);
+      s = cstart[c0 + __ffs(bits) - 1];
+      e = cend[c0 + 31 - __clz(bits)];
+    };
+    next();
+    while (s < e) {
+      const uint32_t cs = s, ce = e;
+      next();  // in flight during this row's particles
+      visit(cs, ce);
     }
-    if (ROWS && s < e) visit(s, e);
-#pragma unroll
-    for (int q = 0; q < NK; ++q) {
-      S[q] = Sn[q];
-      E[q] = En[q];
-      m[q] = mn[q];
+  } else {
+    while (w[0] | w[1]) {
+      int64_t c0;
+      uint32_t bits;
+      pop(c0, bits);
+      for (; bits; bits &= bits - 1u) {
+        const int64_t c = c0 + __ffs(bits) - 1;
+        visit(cstart[c], cend[c]);
+      }
     }
   }
   const float u = (weight > 0) ? (usum / weight) : 0.0f;
@@ -596,13 +632,13 @@ template <bool ROWS>
 __global__ void __launch_bounds__(256)
     k_p2g_air(Grid g, const f3* __restrict__ pos, const f3* __restrict__ vel, const float* __restrict__ mass,
               const int8_t* __restrict__ flag, const uint32_t* __restrict__ cstart, const uint32_t* __restrict__ cend,
-              const uint8_t* __restrict__ cmask, const uint8_t* __restrict__ dm, P2GOut o) {
+              RowBits rb, const uint8_t* __restrict__ dm, P2GOut o) {
   const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int A = blockIdx.y;
   if (f >= (A == 0 ? g.FX : A == 1 ? g.FY : g.FZ)) return;
-  if (A == 0) p2g_air_face<0, ROWS>(g, pos, vel, mass, flag, cstart, cend, cmask, dm, o.u[0], o.u2[0], f);
-  else if (A == 1) p2g_air_face<1, ROWS>(g, pos, vel, mass, flag, cstart, cend, cmask, dm, o.u[1], o.u2[1], f);
-  else p2g_air_face<2, ROWS>(g, pos, vel, mass, flag, cstart, cend, cmask, dm, o.u[2], o.u2[2], f);
+  if (A == 0) p2g_air_face<0, ROWS>(g, pos, vel, mass, flag, cstart, cend, rb, dm, o.u[0], o.u2[0], f);
+  else if (A == 1) p2g_air_face<1, ROWS>(g, pos, vel, mass, flag, cstart, cend, rb, dm, o.u[1], o.u2[1], f);
+  else p2g_air_face<2, ROWS>(g, pos, vel, mass, flag, cstart, cend, rb, dm, o.u[2], o.u2[2], f);
 }
 
 // Liquid+solid P2G, tile scatter (the hot path).  A block owns a 4x8x8 cell
@@ -1716,19 +1752,29 @@ void run_bricks(Ctx& c) {
          by, bz);
 }
 
-void run_levelset(Ctx& c) {
-  const int64_t G = c.g.G;
-  const int cur = c.cur;
-  const int64_t NB = nbricks(c.g);
-  // row bits in the scratch of the liquid P2G (a quarter byte a cell and the
-  // border; it holds 49 bytes a cell of 4x8x8 tiles)
+// Row bits of the current masks, in the scratch of the liquid P2G (a quarter
+// byte a cell and the border; it holds 49 bytes a cell of 4x8x8 tiles): valid
+// until the next P2G or solve.
+RowBits run_row_bits(Ctx& c) {
   const int nw = (c.g.nz + 4 + 63) / 64;
   const int64_t words = (int64_t)(c.g.nx + 4) * (c.g.ny + 4) * nw;
   uint64_t* fb = (uint64_t*)c.p2g_parts;
   uint64_t* ab = fb + words;
   launch(c, "row_bits", dim3(nblocks(words * 64, 256)), dim3(256), 0, k_row_bits, c.g, (const uint8_t*)c.cmask, fb, ab,
-         nw);
-  const RowBits rb{fb, ab, nw};
+         nw, (uint32_t*)(ab + words));
+  return RowBits{fb, ab, nw, c.g.ny + 4, (uint32_t*)(ab + words)};
+}
+void run_air_regular(Ctx& c, const RowBits& rb) {
+  const int cur = c.cur;
+  launch(c, "air_regular", dim3(nblocks((c.P + 15) / 16, 256)), dim3(256), 0, k_air_regular, c.g, c.P,
+         (const f3*)c.pos[cur], (const f3*)c.vel[cur], (const float*)c.mass[cur], (const int8_t*)c.flag[cur], rb.odd);
+}
+
+void run_levelset(Ctx& c) {
+  const int64_t G = c.g.G;
+  const int cur = c.cur;
+  const int64_t NB = nbricks(c.g);
+  const RowBits rb = run_row_bits(c);
   launch(c, "genlevelset", dim3(nblocks(G, 256)), dim3(256), 0, k_genlevelset, c.g, (const f3*)c.pos[cur],
          (const int8_t*)c.flag[cur], (const uint32_t*)c.cstart, (const uint32_t*)c.cend, (const uint8_t*)c.cmask,
          (const uint8_t*)(c.bmask + NB), rb, c.lsfluid, c.lsair, c.mark);
@@ -1753,12 +1799,13 @@ static void p2g_air(Ctx& c, float* const* out, float* const* out2) {
     o.u[a] = out[a];
     o.u2[a] = out2 ? out2[a] : nullptr;
   }
+  const RowBits rb = run_row_bits(c);
+  if (c.own_sort) run_air_regular(c, rb);
   // lists given by the caller need not be consecutive along a row
   auto kern = c.own_sort ? k_p2g_air<true> : k_p2g_air<false>;
   launch(c, "p2g_air", dim3(nblocks(std::max(c.g.FX, std::max(c.g.FY, c.g.FZ)), 256), 3), dim3(256), 0, kern, c.g,
          (const f3*)c.pos[cur], (const f3*)c.vel[cur], (const float*)c.mass[cur], (const int8_t*)c.flag[cur],
-         (const uint32_t*)c.cstart, (const uint32_t*)c.cend, (const uint8_t*)c.cmask,
-         (const uint8_t*)(c.bmask + nbricks(c.g)), o);
+         (const uint32_t*)c.cstart, (const uint32_t*)c.cend, rb, (const uint8_t*)(c.bmask + nbricks(c.g)), o);
 }
 
 static void p2g_liquid(Ctx& c, float* const* out, float* const* out2 = nullptr, const float* band = nullptr,

@@ -312,6 +312,9 @@ int run_solid_motion(Ctx& c);
 int run_write_mesh(Ctx& c, const char* path, int format, const char* object_name);
 void run_solid_phi_and_velocity(Ctx& c);
 int64_t p2g_parts_floats(const Grid& g);
+struct RowBits;
+RowBits run_row_bits(Ctx& c);
+void run_air_regular(Ctx& c, const RowBits& rb);
 // Device counters: 64 single counters, then SPREAD counters 64 bytes apart
 // (a total that many blocks add to, split over cache lines)
 constexpr int NSPREAD = 64;

@@ -64,3 +64,50 @@ def test_row_ranges(pkg, dims):
         err = np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300)
         say("  adjoint output %d: %.2e" % (q, err))
         assert np.any(b) and err <= 1e-12
+
+
+@pytest.mark.parametrize("odd", ["none", "nan velocity", "infinite mass", "off the grid"])
+@pytest.mark.parametrize("dims", [(4, 4, 5), (12, 9, 30), (9, 21, 11)])
+def test_air_window(pkg, dims, odd):
+    """Air P2G leaves out the window's cells beyond the kernel's radius when
+    every air particle is finite and on the grid (library's own sort), and
+    visits them otherwise and for given lists: the same bits either way (a NaN
+    or an infinity two cells off reaches the face as 0 times it), and the same
+    adjoint for finite particles."""
+    say("air window", dims, odd)
+    nx, ny, nz = dims
+    rng = np.random.default_rng(nx * 1000 + ny * 10 + nz)
+    n = nx * ny * nz * 4
+    cfg = pkg.default_config(nx, ny, nz, particle_capacity=n, adjoint_enabled=1, heat_enabled=0, gas_enabled=0,
+                             mc_enabled=0)
+    h = float(cfg.dx)
+    pos = (rng.uniform(0.0, 1.0, (n, 3)) * np.array(dims) * h * 0.999999).astype(np.float32)
+    flag = np.where(rng.uniform(size=n) < 0.4, pkg.TYPEAIR, pkg.TYPEFLUID).astype(np.int8)
+    vel = rng.standard_normal((n, 3)).astype(np.float32)
+    mass = rng.uniform(0.5, 2.0, n).astype(np.float32)
+    a = np.flatnonzero(flag == pkg.TYPEAIR)[n // 5]
+    if odd == "nan velocity":
+        vel[a] = np.nan
+    elif odd == "infinite mass":
+        mass[a] = np.inf
+    elif odd == "off the grid":
+        pos[a, 0] = (nx + 0.3) * h
+    own = pkg.Simulator(cfg)
+    own.set_particles(n, pos=pos, vel=vel, flag=flag, mass=mass)
+    own.hash_sort()
+    given = pkg.Simulator(cfg)
+    given.set_particles(n, **own.get_particles())
+    for nm in ("CELL_START", "CELL_END"):
+        given.set_field(nm, own.get_field(nm))
+    gf = [rng.standard_normal(m) for m in own.face_sizes()]
+    adj = []
+    for sim in (own, given):
+        sim.p2g()
+        adj.append(sim.p2g_adjoint(gf))
+    for f in FACE[3:]:
+        u, v = own.get_field(f), given.get_field(f)
+        assert np.array_equal(u, v, equal_nan=True), f
+        assert np.isnan(u).any() == (odd in ("nan velocity", "infinite mass"))
+    if odd in ("none", "off the grid"):
+        for u, v in zip(*adj):
+            assert np.max(np.abs(u - v)) <= 1e-12 * np.max(np.abs(v))
