@@ -274,6 +274,14 @@ __device__ __forceinline__ double wave_sum(double v) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
+// Workgroup barrier that orders LDS only: global loads issued before it stay
+// in flight (a full __syncthreads would wait for them).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Block-wide sum of N values over NT threads; the result is returned in every
 // thread.  Thread q adds the wave sums of value q in wave order (one thread
 // per value keeps the other threads' registers free of the NT/64 x N terms).
@@ -287,17 +295,17 @@ __device__ __forceinline__ void block_sum_all(double (&v)[N]) {
   if (lane == 0)
 #pragma unroll
     for (int q = 0; q < N; ++q) lds[w][q] = v[q];
-  __syncthreads();
+  lds_barrier();
   if (threadIdx.x < N) {
     double s = 0.0;
 #pragma unroll
     for (int ww = 0; ww < NT / 64; ++ww) s += lds[ww][threadIdx.x];
     tot[threadIdx.x] = s;
   }
-  __syncthreads();
+  lds_barrier();
 #pragma unroll
   for (int q = 0; q < N; ++q) v[q] = tot[q];
-  __syncthreads();
+  lds_barrier();
 }
 
 // This block's partial sums -> P[blockIdx.x * N + q].
@@ -309,14 +317,20 @@ __device__ __forceinline__ void write_partials(double (&v)[N], double* __restric
     for (int q = 0; q < N; ++q) P[(int64_t)blockIdx.x * N + q] = v[q];
 }
 
-// Sum of the previous kernel's partials (nb blocks), identical in every block.
-template <int N, int NT = PB>
-__device__ __forceinline__ void read_partials(const double* __restrict__ P, int nb, double (&out)[N]) {
+// Sum of the previous kernel's partials (nb blocks), identical in every block:
+// each thread's share, then the block's sum of them.
+template <int N, int NT, int M>
+__device__ __forceinline__ void thread_partials(const double* __restrict__ P, int nb, double (&out)[M]) {
+  static_assert(N <= M, "sums fit");
 #pragma unroll
   for (int q = 0; q < N; ++q) out[q] = 0.0;
   for (int b = threadIdx.x; b < nb; b += NT)
 #pragma unroll
     for (int q = 0; q < N; ++q) out[q] += P[(int64_t)b * N + q];
+}
+template <int N, int NT = PB>
+__device__ __forceinline__ void read_partials(const double* __restrict__ P, int nb, double (&out)[N]) {
+  thread_partials<N, NT>(P, nb, out);
   block_sum_all<N, NT>(out);
 }
 
@@ -431,14 +445,6 @@ struct Raw {
   V r, pp, ds;
   uint8_t nb;
 };
-// Workgroup barrier that orders LDS only: global loads issued before it stay
-// in flight (a full __syncthreads would wait for them).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // a + x y in FP64 for FP32 x, y: their product is exact in FP64, so the fused
 // form rounds exactly as a separate multiply and add (one instruction, not two).
 template <class X, class Y>
@@ -455,6 +461,35 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t byte_rsrc(const uint8_t* p) {
 }
 __device__ __forceinline__ uint8_t ld_byte(__amdgpu_buffer_rsrc_t r, uint32_t col, uint32_t plane_off) {
   return __builtin_amdgcn_raw_buffer_load_b8(r, col, plane_off, 0);
+}
+
+// Buffer accesses of one value a lane: lane offset in bytes (OFF_NONE: nothing
+// is read, the value is 0; nothing is written), plane offset in bytes in a
+// scalar register.  The descriptor's size ends at the array's end, so
+// OFF_NONE is out of its range whether or not the plane offset counts.  A
+// lane without a cell then needs no branch around its accesses: with branches
+// the compiler cannot count the stores between a load and its use and waits
+// for younger loads as well.
+constexpr uint32_t OFF_NONE = 0xfffffffcu;
+template <class T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const T* p, int64_t n) {
+  const uint64_t bytes = (uint64_t)n * sizeof(T);
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), 0, (int)(uint32_t)(bytes < 0xfffffff0u ? bytes : 0xfffffff0u),
+                                           0x00020000);
+}
+__device__ __forceinline__ float buf_ld(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t plane_off, float) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, plane_off, 0));
+}
+__device__ __forceinline__ double buf_ld(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t plane_off, double) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, plane_off, 0));
+}
+// (nontemporal, as st_nt)
+__device__ __forceinline__ void buf_st_nt(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t plane_off, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, off, plane_off, 2);
+}
+__device__ __forceinline__ void buf_st_nt(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t plane_off, double v) {
+  using U2 = uint32_t __attribute__((ext_vector_type(2)));
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), r, off, plane_off, 2);
 }
 
 // Vector stores that nothing reads again within the launch (the next launch
@@ -1168,28 +1203,43 @@ struct CgScalars {
   double ald, be;
   bool stop, nonfin, zero_pq;
 };
+// A thread's share of those sums: the loads can be issued well before the
+// block adds them up.
+struct CgSums {
+  double d[FDOT], e[4];
+};
 template <int NT>
-__device__ __forceinline__ CgScalars cg_scalars(const Tiling& T, int nres, int first, int nbu, const double* __restrict__ Pprev,
-                                                const double* __restrict__ Pres, SolveScalars* sc, int k, double tol,
-                                                int cap) {
+__device__ __forceinline__ void cg_sums(const Tiling& T, int nres, int first, int nbu, const double* __restrict__ Pprev,
+                                        const double* __restrict__ Pres, CgSums& s) {
+  if (first == 1) {
+    thread_partials<2, NT>(Pres, nbu, s.d);
+  } else if (first == 2) {
+    thread_partials<4, NT>(Pres, nres, s.e);
+  } else {
+    thread_partials<FDOT, NT>(Pprev, T.nblk + T.ns5, s.d);
+    if (Pres) thread_partials<4, NT>(Pres, nres, s.e);
+  }
+}
+template <int NT>
+__device__ __forceinline__ CgScalars cg_scalars(CgSums& s, int first, const double* __restrict__ Pres,
+                                                SolveScalars* sc, int k, double tol, int cap) {
   double ald = 0.0, rz, rr, be = 0.0, rz_prev = 0.0;
   bool zero_pq = false, bad_pq = false;
   if (first == 1) {
-    double v[2];
-    read_partials<2, NT>(Pres, nbu, v);
+    double v[2] = {s.d[0], s.d[1]};
+    block_sum_all<2, NT>(v);
     rz = v[0];
     rr = v[1];
   } else if (first == 2) {
-    double v[4];
-    read_partials<4, NT>(Pres, nres, v);
-    rz = v[0];
-    rr = v[1];
+    block_sum_all<4, NT>(s.e);
+    rz = s.e[0];
+    rr = s.e[1];
   } else {
-    double d[FDOT];
-    read_partials<FDOT, NT>(Pprev, T.nblk + T.ns5, d);
+    double(&d)[FDOT] = s.d;
+    block_sum_all<FDOT, NT>(d);
     if (Pres) {
-      double e[4];
-      read_partials<4, NT>(Pres, nres, e);
+      double(&e)[4] = s.e;
+      block_sum_all<4, NT>(e);
       d[0] = e[0];
       d[1] = e[1];
       d[3] = e[2];
@@ -1263,6 +1313,14 @@ __device__ __forceinline__ CgScalars cg_scalars(const Tiling& T, int nres, int f
 // launch after a true-residual pass (first = 0, fold = 1 as constants), whose
 // x64 += x + alpha p reads x64 in the plane pipeline with the vectors.  A
 // launch that stops the solve advances x by all it owes.
+// The plane loop is one straight line: every access is a buffer access that
+// lanes without a cell skip by their offset, and the loop has one exit.  With
+// branches around stores and steps, waits were counted for paths that cannot
+// be taken and drained the loads of the plane before in two steps of three.
+// 256^3, 12.6M unknowns: modes 2 and 3 82.6 and 106 -> 78.5 and 100.6 us (the
+// least bytes, 24 and 36 an unknown, take 55 and 83 us at a large copy's
+// 5.5 TB/s), 154 vector instructions a plane and wave against 177; with slow
+// rows 94 us on average against 105.  192^3: 46 and 58 -> 41 and 53 us.
 template <int OPk, bool SLOW, bool STEADY, int XM, int TK>
 __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, int nbu, const double* __restrict__ Pprev,
                                                const double* __restrict__ Pres, double* __restrict__ Pout,
@@ -1276,9 +1334,6 @@ __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, in
   static_assert(XM == 1 || (STEADY && (XM == 2 || XM == 3)) || (XM == 4 && !STEADY),
                 "x modes 2 and 3 are steady launches, mode 4 the fold launch");
   using V = float;
-  // a launch after the one that stopped the solve does nothing (the
-  // stopping launch's own late blocks still finish its x update)
-  if (sc->done && sc->done_k != k) return;
   if (STEADY) {
     first = 0;
     fold = 0;
@@ -1303,14 +1358,11 @@ __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, in
   const int kk = k0 + kl;
   const int64_t sx = (int64_t)g.ny * g.nz;
   uint32_t col[RPT];
-  bool cok[RPT];
 #pragma unroll
   for (int u = 0; u < RPT; ++u) {
     const int j = j0 + jl0 + u;
-    cok[u] = j < g.ny && kk < g.nz;
-    col[u] = cok[u] ? (uint32_t)(j * g.nz + kk) : 0u;
+    col[u] = (j < g.ny && kk < g.nz) ? (uint32_t)(j * g.nz + kk) : OFF_NONE;
   }
-  auto plane = [&](int i) -> int64_t { return (int64_t)min(max(i, 0), g.nx - 1) * sx; };
   int hj = 0, hk = 0;
   const bool ring = tid < NRING;
   if (tid < 2 * TK) {
@@ -1322,11 +1374,21 @@ __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, in
     hk = (t2 < TJ) ? -1 : TK;
   }
   const bool hok = ring && (j0 + hj) >= 0 && (j0 + hj) < g.ny && (k0 + hk) >= 0 && (k0 + hk) < g.nz;
-  const uint32_t hcol = hok ? (uint32_t)((j0 + hj) * g.nz + (k0 + hk)) : 0u;
-  const auto nbm_r = byte_rsrc(o.nbm);
-  auto load_m = [&](int i, bool ok, uint32_t c) -> uint8_t {
-    return ld_byte(nbm_r, (ok && i >= 0 && i < g.nx) ? c : 0u, (uint32_t)plane(i));
-  };
+  const uint32_t hcol = hok ? (uint32_t)((j0 + hj) * g.nz + (k0 + hk)) : OFF_NONE;
+  // buffers from the run's first plane on (plane offsets stay below 2^32,
+  // make_tiling)
+  const int ip0 = max(i_lo - 1, 0);
+  const int64_t b0 = (int64_t)ip0 * sx, nleft = g.G - b0;
+  const auto m_b = buf_rsrc(o.nbm + b0, nleft);
+  const auto r_b = buf_rsrc(rin + b0, nleft), q_b = buf_rsrc(qin + b0, nleft), p_b = buf_rsrc(pin + b0, nleft);
+  const auto x_b = buf_rsrc(x + b0, nleft), p2_b = buf_rsrc(XM == 3 ? p2in + b0 : pin + b0, nleft);
+  const auto ro_b = buf_rsrc(rout + b0, nleft), qo_b = buf_rsrc(qout + b0, nleft), po_b = buf_rsrc(pout + b0, nleft);
+  const auto x64_b = buf_rsrc(x64 + b0, nleft);
+  const auto ds_b = buf_rsrc((const V*)o.dslow + b0, nleft);
+  auto plane = [&](int i) -> uint32_t { return (uint32_t)(min(max(i, ip0), g.nx - 1) - ip0) * (uint32_t)sx; };
+  // the mask as loaded; load_v applies the plane's grid test, so that no
+  // instruction touches the byte before it is needed
+  auto load_m = [&](int i, uint32_t c) -> uint8_t { return __builtin_amdgcn_raw_buffer_load_b8(m_b, c, plane(i), 0); };
   // masks of planes i_lo - 1 .. i_lo + 3 (the plane loop's slots M, HM and
   // the prologue's MA, HA, HB); they do not depend on alpha or beta
   uint8_t M[3][RPT], HM[3];
@@ -1334,19 +1396,83 @@ __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, in
   auto load_masks = [&]() {
 #pragma unroll
     for (int u = 0; u < RPT; ++u) {
-      MA[0][u] = load_m(i_lo - 1, cok[u], col[u]);
-      MA[1][u] = load_m(i_lo, cok[u], col[u]);
-      M[1][u] = load_m(i_lo + 1, cok[u], col[u]);
-      M[2][u] = load_m(i_lo + 2, cok[u], col[u]);
-      M[0][u] = load_m(i_lo + 3, cok[u], col[u]);
+      MA[0][u] = load_m(i_lo - 1, col[u]);
+      MA[1][u] = load_m(i_lo, col[u]);
+      M[1][u] = load_m(i_lo + 1, col[u]);
+      M[2][u] = load_m(i_lo + 2, col[u]);
+      M[0][u] = load_m(i_lo + 3, col[u]);
     }
-    HA = load_m(i_lo, hok, hcol);
-    HB[0] = load_m(i_lo + 1, hok, hcol);
-    HB[1] = load_m(i_lo + 2, hok, hcol);
-    HM[0] = load_m(i_lo + 3, hok, hcol);
+    HA = load_m(i_lo, hcol);
+    HB[0] = load_m(i_lo + 1, hcol);
+    HB[1] = load_m(i_lo + 2, hcol);
+    HM[0] = load_m(i_lo + 3, hcol);
   };
+  // Prologue: the masks of planes i_lo - 1 .. i_lo + 3, this thread's share of
+  // the partial sums, then every vector load, none of which waits for the
+  // sums; then the block's sums and the arithmetic (the fold launch, whose
+  // registers are full, reads its masks and vectors after the sums).
   if constexpr (XM != 4) load_masks();
-  const CgScalars cs = cg_scalars<ST>(T, T.nblk + T.ns5, first, nbu, Pprev, Pres, sc, k, tol, cap);
+  CgSums sums;
+  cg_sums<ST>(T, T.nblk + T.ns5, first, nbu, Pprev, Pres, sums);
+  // a launch after the one that stopped the solve does nothing (the
+  // stopping launch's own late blocks still finish its x update)
+  if (sc->done && sc->done_k != k) return;
+  // a cell's loads: its vectors where it is an unknown, 0 elsewhere
+  // (the slow-row diagonal exists only in the SLOW form: a field that is
+  // constant there still shifts the register allocation of the fast form)
+  struct RwS {
+    V r, q, p, x, p2, ds;
+    uint8_t nb;
+  };
+  struct RwF {
+    V r, q, p, x, p2;
+    uint8_t nb;
+  };
+  using Rw = typename std::conditional<SLOW, RwS, RwF>::type;
+  auto off_of = [&](uint8_t nb, uint32_t c) -> uint32_t { return (nb & NB_UNKNOWN) ? c * 4u : OFF_NONE; };
+  auto load_v = [&](int i, uint8_t raw, uint32_t c, Rw& w, bool with_x) {
+    const uint8_t nb = (i >= 0 && i < g.nx) ? raw : (uint8_t)0;
+    const uint32_t pb = plane(i) * 4u, cv = off_of(nb, c);
+    w.nb = nb;
+    w.r = buf_ld(r_b, cv, pb, V());
+    w.q = buf_ld(q_b, cv, pb, V());
+    w.p = buf_ld(p_b, cv, pb, V());
+    w.x = (with_x && XM != 2) ? buf_ld(x_b, cv, pb, V()) : V(0);
+    w.p2 = (with_x && XM == 3) ? buf_ld(p2_b, cv, pb, V()) : V(0);
+    if constexpr (SLOW) w.ds = buf_ld(ds_b, (nb & NB_SLOW) ? cv : OFF_NONE, pb, V());
+  };
+  // x64 of a cell in mode 4
+  auto load_x64 = [&](int i, uint8_t raw, uint32_t c) -> double {
+    const bool un = i < g.nx && (raw & NB_UNKNOWN);
+    return buf_ld(x64_b, un ? c * 8u : OFF_NONE, plane(i) * 8u, double());
+  };
+  Rw R[3][RPT], HR[3];
+  Rw W0[RPT], W1[RPT], WH;
+  double X0[RPT] = {};
+  // x64 of planes i+1 and i+2 in mode 4 (slot by plane parity within the
+  // unrolled loop), loaded a plane ahead of their use
+  double XD[2][RPT] = {};
+  auto load_prologue = [&]() {
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) {
+      load_v(i_lo - 1, MA[0][u], col[u], W0[u], false);
+      load_v(i_lo, MA[1][u], col[u], W1[u], true);
+    }
+    load_v(i_lo, HA, hcol, WH, false);
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) {
+      load_v(i_lo + 1, M[1][u], col[u], R[1][u], true);
+      load_v(i_lo + 2, M[2][u], col[u], R[2][u], true);
+      if constexpr (XM == 4) {
+        X0[u] = load_x64(i_lo, MA[1][u], col[u]);
+        XD[1][u] = load_x64(i_lo + 1, M[1][u], col[u]);
+      }
+    }
+    load_v(i_lo + 1, HB[0], hcol, HR[1], false);
+    load_v(i_lo + 2, HB[1], hcol, HR[2], false);
+  };
+  if constexpr (XM != 4) load_prologue();
+  const CgScalars cs = cg_scalars<ST>(sums, first, Pres, sc, k, tol, cap);
   const bool stop = cs.stop, nonfin = cs.nonfin, zero_pq = cs.zero_pq;
   const V al = (V)cs.ald, bev = (V)cs.be;
   const V al2 = (XM == 3) ? sc->alh[(k - 1) & 1] : V(0);  // alpha_k-2, as launch k-1 applied it
@@ -1367,104 +1493,62 @@ __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, in
     for (int i = i_lo; i < i_hi; ++i)
 #pragma unroll
       for (int u = 0; u < RPT; ++u) {
-        if (!cok[u]) continue;
+        if (col[u] == OFF_NONE) continue;
         const int64_t idx = (int64_t)i * sx + col[u];
         if (o.nbm[idx] & NB_UNKNOWN) advance_x(idx, pin[idx]);
       }
     return;
   }
-  // loads as in the spmv: uniform plane base, 32-bit column, every lane
-  // issues every load (element 0 of the plane when there is nothing to read)
-  // (the slow-row diagonal exists only in the SLOW form: a field that is
-  // constant there still shifts the register allocation of the fast form)
-  struct RwS {
-    V r, q, p, x, p2, ds;
-    uint8_t nb;
-  };
-  struct RwF {
-    V r, q, p, x, p2;
-    uint8_t nb;
-  };
-  using Rw = typename std::conditional<SLOW, RwS, RwF>::type;
-  auto load_v = [&](int i, bool ok, uint8_t raw, uint32_t c, Rw& w, bool with_x) {
-    const uint8_t nb = (ok && i >= 0 && i < g.nx) ? raw : (uint8_t)0;
-    const int64_t pb = plane(i);
-    const bool un = (nb & NB_UNKNOWN) != 0;
-    const uint32_t cv = un ? c : 0u;
-    w.nb = nb;
-    w.r = (rin + pb)[cv];
-    w.q = (qin + pb)[cv];
-    w.p = (pin + pb)[cv];
-    w.x = (with_x && XM != 2) ? (x + pb)[cv] : V(0);
-    if constexpr (SLOW) w.ds = ((const V*)o.dslow + pb)[(un && (nb & NB_SLOW) && o.precond) ? c : 0u];
-    w.p2 = (with_x && XM == 3) ? (p2in + pb)[cv] : V(0);
-  };
-  // r_k, and p_k = z_k + beta p_{k-1} (0 off the unknowns)
+  // r_k, and p_k = z_k + beta p_{k-1} (0 off the unknowns, whose r, q and p
+  // were read as 0)
   auto r_of = [&](const Rw& w) -> V { return first ? w.r : w.r - al * w.q; };
   auto d_of = [&](uint8_t nb) -> V { return dtab[__popc((unsigned)(nb & 63))]; };
   auto dw_of = [&](const Rw& w) -> V {
-    if constexpr (SLOW) {
-      if (w.nb & NB_SLOW) return o.precond ? w.ds : V(1);
-    }
-    return d_of(w.nb);
+    const V d = d_of(w.nb);
+    if constexpr (SLOW) return (w.nb & NB_SLOW) ? (o.precond ? w.ds : V(1)) : d;
+    return d;
   };
   auto p_of = [&](const Rw& w, V rk) -> V {
-    if (!(w.nb & NB_UNKNOWN)) return V(0);
-    return first ? rk * dw_of(w) : rk * dw_of(w) + bev * w.p;
+    const V z = rk * dw_of(w);
+    return first ? z : z + bev * w.p;
   };
   constexpr int UNR = 6;
   static_assert(UNR % 6 == 0, "slots by d % 3 and d & 1 repeat across the unrolled loop");
-  Rw R[3][RPT], HR[3];
   V PV[3][RPT], RV[3][RPT];  // p_k, r_k of planes i-1 .. i+1
   uint8_t NB[3][RPT];
   double a[FDOT] = {0, 0, 0, 0, 0, 0, 0};
-  // x64 of planes i+1 and i+2 in mode 4 (slot by plane parity within the
-  // unrolled loop), loaded a plane ahead of their use
-  double XD[2][RPT] = {};
-  // a cell of this block's planes once its r_k is formed: r_k and x stored,
-  // r.z and r.r summed (xd: its x64 in mode 4)
-  auto own = [&](int i, int u, const Rw& w, V rk, double xd) {
-    if (!(w.nb & NB_UNKNOWN)) return;
-    const int64_t pb = (int64_t)i * sx;
-    st_nt(rout + pb + col[u], rk);
-    if (fold) {
-      const int64_t idx = pb + col[u];
-      if constexpr (XM == 4) st_nt(x64 + idx, xd + (double)(w.x + al * w.p));
-      else x64[idx] = x64[idx] + (double)(w.x + al * w.p);
-      st_nt(x + idx, V(0));
-    } else if (!first) {
-      if constexpr (XM == 1) st_nt(x + pb + col[u], w.x + al * w.p);
-      if constexpr (XM == 3) st_nt(x + pb + col[u], (w.x + al2 * w.p2) + al * w.p);
-    }
-    const V zv = rk * dw_of(w);
-    a[0] = acc64(a[0], rk, zv);
-    a[1] = acc64(a[1], rk, rk);
-  };
-  // prologue: the masks of planes i_lo - 1 .. i_lo + 3 first (before the
-  // partial sums are read, except in the fold launch, whose registers are
-  // full), then every vector load, then the arithmetic
-  if constexpr (XM == 4) load_masks();
-  Rw W0[RPT], W1[RPT], WH;
-#pragma unroll
-  for (int u = 0; u < RPT; ++u) {
-    load_v(i_lo - 1, cok[u], MA[0][u], col[u], W0[u], false);
-    load_v(i_lo, cok[u], MA[1][u], col[u], W1[u], true);
-  }
-  load_v(i_lo, hok, HA, hcol, WH, false);
-  double X0[RPT] = {};
-#pragma unroll
-  for (int u = 0; u < RPT; ++u) {
-    load_v(i_lo + 1, cok[u], M[1][u], col[u], R[1][u], true);
-    load_v(i_lo + 2, cok[u], M[2][u], col[u], R[2][u], true);
+  // a cell of a plane of this run (mine) once its r_k is formed: r_k and x
+  // stored, r.z and r.r summed (xd: its x64 in mode 4)
+  auto own = [&](int i, int u, const Rw& w, V rk, double xd, bool mine) {
+    const uint32_t pb = plane(i) * 4u, cv = mine ? off_of(w.nb, col[u]) : OFF_NONE;
+    buf_st_nt(ro_b, cv, pb, rk);
     if constexpr (XM == 4) {
-      const uint8_t nb0 = (cok[u] && i_lo < g.nx) ? MA[1][u] : (uint8_t)0;
-      X0[u] = (x64 + plane(i_lo))[(nb0 & NB_UNKNOWN) ? col[u] : 0u];
-      const uint8_t nb1 = (cok[u] && i_lo + 1 < g.nx) ? M[1][u] : (uint8_t)0;
-      XD[1][u] = (x64 + plane(i_lo + 1))[(nb1 & NB_UNKNOWN) ? col[u] : 0u];
+      buf_st_nt(x64_b, cv == OFF_NONE ? OFF_NONE : cv * 2u, pb * 2u, xd + (double)(w.x + al * w.p));
+      buf_st_nt(x_b, cv, pb, V(0));
+    } else if constexpr (XM == 3) {
+      buf_st_nt(x_b, cv, pb, (w.x + al2 * w.p2) + al * w.p);
+    } else if constexpr (XM == 1 && STEADY) {
+      buf_st_nt(x_b, cv, pb, w.x + al * w.p);
+    } else if constexpr (XM == 1) {
+      if (fold) {
+        if (cv != OFF_NONE) {
+          const int64_t idx = (int64_t)i * sx + col[u];
+          x64[idx] = x64[idx] + (double)(w.x + al * w.p);
+        }
+        buf_st_nt(x_b, cv, pb, V(0));
+      } else if (!first) {
+        buf_st_nt(x_b, cv, pb, w.x + al * w.p);
+      }
     }
+    const V rm = mine ? rk : V(0);
+    const V zv = rm * dw_of(w);
+    a[0] = acc64(a[0], rm, zv);
+    a[1] = acc64(a[1], rm, rm);
+  };
+  if constexpr (XM == 4) {
+    load_masks();
+    load_prologue();
   }
-  load_v(i_lo + 1, hok, HB[0], hcol, HR[1], false);
-  load_v(i_lo + 2, hok, HB[1], hcol, HR[2], false);
 #pragma unroll
   for (int u = 0; u < RPT; ++u) {
     PV[2][u] = p_of(W0[u], r_of(W0[u]));
@@ -1472,29 +1556,30 @@ __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, in
     PV[0][u] = p_of(W1[u], RV[0][u]);
     NB[0][u] = W1[u].nb;
     pl[i_lo % 3][jl0 + u + 1][kl + 1] = PV[0][u];
-    if (i_lo < i_hi) own(i_lo, u, W1[u], RV[0][u], X0[u]);
+    own(i_lo, u, W1[u], RV[0][u], X0[u], i_lo < i_hi);
   }
   if (ring) pl[i_lo % 3][hj + 1][hk + 1] = p_of(WH, r_of(WH));
   const V qc = qcoef<V>(o);
-  for (int ib = i_lo; ib < i_hi; ib += UNR) {
+  // One exit, no branch around an access: every step then issues the same
+  // loads and stores, and a wait for one of them leaves the younger ones in
+  // flight.
+  for (int ib = i_lo;; ib += UNR) {
 #pragma unroll
     for (int d = 0; d < UNR; ++d) {
       const int i = ib + d;
-      if (i < i_hi) {  // uniform over the block
+      if (i >= i_hi) goto planes_done;  // uniform over the block
+      {
         const int s0 = d % 3, s1 = (d + 1) % 3, s2 = (d + 2) % 3;
         const int sn = (i + 1) % 3, scur = i % 3;
 #pragma unroll
-        for (int u = 0; u < RPT; ++u) M[s1][u] = load_m(i + 4, cok[u], col[u]);
-        HM[s1] = load_m(i + 4, hok, hcol);
+        for (int u = 0; u < RPT; ++u) M[s1][u] = load_m(i + 4, col[u]);
+        HM[s1] = load_m(i + 4, hcol);
 #pragma unroll
-        for (int u = 0; u < RPT; ++u) load_v(i + 3, cok[u], M[s0][u], col[u], R[s0][u], true);
-        load_v(i + 3, hok, HM[s0], hcol, HR[s0], false);
+        for (int u = 0; u < RPT; ++u) load_v(i + 3, M[s0][u], col[u], R[s0][u], true);
+        load_v(i + 3, HM[s0], hcol, HR[s0], false);
         if constexpr (XM == 4) {  // x64 of plane i+2 (its mask M[s2] was read two planes ago)
 #pragma unroll
-          for (int u = 0; u < RPT; ++u) {
-            const uint8_t nb2 = (cok[u] && i + 2 < g.nx) ? M[s2][u] : (uint8_t)0;
-            XD[d & 1][u] = (x64 + plane(i + 2))[(nb2 & NB_UNKNOWN) ? col[u] : 0u];
-          }
+          for (int u = 0; u < RPT; ++u) XD[d & 1][u] = load_x64(i + 2, M[s2][u], col[u]);
         }
 #pragma unroll
         for (int u = 0; u < RPT; ++u) {
@@ -1502,11 +1587,11 @@ __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, in
           PV[s1][u] = p_of(R[s1][u], RV[s1][u]);
           NB[s1][u] = R[s1][u].nb;
           pl[sn][jl0 + u + 1][kl + 1] = PV[s1][u];
-          if (i + 1 < i_hi) own(i + 1, u, R[s1][u], RV[s1][u], XD[(d + 1) & 1][u]);
+          own(i + 1, u, R[s1][u], RV[s1][u], XD[(d + 1) & 1][u], i + 1 < i_hi);
         }
         if (ring) pl[sn][hj + 1][hk + 1] = p_of(HR[s1], r_of(HR[s1]));
         lds_barrier();
-        const int64_t pb = (int64_t)i * sx;
+        const uint32_t pb = plane(i) * 4u;
 #pragma unroll
         for (int u = 0; u < RPT; ++u) {
           const int jl = jl0 + u;
@@ -1521,26 +1606,26 @@ __global__ void __launch_bounds__(ST, 4) k_cgf(OpArgs o, Tiling T, int first, in
           sum = (nb & 8) ? sum + (PV[s2][u] - pcv) : sum;
           sum = (nb & 16) ? sum + (nym - pcv) : sum;
           sum = (nb & 32) ? sum + (nzm - pcv) : sum;
-          if (SLOW && (nb & NB_SLOW)) {
-            // slow row: p_k only, q_k from k_slow_q5
-            if (nb & NB_UNKNOWN) st_nt(pout + pb + col[u], pcv);
-          } else if (nb & NB_UNKNOWN) {
-            const V qv = sum * qc;
-            const V rk = RV[s0][u];
-            const V dv = d_of(nb);
-            const V zv = rk * dv;
-            st_nt(pout + pb + col[u], pcv);
-            st_nt(qout + pb + col[u], qv);
-            a[2] = acc64(a[2], pcv, qv);
-            a[3] = acc64(a[3], qv, zv);
-            a[4] = acc64(a[4], qv, dv * qv);
-            a[5] = acc64(a[5], qv, rk);
-            a[6] = acc64(a[6], qv, qv);
-          }
+          // a slow row stores p_k only (q_k from k_slow_q5); a cell that is no
+          // unknown has no q and adds 0
+          const bool fast = SLOW ? (nb & (NB_UNKNOWN | NB_SLOW)) == NB_UNKNOWN : (nb & NB_UNKNOWN) != 0;
+          const uint32_t cv = off_of(nb, col[u]);
+          const V qv = fast ? sum * qc : V(0);
+          const V rk = RV[s0][u];
+          const V dv = d_of(nb);
+          const V zv = rk * dv;
+          buf_st_nt(po_b, cv, pb, pcv);
+          buf_st_nt(qo_b, fast ? cv : OFF_NONE, pb, qv);
+          a[2] = acc64(a[2], pcv, qv);
+          a[3] = acc64(a[3], qv, zv);
+          a[4] = acc64(a[4], qv, dv * qv);
+          a[5] = acc64(a[5], qv, rk);
+          a[6] = acc64(a[6], qv, qv);
         }
       }
     }
   }
+planes_done:
   write_partials<FDOT, ST>(a, Pout);
 }
 
@@ -1583,7 +1668,9 @@ __global__ void __launch_bounds__(SQ, 4) k_cgq(OpArgs o, Tiling T, int nres, int
   if (sc->done && sc->done_k != k) return;
   __shared__ V dtab[8];
   if (threadIdx.x < 8) dtab[threadIdx.x] = (threadIdx.x < 7) ? dinv_tab<V>(o, threadIdx.x) : V(1);
-  const CgScalars cs = cg_scalars<SQ>(T, nres, first, nbu, Pprev, Pres, sc, k, tol, cap);
+  CgSums sums;
+  cg_sums<SQ>(T, nres, first, nbu, Pprev, Pres, sums);
+  const CgScalars cs = cg_scalars<SQ>(sums, first, Pres, sc, k, tol, cap);
   const V al = (V)cs.ald, bev = (V)cs.be;
   __shared__ V pa[2][LJ2][LK2];  // p_{k-1}: planes with two rings
   __shared__ V pk[2][LJ][LK];    // p_k: planes with one ring
@@ -1989,6 +2076,9 @@ Tiling make_tiling(const Grid& g, int blocks, int tk) {
   int nseg = blocks / tiles;
   if (nseg < 1) nseg = 1;
   if (nseg > g.nx) nseg = g.nx;
+  // a run's planes as FP64 values stay within 32-bit byte offsets
+  const int64_t most = std::max<int64_t>(1, 0xfffffff0ll / (8 * (int64_t)g.ny * g.nz) - 6);
+  if (nseg < (g.nx + most - 1) / most) nseg = (int)((g.nx + most - 1) / most);
   t.seg = (g.nx + nseg - 1) / nseg;
   nseg = (g.nx + t.seg - 1) / t.seg;
   t.nblk = tiles * nseg;
@@ -1998,8 +2088,9 @@ Tiling make_tiling(const Grid& g, int blocks, int tk) {
 // Wide tiles read whole 512-byte rows and fewer ring cells per plane; narrow
 // ones pad less where nz ends early in the last wide tile.  A launch costs
 // about (seg + 3) plane steps (three fill the pipeline), a narrow step up to
-// 8/7 of a wide one: 105 us a narrow launch against 94 at 256^3, where both
-// run 32 planes; 56 against 64 at 192^3, 14 planes against 20.
+// 8/7 of a wide one (105 us a narrow launch against 94 at 256^3, where both
+// run 32 planes; 56 against 64 at 192^3, 14 planes against 20, before the
+// plane loop lost its branches).
 Tiling make_tiling(const Grid& g, int blocks) {
   const Tiling w = make_tiling(g, blocks, TK_WIDE), n = make_tiling(g, blocks, TK_NARROW);
   return 8 * (n.seg + 3) < 7 * (w.seg + 3) ? n : w;
@@ -2169,9 +2260,7 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
       double* S7[2] = {c.partials + 8 * MAX_BLK, c.partials + 22 * MAX_BLK};
       double* Rs = c.partials + 36 * MAX_BLK;
       // x advances every other launch (modes 2 and 3 of k_cgf), and fully
-      // before each true-residual pass; not with slow rows on wide tiles,
-      // whose mode 3 spills (89 and 124 us a launch in turn against 105 at
-      // 256^3; on narrow tiles 46 and 58 against 55 at 192^3)
+      // before each true-residual pass
       struct Iter {
         decltype(&k_cgf<OPk, false, false, 1, TK_WIDE>) any, steady, skip, twice, fold;
       };
@@ -2179,16 +2268,8 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
   Iter { k_cgf<OPk, SL, false, 1, W>, k_cgf<OPk, SL, true, 1, W>, k_cgf<OPk, SL, true, 2, W>, \
          k_cgf<OPk, SL, true, 3, W>, k_cgf<OPk, SL, false, 4, W> }
       Iter it = wide ? MPF_ITER(false, TK_WIDE) : MPF_ITER(false, TK_NARROW);
-      bool halves = true;
-      if constexpr (OPk == OP_VARDENS) {
-        if (nslow > 0 && wide) {
-          it.any = it.fold = k_cgf<OPk, true, false, 1, TK_WIDE>;
-          it.steady = k_cgf<OPk, true, true, 1, TK_WIDE>;
-          halves = false;
-        } else if (nslow > 0) {
-          it = MPF_ITER(true, TK_NARROW);
-        }
-      }
+      if constexpr (OPk == OP_VARDENS)
+        if (nslow > 0) it = wide ? MPF_ITER(true, TK_WIDE) : MPF_ITER(true, TK_NARROW);
 #undef MPF_ITER
       bool pending = false;  // the last launch left alpha p in x's debt
       auto res_tiles = nslow > 0 ? (wide ? k_resid64<OPk, 2, TK_WIDE> : k_resid64<OPk, 2, TK_NARROW>) : resid64;
@@ -2221,7 +2302,7 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
               if (pending) {
                 kern = it.twice;
                 pending = false;
-              } else if (halves && (k + 1) % R != 0 && k < cap) {
+              } else if ((k + 1) % R != 0 && k < cap) {
                 kern = it.skip;
                 pending = true;
               }
