@@ -26,10 +26,10 @@
 // The launch is cooperative: every block is resident before any polls.
 //
 // Measured per iteration (one MI355X, launch form -> this one): FP32 with an
-// air ball 23.0 -> 5.6 us at 64^3, FP32 28.8 -> 9.8 us at 128^3 and 40.7 -> 19.2
-// at 144^3; FP64 46.1 -> 15.5 us at 96^3 and 44.3 -> 24.5 at 128^3; MIXED 20.9 ->
-// 6.7 us at 64^3, 23.1 -> 12.7 at 128^3 and 33.0 -> 26.9 at 132^3, true residuals
-// included.  About 5.5 us is the meeting (two trips through memory, the sums
+// air ball 23.0 -> 4.8 us at 64^3, FP32 28.8 -> 9.5 us at 128^3 and 40.7 -> 19.2
+// at 144^3; FP64 with six air balls 46.1 -> 12.7 us at 96^3, without 44.3 -> 25.0
+// at 128^3; MIXED 20.9 -> 6.0 us at 64^3, 23.1 -> 12.4 at 128^3 and 33.0 -> 26.9
+// at 132^3, true residuals included.  About 4.5 us is the meeting (two trips through memory, the sums
 // and the scalars; 32 or 200 blocks differ by 0.4 us), the rest grows with the
 // cells per thread and is vector arithmetic and LDS.  Every grid that fits
 // gained, so the rule is that it fits (resident_tile).
@@ -44,6 +44,7 @@ constexpr uint32_t RES_NONE = 0xffffffffu;
 struct ResTile {
   int bi, bj, nti, ntj, nblk, cols, cells;  // tile rows, tiles, blocks; columns (bj * nz) and cells of a full tile
   int m, mj;                                // compiled cells per thread (>= bi), j ring cells per thread
+  int dl, dr;                               // FP64: 1/diag in LDS, of own cells, of ring cells
   size_t lds;
   FastDiv dbi;  // by bi * nz
 };
@@ -224,11 +225,17 @@ __device__ __forceinline__ bool grid_meet(const double (&v)[8], uint32_t seq, ui
 // establishes r.z and r.r: of the start, of the residual whose prediction met
 // the criterion (FP32 and FP64 forms), or of the FP64 true residual of x
 // (MIXED form).
-// Registers are what a larger column runs out of: the FP64 form looks 1/diag
-// up by the open faces of a cell instead of keeping it (KD), and x lives in
-// LDS (XL) in the larger columns, where x64 of the MIXED form (always in LDS)
-// leaves the room.
+// Registers are what a larger column runs out of: the FP64 form keeps 1/diag
+// in LDS where there is room (T.dl, T.dr) and looks it up by the open faces of
+// a cell, or in memory for a slow row, elsewhere, and x lives in LDS (XL) in
+// the larger columns, where x64 of the MIXED form (always in LDS) leaves the
+// room.  The face weights of a slow row are read res_nbf at a time: one by one
+// they were a chain of up to six round trips (FP64 at 96^3 with bubbles 15.7 us
+// an iteration, 12.9 so, 12.7 with 1/diag in LDS, which at 112^3 takes 23.9 to
+// 20.9; MIXED at 128^3 with bubbles 25.4 -> 17.8); all six at once spill in the
+// larger columns.
 constexpr bool res_xl(int m, bool d64, bool mix) { return d64 ? m >= 3 : mix ? m == 8 : m >= 8; }
+constexpr int res_nbf(int m, bool d64, bool mix) { return m <= (d64 ? 4 : mix ? 6 : 8) ? 6 : 3; }
 template <class V, bool MIX, int M, int MJ>
 __global__ void __launch_bounds__(RT)
     k_cg_resident(OpArgs o, ResArgs<V> ra, const V* __restrict__ b, V* __restrict__ xout, double* __restrict__ x64out,
@@ -237,6 +244,8 @@ __global__ void __launch_bounds__(RT)
   __shared__ ResShared sh;
   __shared__ V dtab[8];
   constexpr bool D64 = sizeof(V) == 8, KD = !D64, XL = res_xl(M, D64, MIX);
+  constexpr int NBF = res_nbf(M, D64, MIX);
+  constexpr bool DL = D64 && M <= 6, DR = D64 && M <= 4;
   const Grid& g = o.g;
   const ResTile& T = ra.t;
   const int t = threadIdx.x, blk = blockIdx.x;
@@ -258,6 +267,8 @@ __global__ void __launch_bounds__(RT)
   double* const lx = (double*)smem;                        // MIX: x64 of the tile and its j ring, laid out as p
   V* const lp = (V*)smem + (MIX ? 2 * T.bi * SM : 0);      // p of the tile and its j ring: [bi][bj + 2][nz]
   V* const xs_ = lp + T.bi * SM + (uint32_t)t;             // XL: x of own cell m at xs_[m * RT]
+  V* const ds_ = xs_ + (XL ? M * RT : 0);                  // T.dl: 1/diag of own cell m at ds_[m * RT]
+  V* const dr_ = ds_ + (T.dl ? M * RT : 0);                // T.dr: of the i ring below and above, of j ring cell m at 2 + m
   if (t < 8) dtab[t] = (t < 7 && o.precond) ? dinv_tab<V>(o, t) : V(1);
   if (t == 0) sh = ResShared{0, 0, 0, 0, 0, 0, 0, -1.0, 0, 0, 0, 0, 0, 0, 0};
   for (int q = t; q < T.bi * SM; q += RT) {
@@ -284,11 +295,13 @@ __global__ void __launch_bounds__(RT)
     if constexpr (XL) xs_[m * RT] = V(0);
     else x[m] = V(0);
     if constexpr (KD) d[m] = V(1);
+    else if (DL && T.dl) ds_[m * RT] = V(1);
     if (act && m < ni) {
       const uint32_t idx = gidx + (uint32_t)m * sx;
       const uint32_t nb = o.nbm[idx];
       nbw[m / 4] |= nb << (8 * (m & 3));
       if constexpr (KD) d[m] = dinv_of(idx, nb);
+      else if (DL && T.dl) ds_[m * RT] = dinv_of(idx, nb);
       if (nb & NB_UNKNOWN) r[m] = b[idx];
       if ((nb & (NB_UNKNOWN | NB_SLOW)) == (NB_UNKNOWN | NB_SLOW)) {
         const int8_t mk = o.mark[idx];
@@ -303,15 +316,18 @@ __global__ void __launch_bounds__(RT)
   // i ring: the cells below and above the column, in this thread
   V rl = V(0), rh = V(0), pl = V(0), ph = V(0), dl = V(1), dh = V(1);
   uint32_t nbr = 0;  // their masks
+  if (DR && T.dr) dr_[0] = dr_[RT] = V(1);
   if (has_lo) {
     const uint32_t idx = gidx - sx, nb = o.nbm[idx];
     if constexpr (KD) dl = dinv_of(idx, nb);
+    else if (DR && T.dr) dr_[0] = dinv_of(idx, nb);
     nbr = nb;
     if (nb & NB_UNKNOWN) rl = b[idx];
   }
   if (has_hi) {
     const uint32_t idx = gidx + (uint32_t)ni * sx, nb = o.nbm[idx];
     if constexpr (KD) dh = dinv_of(idx, nb);
+    else if (DR && T.dr) dr_[RT] = dinv_of(idx, nb);
     nbr |= nb << 8;
     if (nb & NB_UNKNOWN) rh = b[idx];
   }
@@ -332,6 +348,7 @@ __global__ void __launch_bounds__(RT)
       const uint32_t idx = ((uint32_t)(i0 + (int)mi) * (uint32_t)g.ny + (uint32_t)j) * (uint32_t)nz + k2;
       const uint32_t nb = o.nbm[idx];
       if constexpr (KD) dg[m] = dinv_of(idx, nb);
+      else if (DR && T.dr) dr_[(2 + m) * RT] = dinv_of(idx, nb);
       if (nb & NB_UNKNOWN) rg[m] = b[idx];
       Lg[m] = (uint32_t)((int)mi * SM + (side == 0 ? 0 : nj + 1) * nz + (int)k2) | (nb << 24);
       ho[m] = (uint32_t)(side == 0 ? blk - 1 : blk + 1) * (uint32_t)T.cells + mi * cols +
@@ -348,6 +365,7 @@ __global__ void __launch_bounds__(RT)
   };
   auto d_own = [&](int m, uint32_t nb) -> V {
     if constexpr (KD) return d[m];
+    else if (DL && T.dl) return ds_[m * RT];
     else return d_table(nb, [&]() { return fresh(gidx) + (uint32_t)m * sx; });
   };
   auto nb_own = [&](int m) -> uint32_t { return (fresh(nbw[m / 4]) >> (8 * (m & 3))) & 0xffu; };
@@ -429,6 +447,9 @@ __global__ void __launch_bounds__(RT)
       if constexpr (KD) {
         pl = rl * dl + be * pl;
         ph = rh * dh + be * ph;
+      } else if (DR && T.dr) {
+        pl = rl * dr_[0] + be * pl;
+        ph = rh * dr_[RT] + be * ph;
       } else {
         pl = rl * d_table(fresh(nbr) & 0xffu, [&]() { return fresh(gidx) - sx; }) + be * pl;
         ph = rh * d_table(fresh(nbr) >> 8, [&]() { return fresh(gidx) + (uint32_t)ni * sx; }) + be * ph;
@@ -439,6 +460,7 @@ __global__ void __launch_bounds__(RT)
           const uint32_t lg = fresh(Lg[m]), L = lg & 0xffffffu;
           V dv;
           if constexpr (KD) dv = dg[m];
+          else if (DR && T.dr) dv = dr_[(2 + m) * RT];
           else dv = d_table(lg >> 24, [&]() {  // the row's plane and column from its place in the tile
             const uint32_t row = fdiv(L, g.dnz), mi = row / (uint32_t)(T.bj + 2);
             const uint32_t jr = row - mi * (uint32_t)(T.bj + 2);
@@ -470,8 +492,15 @@ __global__ void __launch_bounds__(RT)
             s = V(0);
             const V pn[6] = {n0, n1, n2, n3, n4, n5};
 #pragma unroll
-            for (int f = 0; f < 6; ++f)
-              if (nb & (1u << f)) s += ra.beta[f][idx] * (pn[f] - pc);
+            for (int f0 = 0; f0 < 6; f0 += NBF) {
+              V bf[NBF];  // read together (a closed face's weight is not used)
+#pragma unroll
+              for (int f = 0; f < NBF; ++f) bf[f] = ra.beta[f0 + f][idx];
+              if (NBF < 6) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+              for (int f = 0; f < NBF; ++f) s = (nb & (1u << (f0 + f))) ? s + bf[f] * (pn[f0 + f] - pc) : s;
+              if (NBF < 6) __builtin_amdgcn_sched_barrier(0);
+            }
             qv = s / ((V)g.h * (V)g.h);
           }
           q[m] = qv;
@@ -735,7 +764,17 @@ inline bool resident_tile(const Grid& g, int most, int esize, bool mix, ResTile&
       out.cols = bj * g.nz;
       out.cells = bi * bj * g.nz;
       out.m = RES_M[mi]; out.mj = RES_MJ[mi];
-      out.lds = (size_t)lds;
+      out.dl = out.dr = 0;
+      int64_t more = lds;
+      if (esize == 8 && out.m <= 6 && more + (int64_t)out.m * RT * 8 <= RES_LDS_MAX) {
+        out.dl = 1;
+        more += (int64_t)out.m * RT * 8;
+      }
+      if (esize == 8 && out.m <= 4 && more + (int64_t)(2 + out.mj) * RT * 8 <= RES_LDS_MAX) {
+        out.dr = 1;
+        more += (int64_t)(2 + out.mj) * RT * 8;
+      }
+      out.lds = (size_t)more;
     }
   }
   if (best < 0) return false;
