@@ -282,28 +282,33 @@ __global__ void __launch_bounds__(256, 8) k_genlevelset(Grid g, const f3* __rest
   lsair[idx] = mair - r;
 }
 
-// markLS_bigpositive spray_k.cu:3683-3697 (mode 0) / preparels 3708-3722 (mode 1)
-__global__ void k_ls_prepare(int64_t G, const float* __restrict__ ls, float* __restrict__ out,
-                             int8_t* __restrict__ mark, float h, int mode) {
+// markLS_bigpositive spray_k.cu:3683-3697 (outward, from the distances) /
+// setLSback_bigpositive and preparels 3699-3722 (inward, from the outward
+// result; the distances between are not kept: the inward passes write all of
+// ls), of both level sets.
+struct LsPair {
+  float* ls[2];
+  float* out[2];
+  int8_t* mark[2];
+};
+template <bool INWARD>
+__global__ void k_ls_prepare(int64_t G, LsPair p, float h) {
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= G) return;
+  const float* __restrict__ ls = blockIdx.y ? p.ls[1] : p.ls[0];
+  float* __restrict__ out = blockIdx.y ? p.out[1] : p.out[0];
+  int8_t* __restrict__ mark = blockIdx.y ? p.mark[1] : p.mark[0];
   float v = ls[idx];
-  if (mode == 0) {
+  if (!INWARD) {
     v = v / h;
     if (v > 1.99f) { v = 5.0f; mark[idx] = AIR; }
     else mark[idx] = FLUID;
   } else {
-    v = -v / h;
+    v = -(v * h) / h;
     if (v > 0) { v = 5.0f; mark[idx] = AIR; }
     else mark[idx] = FLUID;
   }
   out[idx] = v;
-}
-// setLSback_bigpositive spray_k.cu:3699-3706 (mode 0) / setLSback 3724-3731 (mode 1)
-__global__ void k_ls_back(int64_t G, float* __restrict__ ls, float h, int mode) {
-  int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= G) return;
-  ls[idx] = (mode == 0) ? ls[idx] * h : -ls[idx] * h;
 }
 
 // One triple of solvedistance (spray_k.cu:746-754: d = min(a,b,c) + 1, or
@@ -368,10 +373,25 @@ __device__ __forceinline__ uint8_t tile_flags(bool changed) {
   return (uint8_t)((bal ? SF_ANY : 0) | ((bal & JLO) ? SF_JLO : 0) | ((bal & JHI) ? SF_JHI : 0) |
                    ((bal & KLO) ? SF_KLO : 0) | ((bal & KHI) ? SF_KHI : 0));
 }
+// One pass over one field, or over two at once (blockIdx.y): most passes of a
+// series find few tiles to compute and cost little more than their launch.
+struct SweepPass {
+  const float* in;
+  float* out;
+  const int8_t* mark;
+  int typeflag;
+  const uint8_t* prev;
+  uint8_t* cur;
+};
 __global__ void __launch_bounds__(256)
-    k_sweep(Grid g, const float* __restrict__ in, float* __restrict__ out, const int8_t* __restrict__ mark,
-            int typeflag, const uint8_t* __restrict__ prev, uint8_t* __restrict__ cur, uint32_t ntj, uint32_t ntk,
-            uint32_t ntiles) {
+    k_sweep(Grid g, SweepPass p0, SweepPass p1, uint32_t ntj, uint32_t ntk, uint32_t ntiles) {
+  const bool second = blockIdx.y != 0;
+  const float* __restrict__ in = second ? p1.in : p0.in;
+  float* __restrict__ out = second ? p1.out : p0.out;
+  const int8_t* __restrict__ mark = second ? p1.mark : p0.mark;
+  const int typeflag = second ? p1.typeflag : p0.typeflag;
+  const uint8_t* __restrict__ prev = second ? p1.prev : p0.prev;
+  uint8_t* __restrict__ cur = second ? p1.cur : p0.cur;
   const uint32_t t0 = (blockIdx.x * 4u + threadIdx.x / 64u) * SW_L;
   if (t0 >= ntiles) return;
   const int lane = threadIdx.x & 63;
@@ -430,12 +450,15 @@ __global__ void __launch_bounds__(256)
   if (mine) cur[tl] = myflag;
 }
 
-// mergeLSAndMarkGrid spray_k.cu:3733-3777
-__global__ void k_merge(Grid g, const float* __restrict__ lsfluid, const float* __restrict__ lsair,
-                        float* __restrict__ lsmerge, int8_t* __restrict__ mark) {
+// setLSback spray_k.cu:3724-3731 of both level sets, and mergeLSAndMarkGrid
+// 3733-3777
+__global__ void k_merge(Grid g, float* __restrict__ lsfluid, float* __restrict__ lsair, float* __restrict__ lsmerge,
+                        int8_t* __restrict__ mark) {
   CELL_LOOP_HEAD
   const float h = g.h;
-  float lf = lsfluid[idx], la = lsair[idx], lm;
+  float lf = -lsfluid[idx] * h, la = -lsair[idx] * h, lm;
+  lsfluid[idx] = lf;
+  lsair[idx] = la;
   int8_t m;
   if (la > 4.99f * h) { lm = lf; m = (lf > 0) ? VACUUM : FLUID; }
   else if (lf > 4.99f * h) { lm = la; m = (la > 0) ? VACUUM : AIR; }
@@ -870,11 +893,9 @@ __global__ void __launch_bounds__(ST_CELLS, 4)
 // tile order (also into out2 when given: the copy the FLIP update keeps).
 // Band mode: faces without a cell of band < big beside them are 0.
 template <int A>
-__global__ void k_p2g_collect(Grid g, const float* __restrict__ parts, int ntx, int nty, int ntz,
-                              float* __restrict__ out, float* __restrict__ out2, int64_t nf,
-                              const float* __restrict__ band, float big) {
-  int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nf) return;
+__device__ __forceinline__ void p2g_collect_face(const Grid& g, const float* __restrict__ parts, int ntx, int nty,
+                                                 int ntz, float* __restrict__ out, float* __restrict__ out2, int64_t f,
+                                                 const float* __restrict__ band, float big) {
   int i, j, k;
   ijk_face<A>(g, f, i, j, k);
   if (band) {
@@ -917,11 +938,26 @@ __global__ void k_p2g_collect(Grid g, const float* __restrict__ parts, int ntx, 
   if (out2) out2[f] = u;
 }
 
+__global__ void k_p2g_collect(Grid g, const float* __restrict__ parts, int ntx, int nty, int ntz, P2GOut o,
+                              const float* __restrict__ band, float big) {
+  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int A = blockIdx.y;
+  if (f >= (A == 0 ? g.FX : A == 1 ? g.FY : g.FZ)) return;
+  if (A == 0) p2g_collect_face<0>(g, parts, ntx, nty, ntz, o.u[0], o.u2[0], f, band, big);
+  else if (A == 1) p2g_collect_face<1>(g, parts, ntx, nty, ntz, o.u[1], o.u2[1], f, band, big);
+  else p2g_collect_face<2>(g, parts, ntx, nty, ntz, o.u[2], o.u2[2], f, band, big);
+}
+
 // ---------------- extrapolation + wall conditions (a10) ----------------
 // initphi, spray_k.cu:712-723
-__global__ void k_initphi(int64_t G, const int8_t* __restrict__ mark, float* __restrict__ phi, int8_t type, float big) {
+// (both phases)
+__global__ void k_initphi(int64_t G, const int8_t* __restrict__ mark, float* __restrict__ phi0, int8_t type0,
+                          float* __restrict__ phi1, int8_t type1, float big) {
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx < G) phi[idx] = (mark[idx] == type) ? -0.5f : big;
+  if (idx >= G) return;
+  const int8_t m = mark[idx];
+  phi0[idx] = (m == type0) ? -0.5f : big;
+  phi1[idx] = (m == type1) ? -0.5f : big;
 }
 
 // sweepu_k_bubble spray_k.cu:3779-3880 (one axis, out-of-place): the new
@@ -1018,10 +1054,10 @@ __device__ __forceinline__ float sweep_u_face(const Grid& g, const float* __rest
 // be null) records the changes of this pass; prev == nullptr computes every
 // tile.  A change is a different bit pattern.
 template <int A>
-__global__ void __launch_bounds__(256)
-    k_sweep_u(Grid g, const float* __restrict__ u, float* __restrict__ out, const float* __restrict__ ls,
-              const int8_t* __restrict__ mark, int8_t sf, const uint8_t* __restrict__ prev, uint8_t* __restrict__ cur,
-              uint32_t ntj, uint32_t ntk, uint32_t ntiles, int per_wave) {
+__device__ __forceinline__ void
+    sweep_u_tiles(const Grid& g, const float* __restrict__ u, float* __restrict__ out, const float* __restrict__ ls,
+                  const int8_t* __restrict__ mark, int8_t sf, const uint8_t* __restrict__ prev,
+                  uint8_t* __restrict__ cur, uint32_t ntj, uint32_t ntk, uint32_t ntiles, int per_wave) {
   const uint32_t t0 = (blockIdx.x * 4u + threadIdx.x / 64u) * (uint32_t)per_wave;
   if (t0 >= ntiles) return;
   const int lane = threadIdx.x & 63;
@@ -1051,15 +1087,36 @@ __global__ void __launch_bounds__(256)
   if (cur && lane < per_wave && t0 + lane < ntiles) cur[t0 + lane] = myflag;
 }
 
+// The six fields (phase and axis: blockIdx.y = 3 phase + axis) in one launch:
+// one by one their passes took 19 us each at 128^3, most of it the launch and
+// its last waves.
+struct SweepU {
+  const float* u[6];
+  float* out[6];
+  const float* ls[2];
+  int8_t sf[2];
+  uint8_t* flags[6];
+};
+template <bool FIRST>
+__global__ void __launch_bounds__(256) k_sweep_u(Grid g, SweepU s, const int8_t* __restrict__ mark, int per_wave) {
+  const int ph = blockIdx.y / 3, A = blockIdx.y % 3, q = blockIdx.y;
+  const int64_t nfx = g.nx + (A == 0), nfy = g.ny + (A == 1), nfz = g.nz + (A == 2);
+  const uint32_t ntj = (uint32_t)((nfy + SW_J - 1) / SW_J), ntk = (uint32_t)((nfz + SW_K - 1) / SW_K);
+  const uint32_t nt = (uint32_t)nfx * ntj * ntk;
+  const uint8_t* prev = FIRST ? nullptr : s.flags[q];
+  uint8_t* cur = FIRST ? s.flags[q] : nullptr;
+  if (A == 0) sweep_u_tiles<0>(g, s.u[q], s.out[q], s.ls[ph], mark, s.sf[ph], prev, cur, ntj, ntk, nt, per_wave);
+  else if (A == 1) sweep_u_tiles<1>(g, s.u[q], s.out[q], s.ls[ph], mark, s.sf[ph], prev, cur, ntj, ntk, nt, per_wave);
+  else sweep_u_tiles<2>(g, s.u[q], s.out[q], s.ls[ph], mark, s.sf[ph], prev, cur, ntj, ntk, nt, per_wave);
+}
+
 // setWaterBoundaryU_k spray_k.cu:956-995 (in place).  The ceiling rule reads
 // uz(k-1) after that face's own rule.
 __device__ __forceinline__ bool isb(const Grid& g, const int8_t* mark, int i, int j, int k) {
   return mark[cid(g, i, j, k)] == BOUNDARY;
 }
 template <int A>
-__global__ void k_bc(Grid g, float* __restrict__ u, const int8_t* __restrict__ mark, int64_t nf) {
-  int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nf) return;
+__device__ __forceinline__ void bc_face(const Grid& g, float* __restrict__ u, const int8_t* __restrict__ mark, int64_t f) {
   const int hh = g.ny + (A == 1), d = g.nz + (A == 2);
   int i, j, k;
   ijk_face<A>(g, f, i, j, k);
@@ -1081,6 +1138,19 @@ __global__ void k_bc(Grid g, float* __restrict__ u, const int8_t* __restrict__ m
       u[f] = (b < 0) ? b : 0.0f;
     } else if (k > 0 && k < g.nz && (isb(g, mark, i, j, k) != isb(g, mark, i, j, k - 1))) u[f] = 0.0f;
   }
+}
+
+struct Faces6 {
+  float* u[6];  // water x, y, z, air x, y, z
+};
+__global__ void k_bc(Grid g, Faces6 fs, const int8_t* __restrict__ mark) {
+  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int A = blockIdx.y % 3;
+  if (f >= (A == 0 ? g.FX : A == 1 ? g.FY : g.FZ)) return;
+  float* u = fs.u[blockIdx.y];
+  if (A == 0) bc_face<0>(g, u, mark, f);
+  else if (A == 1) bc_face<1>(g, u, mark, f);
+  else bc_face<2>(g, u, mark, f);
 }
 
 // ---------------- divergence (a11) and gradient (a13) ----------------
@@ -1128,10 +1198,9 @@ __global__ void k_divergence(Grid g, const float* __restrict__ wux, const float*
 
 // subGradPress spray_k.cu:198-224 (unit form, in R) or the 1/rho form (double).
 template <int A, class R>
-__global__ void k_subgrad(Grid g, float* __restrict__ u, const R* __restrict__ p, const int8_t* __restrict__ mark,
-                          int vardens, double inv_rho, int solid_c, int64_t nf) {
-  int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nf) return;
+__device__ __forceinline__ void subgrad_face(const Grid& g, float* __restrict__ u, const R* __restrict__ p,
+                                             const int8_t* __restrict__ mark, int vardens, double inv_rho, int solid_c,
+                                             int64_t f) {
   const int hh = g.ny + (A == 1), d = g.nz + (A == 2);
   int i, j, k;
   ijk_face<A>(g, f, i, j, k);
@@ -1146,6 +1215,19 @@ __global__ void k_subgrad(Grid g, float* __restrict__ u, const R* __restrict__ p
   }
   if (!vardens) u[f] = (float)((R)u[f] - (p[c0] - p[c1]) / (R)g.h);
   else u[f] = (float)((double)u[f] - inv_rho * (((double)p[c0] - (double)p[c1]) / (double)g.h));
+}
+
+template <class R>
+__global__ void k_subgrad(Grid g, Faces6 fs, const R* __restrict__ p, const int8_t* __restrict__ mark, int vardens,
+                          double inv_rho_liquid, double inv_rho_air, int solid_c) {
+  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int A = blockIdx.y % 3;
+  if (f >= (A == 0 ? g.FX : A == 1 ? g.FY : g.FZ)) return;
+  float* u = fs.u[blockIdx.y];
+  const double inv_rho = blockIdx.y < 3 ? inv_rho_liquid : inv_rho_air;
+  if (A == 0) subgrad_face<0, R>(g, u, p, mark, vardens, inv_rho, solid_c, f);
+  else if (A == 1) subgrad_face<1, R>(g, u, p, mark, vardens, inv_rho, solid_c, f);
+  else subgrad_face<2, R>(g, u, p, mark, vardens, inv_rho, solid_c, f);
 }
 
 // ---------------- heat grid stages (a16) ----------------
@@ -1713,33 +1795,44 @@ __global__ void k_mc_density(McGrid m, Grid g2, const f3* __restrict__ pos, cons
 // copy at the end when n is odd).
 // n passes ending in phi; the initial field is in c.ctmp when in_tmp (the
 // preparing kernel wrote it there, so an odd n needs no final copy)
-static void sweep_n(Ctx& c, float* phi, int typeflag, int n, bool in_tmp = false) {
-  float* src = in_tmp ? c.ctmp : phi;
-  float* dst = in_tmp ? phi : c.ctmp;
+// n passes (odd) over one field or two: from tmp into phi and back, the last
+// into phi.  flags: two sets of tile flags.
+struct SweepJob {
+  float* phi;
+  float* tmp;
+  const int8_t* mark;
+  int typeflag;
+  uint8_t* flags;
+};
+static void sweep_n(Ctx& c, const SweepJob* jobs, int njobs, int n) {
   const uint32_t ntj = (uint32_t)((c.g.ny + SW_J - 1) / SW_J), ntk = (uint32_t)((c.g.nz + SW_K - 1) / SW_K);
   const int64_t nt = sweep_tiles(c.g);
   const int64_t nwaves = (nt + SW_L - 1) / SW_L;
   for (int it = 0; it < n; ++it) {
-    const uint8_t* prev = it == 0 ? nullptr : c.sflag + ((it - 1) & 1) * nt;
-    launch(c, "sweep", dim3((unsigned)((nwaves + 3) / 4)), dim3(256), 0, k_sweep, c.g, (const float*)src, dst,
-           (const int8_t*)c.mark, typeflag, prev, c.sflag + (it & 1) * nt, ntj, ntk, (uint32_t)nt);
-    float* t = src;
-    src = dst;
-    dst = t;
+    SweepPass p[2];
+    for (int q = 0; q < 2; ++q) {
+      const SweepJob& j = jobs[q < njobs ? q : 0];
+      p[q] = SweepPass{(it & 1) ? j.phi : j.tmp, (it & 1) ? j.tmp : j.phi, j.mark, j.typeflag,
+                       it == 0 ? nullptr : j.flags + ((it - 1) & 1) * nt, j.flags + (it & 1) * nt};
+    }
+    launch(c, "sweep", dim3((unsigned)((nwaves + 3) / 4), njobs), dim3(256), 0, k_sweep, c.g, p[0], p[1], ntj, ntk,
+           (uint32_t)nt);
   }
-  if (src != phi) hipMemcpyAsync(phi, src, (size_t)c.g.G * 4, hipMemcpyDeviceToDevice, c.stream);
 }
 
-static void redistance(Ctx& c, float* ls) {
+// Both level sets together; the second takes its scratch values from a face
+// field's scratch, its marks from the liquid P2G's (free here) and its flags
+// from the extrapolation's (at least three sets of face tiles).
+static void redistance(Ctx& c) {
   const int64_t G = c.g.G;
-  launch(c, "ls_prepare", dim3(nblocks(G, 256)), dim3(256), 0, k_ls_prepare, G, (const float*)ls, c.ctmp, c.mark,
-         c.g.h, 0);
-  sweep_n(c, ls, FLUID, 5, true);
-  launch(c, "ls_back", dim3(nblocks(G, 256)), dim3(256), 0, k_ls_back, G, ls, c.g.h, 0);
-  launch(c, "ls_prepare", dim3(nblocks(G, 256)), dim3(256), 0, k_ls_prepare, G, (const float*)ls, c.ctmp, c.mark,
-         c.g.h, 1);
-  sweep_n(c, ls, FLUID, 5, true);
-  launch(c, "ls_back", dim3(nblocks(G, 256)), dim3(256), 0, k_ls_back, G, ls, c.g.h, 1);
+  int8_t* mark2 = (int8_t*)c.p2g_parts;
+  const LsPair p{{c.lsfluid, c.lsair}, {c.ctmp, c.ftmp[0]}, {c.mark, mark2}};
+  const SweepJob jobs[2] = {{c.lsfluid, c.ctmp, c.mark, FLUID, c.sflag},
+                            {c.lsair, c.ftmp[0], mark2, FLUID, c.sflag + 2 * sweep_tiles(c.g)}};
+  launch(c, "ls_prepare", dim3(nblocks(G, 256), 2), dim3(256), 0, k_ls_prepare<false>, G, p, c.g.h);
+  sweep_n(c, jobs, 2, 5);
+  launch(c, "ls_prepare", dim3(nblocks(G, 256), 2), dim3(256), 0, k_ls_prepare<true>, G, p, c.g.h);
+  sweep_n(c, jobs, 2, 5);
 }
 
 // Brick summary of the occupancy masks (after every change of the masks).
@@ -1778,10 +1871,8 @@ void run_levelset(Ctx& c) {
   launch(c, "genlevelset", dim3(nblocks(G, 256)), dim3(256), 0, k_genlevelset, c.g, (const f3*)c.pos[cur],
          (const int8_t*)c.flag[cur], (const uint32_t*)c.cstart, (const uint32_t*)c.cend, (const uint8_t*)c.cmask,
          (const uint8_t*)(c.bmask + NB), rb, c.lsfluid, c.lsair, c.mark);
-  redistance(c, c.lsfluid);
-  redistance(c, c.lsair);
-  launch(c, "merge_mark", dim3(nblocks(G, 256)), dim3(256), 0, k_merge, c.g, (const float*)c.lsfluid,
-         (const float*)c.lsair, c.lsmerge, c.mark);
+  redistance(c);
+  launch(c, "merge_mark", dim3(nblocks(G, 256)), dim3(256), 0, k_merge, c.g, c.lsfluid, c.lsair, c.lsmerge, c.mark);
   launch(c, "phigrad", dim3(nblocks(G, 256)), dim3(256), 0, k_phigrad, c.g, (const float*)c.lsmerge, c.phig[0],
          c.phig[1], c.phig[2]);
   if (c.cfg.flags_from_counts)
@@ -1791,6 +1882,8 @@ void run_levelset(Ctx& c) {
     launch(c, "mark_solid", dim3(nblocks(G, 256)), dim3(256), 0, k_mark_solid, c.g, (const uint32_t*)c.cstart,
            (const uint32_t*)c.cend, (const int8_t*)c.flag[cur], (const uint8_t*)c.cmask, c.mark);
 }
+
+static unsigned face_blocks(const Grid& g) { return nblocks(std::max(g.FX, std::max(g.FY, g.FZ)), 256); }
 
 static void p2g_air(Ctx& c, float* const* out, float* const* out2) {
   const int cur = c.cur;
@@ -1803,7 +1896,7 @@ static void p2g_air(Ctx& c, float* const* out, float* const* out2) {
   if (c.own_sort) run_air_regular(c, rb);
   // lists given by the caller need not be consecutive along a row
   auto kern = c.own_sort ? k_p2g_air<true> : k_p2g_air<false>;
-  launch(c, "p2g_air", dim3(nblocks(std::max(c.g.FX, std::max(c.g.FY, c.g.FZ)), 256), 3), dim3(256), 0, kern, c.g,
+  launch(c, "p2g_air", dim3(face_blocks(c.g), 3), dim3(256), 0, kern, c.g,
          (const f3*)c.pos[cur], (const f3*)c.vel[cur], (const float*)c.mass[cur], (const int8_t*)c.flag[cur],
          (const uint32_t*)c.cstart, (const uint32_t*)c.cend, rb, (const uint8_t*)(c.bmask + nbricks(c.g)), o);
 }
@@ -1816,14 +1909,13 @@ static void p2g_liquid(Ctx& c, float* const* out, float* const* out2 = nullptr, 
          k_p2g_tile, c.g, (const f3*)c.pos[cur], (const f3*)c.vel[cur], (const float*)c.mass[cur],
          (const int8_t*)c.flag[cur], (const uint32_t*)c.cstart, (const uint32_t*)c.cend, (const uint8_t*)c.cmask,
          c.p2g_parts, ntx, nty, ntz, band, big, (const uint8_t*)(c.bmask + nbricks(c.g)));
-  const int64_t fc[3] = {c.g.FX, c.g.FY, c.g.FZ};
-  const char* nm = band ? "p2g_solid_collect" : "p2g_collect";
-  launch(c, nm, dim3(nblocks(fc[0], 256)), dim3(256), 0, k_p2g_collect<0>, c.g, (const float*)c.p2g_parts, ntx, nty,
-         ntz, out[0], out2 ? out2[0] : (float*)nullptr, fc[0], band, big);
-  launch(c, nm, dim3(nblocks(fc[1], 256)), dim3(256), 0, k_p2g_collect<1>, c.g, (const float*)c.p2g_parts, ntx, nty,
-         ntz, out[1], out2 ? out2[1] : (float*)nullptr, fc[1], band, big);
-  launch(c, nm, dim3(nblocks(fc[2], 256)), dim3(256), 0, k_p2g_collect<2>, c.g, (const float*)c.p2g_parts, ntx, nty,
-         ntz, out[2], out2 ? out2[2] : (float*)nullptr, fc[2], band, big);
+  P2GOut o;
+  for (int a = 0; a < 3; ++a) {
+    o.u[a] = out[a];
+    o.u2[a] = out2 ? out2[a] : nullptr;
+  }
+  launch(c, band ? "p2g_solid_collect" : "p2g_collect", dim3(face_blocks(c.g), 3), dim3(256), 0, k_p2g_collect, c.g,
+         (const float*)c.p2g_parts, ntx, nty, ntz, o, band, big);
 }
 
 static_assert(2 * ST_RTOT >= 12 * ST_CELLS, "the solver's slow-row weights (six FP64 values a cell) fit as well");
@@ -1841,63 +1933,60 @@ void run_solid_phi_and_velocity(Ctx& c) {
   const int64_t G = c.g.G;
   launch(c, "init_solid_phi", dim3(nblocks(G, 256)), dim3(256), 0, k_init_solid_phi, G, (const uint8_t*)c.cmask,
          c.ctmp, (float)(3 * c.g.nx));
-  sweep_n(c, c.phisolid, -1, 3, true);
+  const SweepJob job{c.phisolid, c.ctmp, c.mark, -1, c.sflag};
+  sweep_n(c, &job, 1, 3);
   // solid velocity only where the collision response can read it
   p2g_liquid(c, c.su, nullptr, c.phisolid, (float)(3 * c.g.nx));
 }
 
-static void sweep_phi(Ctx& c, float* phi, int8_t type) {
-  const int64_t G = c.g.G;
-  launch(c, "initphi", dim3(nblocks(G, 256)), dim3(256), 0, k_initphi, G, (const int8_t*)c.mark, c.ctmp, type,
-         (float)(c.g.nx * 3));
-  sweep_n(c, phi, type, 3, true);
-}
-
-// Two passes: u -> scratch, scratch -> u.
-template <int A>
-static void sweep_u_pass(Ctx& c, const float* src, float* dst, const float* phi, int8_t sf, const uint8_t* prev,
-                         uint8_t* cur) {
-  const int64_t nfy = c.g.ny + (A == 1), nfz = c.g.nz + (A == 2);
-  const uint32_t ntj = (uint32_t)((nfy + SW_J - 1) / SW_J), ntk = (uint32_t)((nfz + SW_K - 1) / SW_K);
-  const int64_t nt = face_tiles(c.g, A);
-  // a pass that computes every tile gives each wave SW_U1 tiles (more waves
-  // in flight for its two rounds of loads); a pass that skips reads the
-  // flags of SW_L tiles per wave
-  const int per_wave = prev ? SW_L : SW_U1;
-  const int64_t nwaves = (nt + per_wave - 1) / per_wave;
-  launch(c, "sweep_u", dim3((unsigned)((nwaves + 3) / 4)), dim3(256), 0, k_sweep_u<A>, c.g, src, dst, phi,
-         (const int8_t*)c.mark, sf, prev, cur, ntj, ntk, (uint32_t)nt, per_wave);
-}
-static void sweep_u(Ctx& c, float* const* u, const float* phi, int8_t sf) {
-  // the first pass records per-tile changes (one flag set per axis), the
-  // second skips the tiles they leave unchanged
-  uint8_t* fl[3] = {c.sflag + 2 * sweep_tiles(c.g), nullptr, nullptr};
-  fl[1] = fl[0] + face_tiles(c.g, 0);
-  fl[2] = fl[1] + face_tiles(c.g, 1);
-  for (int it = 0; it < 2; ++it) {
-    float* const* src = it == 0 ? u : c.ftmp;
-    float* const* dst = it == 0 ? c.ftmp : u;
-    const bool first = it == 0;
-    sweep_u_pass<0>(c, src[0], dst[0], phi, sf, first ? nullptr : fl[0], first ? fl[0] : nullptr);
-    sweep_u_pass<1>(c, src[1], dst[1], phi, sf, first ? nullptr : fl[1], first ? fl[1] : nullptr);
-    sweep_u_pass<2>(c, src[2], dst[2], phi, sf, first ? nullptr : fl[2], first ? fl[2] : nullptr);
-  }
-}
-
-static void bc(Ctx& c, float* const* u) {
-  const int64_t fc[3] = {c.g.FX, c.g.FY, c.g.FZ};
-  launch(c, "bc", dim3(nblocks(fc[0], 256)), dim3(256), 0, k_bc<0>, c.g, u[0], (const int8_t*)c.mark, fc[0]);
-  launch(c, "bc", dim3(nblocks(fc[1], 256)), dim3(256), 0, k_bc<1>, c.g, u[1], (const int8_t*)c.mark, fc[1]);
-  launch(c, "bc", dim3(nblocks(fc[2], 256)), dim3(256), 0, k_bc<2>, c.g, u[2], (const int8_t*)c.mark, fc[2]);
-}
+static Faces6 faces6(Ctx& c) { return Faces6{{c.wu[0], c.wu[1], c.wu[2], c.au[0], c.au[1], c.au[2]}}; }
 
 void run_extrapolate_bc(Ctx& c, bool recompute_phi) {
-  if (recompute_phi) sweep_phi(c, c.phiair, AIR);
-  sweep_u(c, c.au, c.phiair, AIR);
-  if (recompute_phi) sweep_phi(c, c.phifluid, FLUID);
-  sweep_u(c, c.wu, c.phifluid, FLUID);
-  bc(c, c.au);
-  bc(c, c.wu);
+  const int64_t G = c.g.G;
+  const int64_t fc[3] = {c.g.FX, c.g.FY, c.g.FZ};
+  if (recompute_phi) {
+    float* tmp2 = c.ftmp[0];
+    launch(c, "initphi", dim3(nblocks(G, 256)), dim3(256), 0, k_initphi, G, (const int8_t*)c.mark, c.ctmp, (int8_t)AIR,
+           tmp2, (int8_t)FLUID, (float)(c.g.nx * 3));
+    const SweepJob jobs[2] = {{c.phiair, c.ctmp, c.mark, AIR, c.sflag},
+                              {c.phifluid, tmp2, c.mark, FLUID, c.sflag + 2 * sweep_tiles(c.g)}};
+    sweep_n(c, jobs, 2, 3);
+  }
+  // Two passes: u -> scratch, scratch -> u; the first records per-tile changes
+  // (a flag set per field), the second skips the tiles they leave unchanged.
+  // The air faces' scratch is the liquid P2G's (12 floats a cell, three face
+  // fields are at most 6).  A pass that computes every tile gives each wave
+  // SW_U1 tiles (more waves in flight for its two rounds of loads); a pass
+  // that skips reads the flags of SW_L tiles per wave.
+  const Faces6 u = faces6(c);
+  SweepU s;
+  float* air = c.p2g_parts;
+  uint8_t* fl = c.sflag + 2 * sweep_tiles(c.g);
+  float* tmp[6];
+  int64_t most = 0;
+  for (int q = 0; q < 6; ++q) {
+    const int a = q % 3;
+    tmp[q] = q < 3 ? c.ftmp[a] : air;
+    if (q >= 3) air += fc[a];
+    s.flags[q] = fl;
+    fl += face_tiles(c.g, a);
+    most = std::max(most, face_tiles(c.g, a));
+  }
+  s.ls[0] = c.phifluid;
+  s.sf[0] = FLUID;
+  s.ls[1] = c.phiair;
+  s.sf[1] = AIR;
+  for (int it = 0; it < 2; ++it) {
+    for (int q = 0; q < 6; ++q) {
+      s.u[q] = it == 0 ? u.u[q] : tmp[q];
+      s.out[q] = it == 0 ? tmp[q] : u.u[q];
+    }
+    const int per_wave = it ? SW_L : SW_U1;
+    const int64_t nwaves = (most + per_wave - 1) / per_wave;
+    launch(c, "sweep_u", dim3((unsigned)((nwaves + 3) / 4), 6), dim3(256), 0,
+           it == 0 ? k_sweep_u<true> : k_sweep_u<false>, c.g, s, (const int8_t*)c.mark, per_wave);
+  }
+  launch(c, "bc", dim3(face_blocks(c.g), 6), dim3(256), 0, k_bc, c.g, u, (const int8_t*)c.mark);
 }
 
 void run_divergence(Ctx& c) {
@@ -1915,27 +2004,15 @@ void run_divergence(Ctx& c) {
 }
 
 template <class R>
-static void subgrad_t(Ctx& c, float* const* u, double inv_rho) {
-  const int64_t fc[3] = {c.g.FX, c.g.FY, c.g.FZ};
-  const int vd = c.cfg.op == MPF_OPERATOR_VARDENS, sc = c.cfg.solid_constraint;
-  const R* p = (const R*)c.press;
-  launch(c, "subgrad", dim3(nblocks(fc[0], 256)), dim3(256), 0, k_subgrad<0, R>, c.g, u[0], p, (const int8_t*)c.mark, vd,
-         inv_rho, sc, fc[0]);
-  launch(c, "subgrad", dim3(nblocks(fc[1], 256)), dim3(256), 0, k_subgrad<1, R>, c.g, u[1], p, (const int8_t*)c.mark, vd,
-         inv_rho, sc, fc[1]);
-  launch(c, "subgrad", dim3(nblocks(fc[2], 256)), dim3(256), 0, k_subgrad<2, R>, c.g, u[2], p, (const int8_t*)c.mark, vd,
-         inv_rho, sc, fc[2]);
+static void subgrad_t(Ctx& c) {
+  launch(c, "subgrad", dim3(face_blocks(c.g), 6), dim3(256), 0, k_subgrad<R>, c.g, faces6(c), (const R*)c.press,
+         (const int8_t*)c.mark, (int)(c.cfg.op == MPF_OPERATOR_VARDENS), 1.0 / (double)c.cfg.rho_liquid,
+         1.0 / (double)c.cfg.rho_air, (int)c.cfg.solid_constraint);
 }
 
 void run_subgrad(Ctx& c) {
-  double il = 1.0 / (double)c.cfg.rho_liquid, ia = 1.0 / (double)c.cfg.rho_air;
-  if (c.cfg.precision == MPF_FP32) {
-    subgrad_t<float>(c, c.wu, il);
-    subgrad_t<float>(c, c.au, ia);
-  } else {
-    subgrad_t<double>(c, c.wu, il);
-    subgrad_t<double>(c, c.au, ia);
-  }
+  if (c.cfg.precision == MPF_FP32) subgrad_t<float>(c);
+  else subgrad_t<double>(c);
 }
 
 void run_heat_grid_pre(Ctx& c) {

@@ -3,6 +3,7 @@
 // (a16, particle half) and phase change with nucleation (a17).
 #include "mpf_internal.h"
 #include "interp.h"
+#include <algorithm>
 
 namespace mpf {
 
@@ -36,10 +37,16 @@ __global__ void k_forces(int64_t P, f3* __restrict__ vel, const int8_t* __restri
   vel[p] = v;
 }
 
-// computeDeltaU, spray_k.cu:997-1006 (old <- new - old), one axis
-__global__ void k_delta_u(int64_t n, const float* __restrict__ u, float* __restrict__ uo) {
-  int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f < n) uo[f] = u[f] - uo[f];
+// computeDeltaU, spray_k.cu:997-1006 (old <- new - old), the six fields
+struct Deltas {
+  const float* u[6];
+  float* uo[6];
+  int64_t n[3];
+};
+__global__ void k_delta_u(Deltas d) {
+  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int q = blockIdx.y;
+  if (f < d.n[q % 3]) d.uo[q][f] = d.u[q][f] - d.uo[q][f];
 }
 
 // mapvelg2p_flip_bubble spray_k.cu:3525-3540 ; blend of advectparticle_RK2
@@ -572,11 +579,10 @@ void run_apply_forces(Ctx& c) {
 }
 
 void run_g2p(Ctx& c) {
-  const int64_t fc[3] = {c.g.FX, c.g.FY, c.g.FZ};
-  for (int a = 0; a < 3; ++a) {
-    launch(c, "delta_u", dim3(nblocks(fc[a], 256)), dim3(256), 0, k_delta_u, fc[a], (const float*)c.wu[a], c.wuo[a]);
-    launch(c, "delta_u", dim3(nblocks(fc[a], 256)), dim3(256), 0, k_delta_u, fc[a], (const float*)c.au[a], c.auo[a]);
-  }
+  Deltas d{{c.wu[0], c.wu[1], c.wu[2], c.au[0], c.au[1], c.au[2]},
+           {c.wuo[0], c.wuo[1], c.wuo[2], c.auo[0], c.auo[1], c.auo[2]},
+           {c.g.FX, c.g.FY, c.g.FZ}};
+  launch(c, "delta_u", dim3(nblocks(std::max(c.g.FX, std::max(c.g.FY, c.g.FZ)), 256), 6), dim3(256), 0, k_delta_u, d);
   Faces3 wdu{{c.wuo[0], c.wuo[1], c.wuo[2]}}, adu{{c.auo[0], c.auo[1], c.auo[2]}};
   Faces3 wu{{c.wu[0], c.wu[1], c.wu[2]}}, au{{c.au[0], c.au[1], c.au[2]}};
   launch(c, "g2p", dim3(nblocks(c.P, 256)), dim3(256), 0, k_g2p, c.g, c.P, (const f3*)c.pos[c.cur], c.vel[c.cur],
