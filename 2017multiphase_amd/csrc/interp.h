@@ -16,22 +16,36 @@ __device__ __forceinline__ int64_t xcd_block() {
   return x * q + (x < r ? x : r) + (b >> 3);
 }
 
-// trilinear, spray_k.cu:111-122
-__device__ __forceinline__ float trilinear(const float* __restrict__ u, float x, float y, float z, int w, int hh,
-                                           int d) {
+// trilinear, spray_k.cu:111-122: base corner and weights, then the value (b:
+// the base corner; si, sj: strides along i and j)
+struct TriPos {
+  int i, j, k;
+  float ix1, ix0, jy1, jy0, kz1, kz0;
+};
+__device__ __forceinline__ TriPos tri_pos(float x, float y, float z, int w, int hh, int d) {
   x = fmaxf(0.0f, fminf(x, (float)w));
   y = fmaxf(0.0f, fminf(y, (float)hh));
   z = fmaxf(0.0f, fminf(z, (float)d));
-  int i = (int)fminf(x, (float)(w - 2));
-  int j = (int)fminf(y, (float)(hh - 2));
-  int k = (int)fminf(z, (float)(d - 2));
+  TriPos t;
+  t.i = (int)fminf(x, (float)(w - 2));
+  t.j = (int)fminf(y, (float)(hh - 2));
+  t.k = (int)fminf(z, (float)(d - 2));
+  t.ix1 = (float)(t.i + 1) - x, t.ix0 = x - (float)t.i;
+  t.jy1 = (float)(t.j + 1) - y, t.jy0 = y - (float)t.j;
+  t.kz1 = (float)(t.k + 1) - z, t.kz0 = z - (float)t.k;
+  return t;
+}
+__device__ __forceinline__ float tri_eval(const float* __restrict__ b, int64_t si, int64_t sj, const TriPos& t) {
+  return t.kz1 * (t.jy1 * (t.ix1 * b[0] + t.ix0 * b[si]) + t.jy0 * (t.ix1 * b[sj] + t.ix0 * b[si + sj])) +
+         t.kz0 * (t.jy1 * (t.ix1 * b[1] + t.ix0 * b[si + 1]) + t.jy0 * (t.ix1 * b[sj + 1] + t.ix0 * b[si + sj + 1]));
+}
+__device__ __forceinline__ float tri_grid(const float* __restrict__ u, const TriPos& t, int hh, int d) {
   const int64_t sj = d, si = (int64_t)hh * d;
-  const float* b = u + i * si + j * sj + k;
-  float ix1 = (float)(i + 1) - x, ix0 = x - (float)i;
-  float jy1 = (float)(j + 1) - y, jy0 = y - (float)j;
-  float kz1 = (float)(k + 1) - z, kz0 = z - (float)k;
-  return kz1 * (jy1 * (ix1 * b[0] + ix0 * b[si]) + jy0 * (ix1 * b[sj] + ix0 * b[si + sj])) +
-         kz0 * (jy1 * (ix1 * b[1] + ix0 * b[si + 1]) + jy0 * (ix1 * b[sj + 1] + ix0 * b[si + sj + 1]));
+  return tri_eval(u + t.i * si + t.j * sj + t.k, si, sj, t);
+}
+__device__ __forceinline__ float trilinear(const float* __restrict__ u, float x, float y, float z, int w, int hh,
+                                           int d) {
+  return tri_grid(u, tri_pos(x, y, z, w, hh, d), hh, d);
 }
 // getParticleVelFromGrid, spray_k.cu:227-240
 __device__ __forceinline__ f3 vel_from_grid(const Grid& g, f3 p, const float* ux, const float* uy, const float* uz) {

@@ -111,3 +111,46 @@ def test_air_window(pkg, dims, odd):
     if odd in ("none", "off the grid"):
         for u, v in zip(*adj):
             assert np.max(np.abs(u - v)) <= 1e-12 * np.max(np.abs(v))
+
+
+@pytest.mark.parametrize("per_cell", [0.4, 9.0])
+@pytest.mark.parametrize("dims", [(4, 4, 5), (13, 17, 23), (8, 16, 8)])
+def test_tile_gather(pkg, dims, per_cell):
+    """G2P, the bubble-side correction and the heat transfer interpolate from
+    tiles staged in LDS with the library's own sort, from memory with given
+    lists: the same bits, for tiles with many and with few particles and for
+    particles off the grid."""
+    say("tile gather", dims, per_cell)
+    nx, ny, nz = dims
+    rng = np.random.default_rng([nx, ny, nz, int(10 * per_cell)])
+    n = int(nx * ny * nz * per_cell)
+    for alpha in (1.0, 0.95):
+        cfg = pkg.default_config(nx, ny, nz, particle_capacity=n, flip_alpha=alpha, heat_enabled=1, gas_enabled=0,
+                                 mc_enabled=0)
+        h = float(cfg.dx)
+        pos = (rng.uniform(0.0, 1.0, (n, 3)) * np.array(dims) * h).astype(np.float32)
+        pos[::37] += np.float32(0.6 * nx * h)
+        flag = rng.choice([pkg.TYPEFLUID, pkg.TYPESOLID, pkg.TYPEAIR, pkg.TYPEAIRSOLO], n, p=[0.6, 0.1, 0.25, 0.05])
+        own = pkg.Simulator(cfg)
+        own.set_particles(n, pos=pos, flag=flag.astype(np.int8), vel=rng.standard_normal((n, 3)).astype(np.float32),
+                          mass=np.ones(n, np.float32), T=rng.uniform(250.0, 400.0, n).astype(np.float32))
+        own.hash_sort()
+        own.levelset_update()
+        given = pkg.Simulator(cfg)
+        given.set_particles(n, **own.get_particles())
+        for nm in ("CELL_START", "CELL_END"):
+            given.set_field(nm, own.get_field(nm))
+        given.levelset_update()
+        fields = [f + s for f in FACE for s in ("", "_OLD")]
+        values = {f: rng.standard_normal(own.get_field(f).shape).astype(np.float32) for f in fields}
+        before = own.get_particles()
+        for sim in (own, given):
+            for f, v in values.items():
+                sim.set_field(f, v)
+            sim.g2p()
+            sim.heat()
+            sim.correct_bubble_positions()
+        a, b = own.get_particles(), given.get_particles()
+        for f in ("vel", "T", "lheat", "pos"):
+            assert np.array_equal(a[f].view(np.uint32), b[f].view(np.uint32)), f
+        assert np.any(a["vel"] != before["vel"]) and np.any(a["T"] != before["T"])
