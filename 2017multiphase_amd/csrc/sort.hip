@@ -59,22 +59,37 @@ __device__ __forceinline__ void wave_runs(bool act, uint32_t k, bool& head, int&
 }
 
 // rank: the particle's place among its cell's, in the order the atomics came.
-__global__ void k_hash_count(Grid g, const f3* __restrict__ pos, int64_t P, uint32_t* __restrict__ key,
-                             uint32_t* __restrict__ rank, uint32_t* __restrict__ count) {
-  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  bool act = p < P;
-  uint32_t k = 0xffffffffu;
-  if (act) {
-    k = hash_key(g, pos[p]);
-    key[p] = k;
+// HC waves' worth of particles per wave, their loads and then their atomics
+// in flight together.
+constexpr int HC = 4;
+__global__ void __launch_bounds__(256) k_hash_count(Grid g, const f3* __restrict__ pos, int64_t P,
+                                                    uint32_t* __restrict__ key, uint32_t* __restrict__ rank,
+                                                    uint32_t* __restrict__ count) {
+  const int64_t p0 = (int64_t)blockIdx.x * (256 * HC) + threadIdx.x;
+  uint32_t k[HC], base[HC];
+  int headlane[HC];
+  f3 x[HC];
+#pragma unroll
+  for (int u = 0; u < HC; ++u) x[u] = pos[min(p0 + u * 256, P - 1)];
+#pragma unroll
+  for (int u = 0; u < HC; ++u) {
+    const bool act = p0 + u * 256 < P;
+    k[u] = act ? hash_key(g, x[u]) : 0xffffffffu;
+    bool head;
+    int runlen;
+    wave_runs(act, k[u], head, runlen, headlane[u]);
+    base[u] = 0;
+    if (head) base[u] = atomicAdd(&count[k[u]], (uint32_t)runlen);
   }
-  bool head;
-  int runlen, headlane;
-  wave_runs(act, k, head, runlen, headlane);
-  uint32_t base = 0;
-  if (head) base = atomicAdd(&count[k], (uint32_t)runlen);
-  base = __shfl(base, headlane);
-  if (act) rank[p] = base + (uint32_t)(lane_id() - headlane);
+#pragma unroll
+  for (int u = 0; u < HC; ++u) {
+    const int64_t p = p0 + u * 256;
+    const uint32_t first = __shfl(base[u], headlane[u]);
+    if (p < P) {
+      key[p] = k[u];
+      rank[p] = first + (uint32_t)(lane_id() - headlane[u]);
+    }
+  }
 }
 
 // Every particle's cell has a start, so no atomics here.
@@ -434,7 +449,7 @@ void run_hash_sort(Ctx& c) {
   }
   uint32_t* rank = (uint32_t*)c.temp[nxt];  // the reorder's output, free until then
   hipMemsetAsync(c.count, 0, (size_t)G * 4, c.stream);
-  launch(c, "hash_count", dim3(nblocks(P, 256)), dim3(256), 0, k_hash_count, c.g, (const f3*)c.pos[cur], P,
+  launch(c, "hash_count", dim3(nblocks(P, 256 * HC)), dim3(256), 0, k_hash_count, c.g, (const f3*)c.pos[cur], P,
          c.key, rank, c.count);
   scan<SCAN_CELLS>(c, c.count, c.cstart, c.cend, G, false);
   launch(c, "scatter", dim3(nblocks(P, 256)), dim3(256), 0, k_scatter, P, (const uint32_t*)c.key,
@@ -463,7 +478,7 @@ void run_hash_sort_mc(Ctx& c) {
   const int cur = c.cur, nxt = 1 - c.cur;
   uint32_t* rank = (uint32_t*)c.temp[nxt];
   hipMemsetAsync(c.mc_count, 0, (size_t)G2 * 4, c.stream);
-  launch(c, "mc_hash_count", dim3(nblocks(P, 256)), dim3(256), 0, k_hash_count, c.g2, (const f3*)c.pos[cur], P,
+  launch(c, "mc_hash_count", dim3(nblocks(P, 256 * HC)), dim3(256), 0, k_hash_count, c.g2, (const f3*)c.pos[cur], P,
          c.key, rank, c.mc_count);
   scan<SCAN_CELLS>(c, c.mc_count, c.mc_cstart, c.mc_cend, G2, false);
   launch(c, "mc_scatter", dim3(nblocks(P, 256)), dim3(256), 0, k_scatter, P, (const uint32_t*)c.key,
