@@ -107,31 +107,50 @@ __global__ void k_scatter(int64_t P, const uint32_t* __restrict__ key, const uin
 // Keyless variants for mpf_hash_sort_noalloc: the count goes straight into
 // the caller's cell_end, and the scatter recomputes each key from the
 // position (no per-particle key array).
-__global__ void k_hash_count_nokey(Grid g, const f3* __restrict__ pos, int64_t P, uint32_t* __restrict__ count) {
-  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  bool act = p < P;
-  uint32_t k = act ? hash_key(g, pos[p]) : 0xffffffffu;
-  bool head;
-  int runlen, headlane;
-  wave_runs(act, k, head, runlen, headlane);
-  if (head) atomicAdd(&count[k], (uint32_t)runlen);
+__global__ void __launch_bounds__(256) k_hash_count_nokey(Grid g, const f3* __restrict__ pos, int64_t P,
+                                                          uint32_t* __restrict__ count) {
+  const int64_t p0 = (int64_t)blockIdx.x * (256 * HC) + threadIdx.x;
+  f3 x[HC];
+#pragma unroll
+  for (int u = 0; u < HC; ++u) x[u] = pos[min(p0 + u * 256, P - 1)];
+#pragma unroll
+  for (int u = 0; u < HC; ++u) {
+    const bool act = p0 + u * 256 < P;
+    const uint32_t k = act ? hash_key(g, x[u]) : 0xffffffffu;
+    bool head;
+    int runlen, headlane;
+    wave_runs(act, k, head, runlen, headlane);
+    if (head) atomicAdd(&count[k], (uint32_t)runlen);
+  }
 }
 
-__global__ void k_scatter_rehash(Grid g, const f3* __restrict__ pos, int64_t P, uint32_t* __restrict__ cursor,
-                                 uint32_t* __restrict__ perm, uint32_t* __restrict__ skey) {
-  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  bool act = p < P;
-  uint32_t k = act ? hash_key(g, pos[p]) : 0xffffffffu;
-  bool head;
-  int runlen, headlane;
-  wave_runs(act, k, head, runlen, headlane);
-  uint32_t base = 0;
-  if (head) base = atomicAdd(&cursor[k], (uint32_t)runlen);
-  base = __shfl(base, headlane);
-  if (act) {
-    uint32_t slot = base + (uint32_t)(lane_id() - headlane);
-    perm[slot] = (uint32_t)p;
-    skey[slot] = k;
+__global__ void __launch_bounds__(256) k_scatter_rehash(Grid g, const f3* __restrict__ pos, int64_t P,
+                                                        uint32_t* __restrict__ cursor, uint32_t* __restrict__ perm,
+                                                        uint32_t* __restrict__ skey) {
+  const int64_t p0 = (int64_t)blockIdx.x * (256 * HC) + threadIdx.x;
+  f3 x[HC];
+  uint32_t k[HC], base[HC];
+  int headlane[HC];
+#pragma unroll
+  for (int u = 0; u < HC; ++u) x[u] = pos[min(p0 + u * 256, P - 1)];
+#pragma unroll
+  for (int u = 0; u < HC; ++u) {
+    const bool act = p0 + u * 256 < P;
+    k[u] = act ? hash_key(g, x[u]) : 0xffffffffu;
+    bool head;
+    int runlen;
+    wave_runs(act, k[u], head, runlen, headlane[u]);
+    base[u] = 0;
+    if (head) base[u] = atomicAdd(&cursor[k[u]], (uint32_t)runlen);
+  }
+#pragma unroll
+  for (int u = 0; u < HC; ++u) {
+    const uint32_t first = __shfl(base[u], headlane[u]);
+    if (p0 + u * 256 < P) {
+      const uint32_t slot = first + (uint32_t)(lane_id() - headlane[u]);
+      perm[slot] = (uint32_t)(p0 + u * 256);
+      skey[slot] = k[u];
+    }
   }
 }
 
@@ -572,14 +591,14 @@ extern "C" mpf_status mpf_hash_sort_noalloc(const mpf_config* cfg, int64_t n, co
     const int64_t nb = (G + SCAN_TILE - 1) / SCAN_TILE;
     // counts in cell_end (cleared by a kernel, not a memset: graph-capture safe)
     hipLaunchKernelGGL(k_fill_u32, dim3(nblocks(G, 256)), dim3(256), 0, st, G, cell_end, 0u);
-    hipLaunchKernelGGL(k_hash_count_nokey, dim3(nblocks(n, 256)), dim3(256), 0, st, g, p3, n, cell_end);
+    hipLaunchKernelGGL(k_hash_count_nokey, dim3(nblocks(n, 256 * HC)), dim3(256), 0, st, g, p3, n, cell_end);
     hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SCAN_THREADS), 0, st, (const uint32_t*)cell_end, G,
                        blk);
     const bool own = nb <= SCAN_OWN_TILES;
     if (!own) hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(SCAN_THREADS), 0, st, blk, nb);
     hipLaunchKernelGGL(k_scan_apply<SCAN_CURSORS>, dim3((unsigned)nb), dim3(SCAN_THREADS), 0, st,
                        (const uint32_t*)cell_end, G, blk, own, cell_start, cell_end);
-    hipLaunchKernelGGL(k_scatter_rehash, dim3(nblocks(n, 256)), dim3(256), 0, st, g, p3, n, cell_end, grid_index,
+    hipLaunchKernelGGL(k_scatter_rehash, dim3(nblocks(n, 256 * HC)), dim3(256), 0, st, g, p3, n, cell_end, grid_index,
                        grid_hash);
     hipLaunchKernelGGL(k_segsort, dim3(nblocks(G, 256)), dim3(256), 0, st, G, (const uint32_t*)cell_start,
                        (const uint32_t*)cell_end, grid_index);
