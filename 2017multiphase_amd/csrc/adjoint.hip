@@ -484,12 +484,6 @@ __global__ void __launch_bounds__(GT)
   }
 }
 
-// g_uold = -alpha g_u
-__global__ void k_adj_uold(int64_t n, const double* __restrict__ gu, double alpha, double* __restrict__ guo) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) guo[i] = 0.0 - alpha * gu[i];
-}
-
 // ---------------- advection ----------------
 // Forward (CollisionWithSolid_k, spray_k.cu:5276-5345, away from solids):
 //   x' = clamp(x + v dt), v' = v with clamped components zeroed; SOLID fixed.
@@ -587,11 +581,13 @@ struct SweepRules {
   float* w[3];
   uint8_t* code;
 };
+struct SweepRules3 {
+  SweepRules a[3];  // by axis
+};
 template <int A>
-__global__ void k_adj_sweep_rules(Grid g, const float* __restrict__ ls, const int8_t* __restrict__ mark, int8_t sf,
-                                  SweepRules r, int64_t nf) {
-  int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nf) return;
+__device__ __forceinline__ void adj_sweep_rules_face(const Grid& g, const float* __restrict__ ls,
+                                                     const int8_t* __restrict__ mark, int8_t sf, const SweepRules& r,
+                                                     int64_t f) {
   int i, j, k;
   ijk_face<A>(g, f, i, j, k);
   int dsel[3];
@@ -612,10 +608,8 @@ __global__ void k_adj_sweep_rules(Grid g, const float* __restrict__ ls, const in
 // One transposed pass, as a gather: face n collects its identity term and the
 // weights of the (at most 6) faces whose chosen blend reads it.
 template <int A>
-__global__ void k_adj_sweep_u(Grid g, const double* __restrict__ gout, double* __restrict__ gin, SweepRules r,
-                              int64_t nf) {
-  int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nf) return;
+__device__ __forceinline__ void adj_sweep_u_face(const Grid& g, const double* __restrict__ gout,
+                                                 double* __restrict__ gin, const SweepRules& r, int64_t f) {
   int i, j, k;
   ijk_face<A>(g, f, i, j, k);
   const int dims[3] = {g.nx + (A == 0), g.ny + (A == 1), g.nz + (A == 2)};
@@ -668,10 +662,9 @@ __device__ __forceinline__ int bc_rule(const Grid& g, const int8_t* mark, int i,
 // Transposed wall rule.  The ceiling's branch (uz(nz-2) < 0) is read from the
 // forward's output `u_after`: the output is negative exactly when it copied.
 template <int A>
-__global__ void k_adj_bc(Grid g, const double* __restrict__ gout, double* __restrict__ gin,
-                         const int8_t* __restrict__ mark, const float* __restrict__ u_after, int64_t nf) {
-  int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nf) return;
+__device__ __forceinline__ void adj_bc_face(const Grid& g, const double* __restrict__ gout, double* __restrict__ gin,
+                                            const int8_t* __restrict__ mark, const float* __restrict__ u_after,
+                                            int64_t f) {
   int i, j, k;
   ijk_face<A>(g, f, i, j, k);
   const int r = bc_rule<A>(g, mark, i, j, k);
@@ -679,6 +672,52 @@ __global__ void k_adj_bc(Grid g, const double* __restrict__ gout, double* __rest
   if (A == 2 && r == 0 && k + 1 <= g.nz && bc_rule<2>(g, mark, i, j, k + 1) == 2 && u_after[f + 1] < 0.0f)
     acc += gout[f + 1];
   gin[f] = acc;
+}
+
+// Three axes (rules, passes: blockIdx.y = axis) or six fields (3 phase + axis)
+// in one launch.
+struct Grads6 {
+  const double* in[6];
+  double* out[6];
+  const float* u[6];
+};
+__device__ __forceinline__ int64_t face_n(const Grid& g, int A) { return A == 0 ? g.FX : A == 1 ? g.FY : g.FZ; }
+__global__ void k_adj_sweep_rules(Grid g, const float* __restrict__ ls, const int8_t* __restrict__ mark, int8_t sf,
+                                  SweepRules3 r) {
+  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int A = blockIdx.y;
+  if (f >= face_n(g, A)) return;
+  if (A == 0) adj_sweep_rules_face<0>(g, ls, mark, sf, r.a[0], f);
+  else if (A == 1) adj_sweep_rules_face<1>(g, ls, mark, sf, r.a[1], f);
+  else adj_sweep_rules_face<2>(g, ls, mark, sf, r.a[2], f);
+}
+__global__ void k_adj_sweep_u(Grid g, Grads6 gr, int ph, SweepRules3 r) {
+  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int A = blockIdx.y;
+  if (f >= face_n(g, A)) return;
+  const double* src = gr.in[3 * ph + A];
+  double* dst = gr.out[3 * ph + A];
+  if (A == 0) adj_sweep_u_face<0>(g, src, dst, r.a[0], f);
+  else if (A == 1) adj_sweep_u_face<1>(g, src, dst, r.a[1], f);
+  else adj_sweep_u_face<2>(g, src, dst, r.a[2], f);
+}
+__global__ void k_adj_bc(Grid g, Grads6 gr, const int8_t* __restrict__ mark) {
+  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int q = blockIdx.y, A = q % 3;
+  if (f >= face_n(g, A)) return;
+  if (A == 0) adj_bc_face<0>(g, gr.in[q], gr.out[q], mark, gr.u[q], f);
+  else if (A == 1) adj_bc_face<1>(g, gr.in[q], gr.out[q], mark, gr.u[q], f);
+  else adj_bc_face<2>(g, gr.in[q], gr.out[q], mark, gr.u[q], f);
+}
+__global__ void k_zero6(Grid g, Grads6 gr) {
+  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (f < face_n(g, blockIdx.y % 3)) gr.out[blockIdx.y][f] = 0.0;
+}
+// g_uold = -alpha g_u
+__global__ void k_adj_uold(Grid g, Grads6 gr, double alpha) {
+  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int q = blockIdx.y;
+  if (f < face_n(g, q % 3)) gr.out[q][f] = 0.0 - alpha * gr.in[q][f];
 }
 
 __global__ void k_fill_d(int64_t n, double* __restrict__ a, double v) {
@@ -780,43 +819,34 @@ int run_extrapolate_adjoint(Ctx& c, const double* const* gout, double* const* gi
   if (!adj_alloc(c)) return MPF_INVALID_ARG;
   for (int q = 0; q < 6; ++q) copy_in(c, c.adj_fin[q], gout ? gout[q] : nullptr, face_count(c, q), where);
   const int64_t fc[3] = {c.g.FX, c.g.FY, c.g.FZ};
-  // the decisions of one axis at a time, in the P2G's tile buffer (over 12
+  const unsigned nb = nblocks(std::max(fc[0], std::max(fc[1], fc[2])), 256);
+  // the decisions of one phase at a time, in the P2G's tile buffer (over 12
   // floats per cell; they take 13 bytes per face)
-  SweepRules rules;
-  const int64_t fmax_ = std::max(fc[0], std::max(fc[1], fc[2]));
-  for (int d = 0; d < 3; ++d) rules.w[d] = c.p2g_parts + d * fmax_;
-  rules.code = (uint8_t*)(c.p2g_parts + 3 * fmax_);
-  if (3 * fmax_ + (fmax_ + 3) / 4 > p2g_parts_floats(c.g)) {
+  SweepRules3 rules;
+  float* at = c.p2g_parts;
+  for (int A = 0; A < 3; ++A) {
+    for (int d = 0; d < 3; ++d, at += fc[A]) rules.a[A].w[d] = at;
+    rules.a[A].code = (uint8_t*)at;
+    at += (fc[A] + 3) / 4;
+  }
+  if (at - c.p2g_parts > p2g_parts_floats(c.g)) {
     c.err = "extrapolation adjoint: scratch too small";
     return MPF_INVALID_ARG;
   }
+  // wall rule^T: fin -> fout; then two sweep passes^T: fout -> fin -> fout
+  Grads6 to, back;
+  for (int q = 0; q < 6; ++q) {
+    to.in[q] = back.out[q] = c.adj_fin[q];
+    to.out[q] = c.adj_fout[q];
+    back.in[q] = c.adj_fout[q];
+    to.u[q] = back.u[q] = q < 3 ? c.wu[q] : c.au[q - 3];
+  }
+  launch(c, "adj_bc", dim3(nb, 6), dim3(256), 0, k_adj_bc, c.g, to, (const int8_t*)c.mark);
   for (int ph = 0; ph < 2; ++ph) {
-    float* const* u = ph == 0 ? c.wu : c.au;
-    const float* phi = ph == 0 ? c.phifluid : c.phiair;
-    const int8_t sf = ph == 0 ? FLUID : AIR;
-    double* a = nullptr;
-    double* b = nullptr;
-    // wall rule^T: fin -> fout; then two sweep passes^T: fout -> fin -> fout
-    for (int A = 0; A < 3; ++A) {
-      a = c.adj_fin[3 * ph + A];
-      b = c.adj_fout[3 * ph + A];
-      const unsigned nb = nblocks(fc[A], 256);
-      const int8_t* mk = c.mark;
-      if (A == 0) launch(c, "adj_bc", dim3(nb), dim3(256), 0, k_adj_bc<0>, c.g, (const double*)a, b, mk, (const float*)u[0], fc[0]);
-      if (A == 1) launch(c, "adj_bc", dim3(nb), dim3(256), 0, k_adj_bc<1>, c.g, (const double*)a, b, mk, (const float*)u[1], fc[1]);
-      if (A == 2) launch(c, "adj_bc", dim3(nb), dim3(256), 0, k_adj_bc<2>, c.g, (const double*)a, b, mk, (const float*)u[2], fc[2]);
-      const char* rn = "adj_sweep_rules";
-      if (A == 0) launch(c, rn, dim3(nb), dim3(256), 0, k_adj_sweep_rules<0>, c.g, phi, mk, sf, rules, fc[0]);
-      if (A == 1) launch(c, rn, dim3(nb), dim3(256), 0, k_adj_sweep_rules<1>, c.g, phi, mk, sf, rules, fc[1]);
-      if (A == 2) launch(c, rn, dim3(nb), dim3(256), 0, k_adj_sweep_rules<2>, c.g, phi, mk, sf, rules, fc[2]);
-      for (int pass = 0; pass < 2; ++pass) {
-        const double* src = pass == 0 ? b : a;
-        double* dst = pass == 0 ? a : b;
-        if (A == 0) launch(c, "adj_sweep_u", dim3(nb), dim3(256), 0, k_adj_sweep_u<0>, c.g, src, dst, rules, fc[0]);
-        if (A == 1) launch(c, "adj_sweep_u", dim3(nb), dim3(256), 0, k_adj_sweep_u<1>, c.g, src, dst, rules, fc[1]);
-        if (A == 2) launch(c, "adj_sweep_u", dim3(nb), dim3(256), 0, k_adj_sweep_u<2>, c.g, src, dst, rules, fc[2]);
-      }
-    }
+    launch(c, "adj_sweep_rules", dim3(nb, 3), dim3(256), 0, k_adj_sweep_rules, c.g,
+           (const float*)(ph == 0 ? c.phifluid : c.phiair), (const int8_t*)c.mark, (int8_t)(ph == 0 ? FLUID : AIR), rules);
+    launch(c, "adj_sweep_u", dim3(nb, 3), dim3(256), 0, k_adj_sweep_u, c.g, back, ph, rules);
+    launch(c, "adj_sweep_u", dim3(nb, 3), dim3(256), 0, k_adj_sweep_u, c.g, to, ph, rules);
   }
   for (int q = 0; q < 6; ++q) copy_out(c, gin[q], c.adj_fout[q], face_count(c, q), where);
   return hip_ok(c, hipStreamSynchronize(c.stream), "extrapolate_adjoint") ? MPF_OK : MPF_HIP_ERROR;
@@ -872,7 +902,13 @@ int run_g2p_adjoint(Ctx& c, const double* gvel_out, double* gvel_in, double* con
   const int cur = c.cur;
   const int64_t P = c.P;
   copy_in(c, c.adj_part[0], gvel_out, 3 * P, where);
-  for (int q = 0; q < 6; ++q) zero(c, c.adj_fin[q], face_count(c, q));
+  Grads6 gr;
+  for (int q = 0; q < 6; ++q) {
+    gr.in[q] = gr.out[q] = c.adj_fin[q];
+    gr.u[q] = nullptr;
+  }
+  const unsigned nb6 = nblocks(std::max(c.g.FX, std::max(c.g.FY, c.g.FZ)), 256);
+  launch(c, "adj_fill", dim3(nb6, 6), dim3(256), 0, k_zero6, c.g, gr);
   G2PArgs a;
   for (int A = 0; A < 3; ++A) {
     a.u[A] = c.wu[A];
@@ -893,11 +929,10 @@ int run_g2p_adjoint(Ctx& c, const double* gvel_out, double* gvel_in, double* con
     launch(c, "adj_g2p", dim3(nblocks(P, 256)), dim3(256), 0, k_adj_g2p, c.g, P, (const f3*)c.pos[cur],
            (const int8_t*)c.flag[cur], a, alpha, (const double*)c.adj_part[0], c.adj_part[1], c.adj_part[2]);
   }
-  if (guo)
-    for (int q = 0; q < 6; ++q)
-      if (guo[q])
-        launch(c, "adj_uold", dim3(nblocks(face_count(c, q), 256)), dim3(256), 0, k_adj_uold, face_count(c, q),
-               (const double*)c.adj_fin[q], alpha, c.adj_fout[q]);
+  if (guo) {
+    for (int q = 0; q < 6; ++q) gr.out[q] = c.adj_fout[q];
+    launch(c, "adj_uold", dim3(nb6, 6), dim3(256), 0, k_adj_uold, c.g, gr, alpha);
+  }
   copy_out(c, gvel_in, c.adj_part[1], 3 * P, where);
   copy_out(c, gpos, c.adj_part[2], 3 * P, where);
   for (int q = 0; q < 6; ++q) {
