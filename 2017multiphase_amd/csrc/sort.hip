@@ -10,10 +10,12 @@
 //
 // Counting sort instead of a comparison/radix sort, since keys are cell ids:
 //  1. hash + count: one atomic per run of equal keys in a wavefront (input is
-//     nearly sorted from the previous step, so runs are long);
-//  2. exclusive scan of the per-cell counts (reduce-then-scan, LDS tiles);
-//  3. scatter: one atomic per run reserves slots, lanes of a run take
-//     consecutive slots in index order;
+//     nearly sorted from the previous step, so runs are long), whose value
+//     ranks the run's particles in their cell;
+//  2. exclusive scan of the per-cell counts (reduce-then-scan, LDS tiles),
+//     written as the cells' lists;
+//  3. scatter: cell start plus rank (without a context, which has no room for
+//     the ranks: one more atomic per run);
 //  4. per-cell segment sort of the permutation (runs from different waves can
 //     interleave within a cell): a register sorting network for <=16 entries;
 //  5. gather of the 45-byte particle record into the other buffer.
@@ -60,8 +62,9 @@ __device__ __forceinline__ void wave_runs(bool act, uint32_t k, bool& head, int&
 
 // rank: the particle's place among its cell's, in the order the atomics came.
 // HC waves' worth of particles per wave, their loads and then their atomics
-// in flight together.
-constexpr int HC = 4;
+// in flight together: four for many particles, one where that would leave the
+// chip with few waves (HC_MANY).
+template <int HC>
 __global__ void __launch_bounds__(256) k_hash_count(Grid g, const f3* __restrict__ pos, int64_t P,
                                                     uint32_t* __restrict__ key, uint32_t* __restrict__ rank,
                                                     uint32_t* __restrict__ count) {
@@ -107,6 +110,7 @@ __global__ void k_scatter(int64_t P, const uint32_t* __restrict__ key, const uin
 // Keyless variants for mpf_hash_sort_noalloc: the count goes straight into
 // the caller's cell_end, and the scatter recomputes each key from the
 // position (no per-particle key array).
+template <int HC>
 __global__ void __launch_bounds__(256) k_hash_count_nokey(Grid g, const f3* __restrict__ pos, int64_t P,
                                                           uint32_t* __restrict__ count) {
   const int64_t p0 = (int64_t)blockIdx.x * (256 * HC) + threadIdx.x;
@@ -124,6 +128,7 @@ __global__ void __launch_bounds__(256) k_hash_count_nokey(Grid g, const f3* __re
   }
 }
 
+template <int HC>
 __global__ void __launch_bounds__(256) k_scatter_rehash(Grid g, const f3* __restrict__ pos, int64_t P,
                                                         uint32_t* __restrict__ cursor, uint32_t* __restrict__ perm,
                                                         uint32_t* __restrict__ skey) {
@@ -338,6 +343,10 @@ __global__ void k_scan_blocks(uint32_t* blk, int64_t nb) {
   if (threadIdx.x == 0) blk[nb] = carry;
 }
 
+// 23.0 us with one against 25.2 with four at 200k particles, 44.3 and 44.5 at
+// 1.2M, 75.2 and 74.7 at 2.9M, 988 and 895 at 45M (the sort without a context).
+constexpr int64_t HC_MANY = 2500000;
+
 // The exclusive scan of in, tile by tile.  blk: the tiles' exclusive prefixes
 // (own = false), or their sums, of which each block adds up those before it
 // (own = true: one launch less; the last block then leaves the total at
@@ -466,10 +475,11 @@ void run_hash_sort(Ctx& c) {
     run_cell_mask(c);
     return;
   }
+  const bool many = P >= HC_MANY;
   uint32_t* rank = (uint32_t*)c.temp[nxt];  // the reorder's output, free until then
   hipMemsetAsync(c.count, 0, (size_t)G * 4, c.stream);
-  launch(c, "hash_count", dim3(nblocks(P, 256 * HC)), dim3(256), 0, k_hash_count, c.g, (const f3*)c.pos[cur], P,
-         c.key, rank, c.count);
+  launch(c, "hash_count", dim3(nblocks(P, many ? 1024 : 256)), dim3(256), 0,
+         many ? k_hash_count<4> : k_hash_count<1>, c.g, (const f3*)c.pos[cur], P, c.key, rank, c.count);
   scan<SCAN_CELLS>(c, c.count, c.cstart, c.cend, G, false);
   launch(c, "scatter", dim3(nblocks(P, 256)), dim3(256), 0, k_scatter, P, (const uint32_t*)c.key,
          (const uint32_t*)rank, (const uint32_t*)c.cstart, c.perm, c.ghash);
@@ -495,10 +505,11 @@ void run_hash_sort(Ctx& c) {
 void run_hash_sort_mc(Ctx& c) {
   const int64_t P = c.P, G2 = c.g2.G;
   const int cur = c.cur, nxt = 1 - c.cur;
+  const bool many = P >= HC_MANY;
   uint32_t* rank = (uint32_t*)c.temp[nxt];
   hipMemsetAsync(c.mc_count, 0, (size_t)G2 * 4, c.stream);
-  launch(c, "mc_hash_count", dim3(nblocks(P, 256 * HC)), dim3(256), 0, k_hash_count, c.g2, (const f3*)c.pos[cur], P,
-         c.key, rank, c.mc_count);
+  launch(c, "mc_hash_count", dim3(nblocks(P, many ? 1024 : 256)), dim3(256), 0,
+         many ? k_hash_count<4> : k_hash_count<1>, c.g2, (const f3*)c.pos[cur], P, c.key, rank, c.mc_count);
   scan<SCAN_CELLS>(c, c.mc_count, c.mc_cstart, c.mc_cend, G2, false);
   launch(c, "mc_scatter", dim3(nblocks(P, 256)), dim3(256), 0, k_scatter, P, (const uint32_t*)c.key,
          (const uint32_t*)rank, (const uint32_t*)c.mc_cstart, c.perm, c.ghash);
@@ -589,17 +600,19 @@ extern "C" mpf_status mpf_hash_sort_noalloc(const mpf_config* cfg, int64_t n, co
     hipLaunchKernelGGL(k_fill_u32, dim3(nblocks(G, 256)), dim3(256), 0, st, G, cell_end, MPF_CELL_UNDEF);
   } else {
     const int64_t nb = (G + SCAN_TILE - 1) / SCAN_TILE;
+    const bool many = n >= HC_MANY;
     // counts in cell_end (cleared by a kernel, not a memset: graph-capture safe)
     hipLaunchKernelGGL(k_fill_u32, dim3(nblocks(G, 256)), dim3(256), 0, st, G, cell_end, 0u);
-    hipLaunchKernelGGL(k_hash_count_nokey, dim3(nblocks(n, 256 * HC)), dim3(256), 0, st, g, p3, n, cell_end);
+    hipLaunchKernelGGL(many ? k_hash_count_nokey<4> : k_hash_count_nokey<1>, dim3(nblocks(n, many ? 1024 : 256)),
+                       dim3(256), 0, st, g, p3, n, cell_end);
     hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SCAN_THREADS), 0, st, (const uint32_t*)cell_end, G,
                        blk);
     const bool own = nb <= SCAN_OWN_TILES;
     if (!own) hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(SCAN_THREADS), 0, st, blk, nb);
     hipLaunchKernelGGL(k_scan_apply<SCAN_CURSORS>, dim3((unsigned)nb), dim3(SCAN_THREADS), 0, st,
                        (const uint32_t*)cell_end, G, blk, own, cell_start, cell_end);
-    hipLaunchKernelGGL(k_scatter_rehash, dim3(nblocks(n, 256 * HC)), dim3(256), 0, st, g, p3, n, cell_end, grid_index,
-                       grid_hash);
+    hipLaunchKernelGGL(many ? k_scatter_rehash<4> : k_scatter_rehash<1>, dim3(nblocks(n, many ? 1024 : 256)),
+                       dim3(256), 0, st, g, p3, n, cell_end, grid_index, grid_hash);
     hipLaunchKernelGGL(k_segsort, dim3(nblocks(G, 256)), dim3(256), 0, st, G, (const uint32_t*)cell_start,
                        (const uint32_t*)cell_end, grid_index);
   }
