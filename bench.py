@@ -59,18 +59,18 @@ KERNEL_BYTES = {
     "genlevelset": (17, 0, 13),
     # one launch, 3 axes: start/end 8, mask 1, 3 faces 12 written; pos 12, vel 12, mass 4, flag 1
     "p2g_liquid": (21, 0, 29),
-    # one launch per axis: start/end 8, mask 1, face 4 written; particles as above
-    "p2g_air": (13, 0, 29),
+    # one launch, 3 axes: start/end 8, phase bits, 3 faces 12 written; particles as above
+    "p2g_air": (20.25, 0, 29),
     # start/end 8, mask 1, T 4 written; pos 12, T 4, flag 1
     "heat_p2g": (13, 0, 17),
     # 45-byte record read and written + perm 4
     "reorder": (0, 0, 94),
     # position and flag read, position written (neighbours from cache)
     "correct_pos": (0, 0, 25),
-    # level-set sweep: ls 4 read, mark 1, ls 4 written
-    "sweep": (9, 0, 0),
-    # extrapolation pass per face: u 4, out 4, ls 2x4, mark 2
-    "sweep_u": (18, 0, 0),
+    # sweep of two fields: each 4 read, mark 1, 4 written
+    "sweep": (18, 0, 0),
+    # extrapolation pass of six face fields: each u 4, out 4, ls 2x4, mark 2
+    "sweep_u": (108, 0, 0),
 }
 FP64_VEC = {"pcg_spmv": (1, 32, 0), "pcg_update": (1, 40, 0)}
 
