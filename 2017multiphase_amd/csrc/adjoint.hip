@@ -136,6 +136,10 @@ __global__ void k_adj_divT(Grid g, const int8_t* __restrict__ mark, const float*
 // The air window's rows are dealt to AIR_LANES lanes per face: few faces have
 // air near them, and one lane's walk over 25 rows is a chain of loads.
 constexpr int AIR_LANES = 8;
+// Marks a face without weight, or whose weight is not a number, in place of
+// g_u / W: a NaN whose payload arithmetic does not make.  Such a face passes
+// nothing on, whatever a particle beside it holds.
+constexpr long long NO_WEIGHT = 0x7ff8a5c3f00d1e2dll;
 // W_f and u_f recomputed in FP64 (face gather with the forward's windows, one
 // launch for the three axes).  Bound by FP64 arithmetic: about 30 operations
 // at half rate, a division among them, for each of a face's 144 particles.
@@ -146,7 +150,7 @@ constexpr int AIR_LANES = 8;
 // bits, the 36 cells within the radius) now.
 struct FaceOut {
   const double* gu[3];
-  double* B[3];  // g_u / W (0 without weight)
+  double* B[3];  // g_u / W (NO_WEIGHT without weight)
   double* U[3];
 };
 template <int A, bool AIRPH, bool ROWS>
@@ -165,7 +169,7 @@ __device__ __forceinline__ void adj_p2g_face(const Grid& g, const f3* __restrict
     const int64_t b = ((int64_t)(min(i, g.nx - 1) >> 2) * by + (min(j, g.ny - 1) >> 2)) * bz + (min(k, g.nz - 1) >> 2);
     if (!(dm[b] & need)) {  // the same for all lanes of a face
       if (sub == 0) {
-        Bout[f] = 0.0;
+        Bout[f] = __longlong_as_double(NO_WEIGHT);
         Uout[f] = 0.0;
       }
       return;
@@ -257,7 +261,7 @@ __device__ __forceinline__ void adj_p2g_face(const Grid& g, const f3* __restrict
     }
   }
   if (sub == 0) {
-    Bout[f] = (W > 0) ? gu[f] / W : 0.0;
+    Bout[f] = (W > 0) ? gu[f] / W : __longlong_as_double(NO_WEIGHT);
     Uout[f] = (W > 0) ? U / W : 0.0;
   }
 }
@@ -284,7 +288,7 @@ struct P2GFaceData {
 // The liquid launch writes every particle (0 off its phase), the air launch
 // adds.  Bound by FP64 arithmetic and the gathers: with g_u / W formed once per
 // face and one reciprocal of r^2 a pair takes one division where it took four
-// (0.60 -> 0.42 ms at 96^3, liquid; 0.23 -> 0.09 air).
+// (0.60 -> 0.40 ms at 96^3, liquid; 0.23 -> 0.11 air).
 template <bool AIRPH>
 __global__ void k_adj_p2g_part(Grid g, int64_t P, const f3* __restrict__ pos, const f3* __restrict__ vel,
                                const float* __restrict__ mass, const int8_t* __restrict__ flag, P2GFaceData fd,
@@ -320,7 +324,7 @@ __global__ void k_adj_p2g_part(Grid g, int64_t P, const f3* __restrict__ pos, co
           const int fi = ci - oi, fj = cj - oj, fk = ck - ok;
           if (fi < 0 || fj < 0 || fk < 0 || fi >= dims[0] || fj >= dims[1] || fk >= dims[2]) continue;
           const int64_t f = fid(g, A, fi, fj, fk);
-          const double B = fd.B[A][f], U = fd.U[A][f];  // both 0 on a face without weight
+          const double B = fd.B[A][f], U = fd.U[A][f];
           const double gxf = (double)fi + (A == 0 ? 0.0 : 0.5), gyf = (double)fj + (A == 1 ? 0.0 : 0.5),
                        gzf = (double)fk + (A == 2 ? 0.0 : 0.5);
           const double dx = X - gxf, dy = Y - gyf, dz = Z - gzf;
@@ -328,7 +332,7 @@ __global__ void k_adj_p2g_part(Grid g, int64_t P, const f3* __restrict__ pos, co
           if (r2 >= RE2) continue;
           const double ir2 = 1.0 / fmax(r2, (double)0.0001f);
           const double s = RE2 * ir2 - 1.0;
-          if (!(s > 0)) continue;
+          if (!(s > 0) || __double_as_longlong(B) == NO_WEIGHT) continue;
           av[A] += (m * s) * B;
           if (r2 > (double)0.0001f) {
             // dw/dx_d = -2 m RE^2 d_d / r^4 * scale
