@@ -334,6 +334,38 @@ __device__ __forceinline__ void read_partials(const double* __restrict__ P, int 
   block_sum_all<N, NT>(out);
 }
 
+// The same for N sums of each of two arrays together (a in out[0, N), b in
+// out[N, 2 N)), in one trip through memory: the loads of each thread's first
+// two blocks of both are in flight before the first is added.
+template <int N, int NT = PB>
+__device__ __forceinline__ void read_partials_of_two(const double* __restrict__ a, int na, const double* __restrict__ b,
+                                                     int nb, double (&out)[2 * N]) {
+  double v[2][2][N];  // array, turn
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      const int64_t t = (int)threadIdx.x + s * NT;
+      v[0][s][q] = a[(t < na ? t : 0) * N + q];
+      v[1][s][q] = b[(t < nb ? t : 0) * N + q];
+    }
+#pragma unroll
+  for (int w = 0; w < 2; ++w)
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      out[w * N + q] = 0.0;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) out[w * N + q] += ((int)threadIdx.x + s * NT < (w ? nb : na)) ? v[w][s][q] : 0.0;
+    }
+  for (int t = threadIdx.x + 2 * NT; t < na || t < nb; t += NT)
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      if (t < na) out[q] += a[(int64_t)t * N + q];
+      if (t < nb) out[N + q] += b[(int64_t)t * N + q];
+    }
+  block_sum_all<2 * N, NT>(out);
+}
+
 // Zeros for the (r.z, r.r) partials of blocks [nblk, npad) of a U slot, so
 // that kernels launched with fewer blocks than npad leave npad summands.
 template <int NT = PB>
@@ -601,10 +633,8 @@ __global__ void __launch_bounds__(ST, (sizeof(V) == 4 && !SLOW) ? 6 : 4) k_spmv(
   if (sc->done) return;
   __shared__ V dtab[8];  // 1/diag of the fast rows by open-face count (ordered by read_partials' barriers)
   if (threadIdx.x < 8) dtab[threadIdx.x] = (threadIdx.x < 7) ? dinv_tab<V>(o, threadIdx.x) : V(1);
-  double cur[2], prv[2];
-  read_partials<2, ST>(uslot(P, k - 1), nbu, cur);
-  if (k > 0) read_partials<2, ST>(uslot(P, k), nbu, prv);
-  else prv[0] = prv[1] = 0.0;
+  double cur[4];  // (r.z, r.r) of update(k-1), then of update(k-2)
+  read_partials_of_two<2, ST>(uslot(P, k - 1), nbu, uslot(P, k), k > 0 ? nbu : 0, cur);
   const double bb = (k == 0) ? cur[1] : sc->bb;
   const bool nonfin = bad(cur[0]) || bad(cur[1]);
   const bool conv = ref ? (cur[1] < eps_abs) : (cur[1] == 0.0 || sqrt(cur[1]) <= tol * sqrt(bb));
@@ -620,7 +650,7 @@ __global__ void __launch_bounds__(ST, (sizeof(V) == 4 && !SLOW) ? 6 : 4) k_spmv(
     }
     return;
   }
-  const V be = (k == 0) ? V(0) : (V)(cur[0] / prv[0]);
+  const V be = (k == 0) ? V(0) : (V)(cur[0] / cur[2]);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     sc->rz = cur[0];
     sc->rr = cur[1];
@@ -832,15 +862,47 @@ __global__ void __launch_bounds__(PB) k_slow_q(OpArgs o, const uint32_t* __restr
 // adds alpha_k p_k, mode 2 adds the pending alpha_{k-1} p_{k-1} and then
 // alpha_k p_k, rounding after each add exactly like two updates.
 template <class V, class Dacc, int OPk>
-__global__ void __launch_bounds__(PB) k_update(OpArgs o, Launch L, V* __restrict__ x, V* __restrict__ r,
+__global__ void __launch_bounds__(PB, 6) k_update(OpArgs o, Launch L, V* __restrict__ x, V* __restrict__ r,
                                                const V* __restrict__ pc, const V* __restrict__ ppv,
                                                const V* __restrict__ q, double* __restrict__ x64, Parts P, int nbs,
-                                               int nbs2, SolveScalars* sc, int k, int fold, int mode, int npad) {
+                                               int nbs2, SolveScalars* sc, int k, int fold_, int mode, int npad) {
   if (sc->done) return;
-  double t[1], t2[1];
-  read_partials<1>(P.S, nbs, t);
-  read_partials<1>(P.S2, nbs2, t2);
-  t[0] += t2[0];
+  const bool fold = sizeof(V) == 4 && fold_;  // MIXED only
+  // One quad of 4 consecutive cells per thread and pass (one 16-byte access
+  // per FP32 vector, two per FP64 vector).  A pass' vectors are loaded at the
+  // end of the one before it, the first one's before the sums are read, and
+  // the masks one pass further ahead; the vectors of a quad are read only if
+  // it holds an unknown, and a quad of unknowns is stored whole, others cell
+  // by cell.  (Two quads a pass took registers for 8 FP64 waves a CU, four
+  // rounds of blocks; one takes 24: 100 -> 70 us FP64 at 256^3, 30 -> 20 at
+  // 133x131x124, FP32 57 -> 52 at 256^3.)
+  struct alignas(4 * sizeof(V)) Q4 { V e[4]; };
+  struct alignas(32) D4 { double e[4]; };
+  const int64_t c0 = chunk_begin(L);
+  const int64_t c1 = max(c0, (o.g.G < c0 + L.chunk) ? o.g.G : c0 + L.chunk);  // blocks past the grid: empty
+  const int64_t cq = c0 + ((c1 - c0) & ~(int64_t)3);                            // end of the whole quads
+  constexpr int64_t PASS = (int64_t)4 * PB;
+  auto mask_at = [&](int64_t b4) { return b4 < cq ? *(const uint32_t*)(o.nbm + b4) : 0u; };
+  Q4 pv = {}, p1 = {}, xv = {}, rv, qv;
+  D4 x64v = {};
+  auto load = [&](int64_t b4, uint32_t m) {
+    if (!(m & 0x40404040u)) return;
+    rv = *(const Q4*)(r + b4);
+    qv = *(const Q4*)(q + b4);  // q is only defined on the unknowns; used only there
+    if (mode != 0) {
+      pv = *(const Q4*)(pc + b4);
+      xv = *(const Q4*)(x + b4);
+      if (mode == 2) p1 = *(const Q4*)(ppv + b4);
+      if (fold) x64v = *(const D4*)(x64 + b4);
+    }
+  };
+  const int64_t base0 = c0 + 4 * (int64_t)threadIdx.x;
+  uint32_t m4 = mask_at(base0);
+  load(base0, m4);
+  uint32_t mn = mask_at(base0 + PASS);
+  double t[2];  // p.q of the tiles, of the slow rows
+  read_partials_of_two<1>(P.S, nbs, P.S2, nbs2, t);
+  t[0] += t[1];
   if (t[0] == 0.0 || bad(t[0])) {  // spray.cu:1654-1656: zp == 0 ends the solve
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       sc->done = 1;
@@ -870,81 +932,29 @@ __global__ void __launch_bounds__(PB) k_update(OpArgs o, Launch L, V* __restrict
     a_rz += (Dacc)rn * (Dacc)z;
     a_rr += (Dacc)rn * (Dacc)rn;
   };
-  // Quads of 4 consecutive cells per thread (one 16-byte access per FP32
-  // vector, two per FP64 vector), UQ quads per pass.  The masks of the next
-  // pass are loaded one pass ahead; the vectors of a quad are read only if it
-  // holds an unknown, and a quad of unknowns is stored whole, others cell by
-  // cell.
-  constexpr int UQ = 2;
-  struct alignas(4 * sizeof(V)) Q4 { V e[4]; };
-  struct alignas(32) D4 { double e[4]; };
-  const int64_t c0 = chunk_begin(L);
-  const int64_t c1 = max(c0, (o.g.G < c0 + L.chunk) ? o.g.G : c0 + L.chunk);  // blocks past the grid: empty
-  const int64_t cq = c0 + ((c1 - c0) & ~(int64_t)3);                            // end of the whole quads
-  constexpr int64_t PASS = (int64_t)4 * UQ * PB;
-  auto load_masks = [&](int64_t base, uint32_t (&m)[UQ]) {
+  for (int64_t b4 = base0; b4 < cq; b4 += PASS) {
+    const uint32_t un4 = m4 & 0x40404040u;
+    if (un4) {
+      // slow-row diagonals, for quads holding a slow row (the quad's other
+      // cells read its first element)
+      Q4 ds;
+      const bool slow = o.precond && (m4 & 0x80808080u);
 #pragma unroll
-    for (int u = 0; u < UQ; ++u) {
-      const int64_t b4 = base + (int64_t)u * 4 * PB;
-      m[u] = (b4 < cq) ? *(const uint32_t*)(o.nbm + b4) : 0u;
-    }
-  };
-  uint32_t mn[UQ];
-  load_masks(c0 + 4 * (int64_t)threadIdx.x, mn);
-  for (int64_t base = c0 + 4 * (int64_t)threadIdx.x; base < cq; base += PASS) {
-    uint32_t m4[UQ];
-#pragma unroll
-    for (int u = 0; u < UQ; ++u) m4[u] = mn[u];
-    Q4 pv[UQ] = {}, p1[UQ] = {}, xv[UQ] = {}, rv[UQ], qv[UQ], ds[UQ];
-    D4 x64v[UQ] = {};
-#pragma unroll
-    for (int u = 0; u < UQ; ++u) {
-      const int64_t b4 = base + (int64_t)u * 4 * PB;
-      if (m4[u] & 0x40404040u) {
-        rv[u] = *(const Q4*)(r + b4);
-        qv[u] = *(const Q4*)(q + b4);  // q is only defined on the unknowns; used only there
-        if (mode != 0) {
-          pv[u] = *(const Q4*)(pc + b4);
-          xv[u] = *(const Q4*)(x + b4);
-          if (mode == 2) p1[u] = *(const Q4*)(ppv + b4);
-          if (fold) x64v[u] = *(const D4*)(x64 + b4);
-        }
+      for (int e = 0; e < 4; ++e) {
+        const uint8_t nb = (uint8_t)(m4 >> (8 * e));
+        const bool sl = (nb & (NB_UNKNOWN | NB_SLOW)) == (NB_UNKNOWN | NB_SLOW);
+        ds.e[e] = slow ? dslow_at<V>(o, sl ? b4 + e : b4) : V(1);
       }
-    }
-    load_masks(base + PASS, mn);
-    // slow-row diagonals, for quads holding a slow row (the quad's other
-    // cells read its first element)
-#pragma unroll
-    for (int u = 0; u < UQ; ++u) {
-      const int64_t b4 = base + (int64_t)u * 4 * PB;
-      if (o.precond && (m4[u] & 0x80808080u)) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint8_t nb = (uint8_t)(m4[u] >> (8 * e));
-          const bool sl = (nb & (NB_UNKNOWN | NB_SLOW)) == (NB_UNKNOWN | NB_SLOW);
-          ds[u].e[e] = dslow_at<V>(o, sl ? b4 + e : b4);
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) ds[u].e[e] = V(1);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < UQ; ++u) {
-      const uint32_t un4 = m4[u] & 0x40404040u;
-      if (!un4) continue;
-      const int64_t b4 = base + (int64_t)u * 4 * PB;
       Q4 xo, ro;
       D4 x64o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const uint8_t nb = (uint8_t)(m4[u] >> (8 * e));
-        xo.e[e] = xv[u].e[e];
-        ro.e[e] = rv[u].e[e];
-        x64o.e[e] = fold ? x64v[u].e[e] : 0.0;
+        const uint8_t nb = (uint8_t)(m4 >> (8 * e));
+        xo.e[e] = xv.e[e];
+        ro.e[e] = rv.e[e];
+        x64o.e[e] = fold ? x64v.e[e] : 0.0;
         if (nb & NB_UNKNOWN)
-          cell(nb, pv[u].e[e], p1[u].e[e], xv[u].e[e], rv[u].e[e], qv[u].e[e], ds[u].e[e], x64o.e[e], xo.e[e],
-               ro.e[e], x64o.e[e]);
+          cell(nb, pv.e[e], p1.e[e], xv.e[e], rv.e[e], qv.e[e], ds.e[e], x64o.e[e], xo.e[e], ro.e[e], x64o.e[e]);
       }
       if (un4 == 0x40404040u) {
         st_nt4(r + b4, ro.e);
@@ -953,13 +963,16 @@ __global__ void __launch_bounds__(PB) k_update(OpArgs o, Launch L, V* __restrict
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if ((m4[u] >> (8 * e)) & NB_UNKNOWN) {
+          if ((m4 >> (8 * e)) & NB_UNKNOWN) {
             st_nt(r + b4 + e, ro.e[e]);
             if (mode != 0) st_nt(x + b4 + e, xo.e[e]);
             if (fold) st_nt(x64 + b4 + e, x64o.e[e]);
           }
       }
     }
+    m4 = mn;
+    load(b4 + PASS, m4);
+    mn = mask_at(b4 + 2 * PASS);
   }
   // cells after the last whole quad (grids whose size is not a multiple of 4)
   if (threadIdx.x < c1 - cq) {
