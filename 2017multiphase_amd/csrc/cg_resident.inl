@@ -717,9 +717,9 @@ __global__ void __launch_bounds__(RT)
   }
 }
 
-__global__ void k_res_clear(uint32_t* quit, SolveScalars* sc) {
+__global__ void k_res_clear(uint32_t* quit, uint32_t raised, SolveScalars* sc) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *quit = 0;
+    *quit = raised;
     sc->done = 0;
   }
 }
@@ -799,6 +799,8 @@ ResKernel<V, MIX> resident_kernel(int m) {
   return nullptr;
 }
 
+inline uint32_t* resident_quit(Ctx& c) { return (uint32_t*)(c.res_buf + 2 * RG * RWORDS); }
+
 // Queues a resident solve (after the masks).  False when it cannot run: the
 // grid does not fit, or the device cannot hold all blocks at once.
 template <class V, bool MIX>
@@ -812,7 +814,7 @@ bool resident_launch(Ctx& c, const OpArgs& o, const V* b, V* x, double* x64, dou
   const int64_t words = 2 * RG * RWORDS + 16 + 4 * c.res_cells;
   uint64_t* base = (uint64_t*)c.res_buf;
   a.rec = base;
-  a.quit = (uint32_t*)(base + 2 * RG * RWORDS);
+  a.quit = resident_quit(c);
   uint64_t* h = base + 2 * RG * RWORDS + 16;
   a.plane = (uint64_t)c.res_cells;
   a.hq[0] = h;
@@ -835,7 +837,8 @@ bool resident_launch(Ctx& c, const OpArgs& o, const V* b, V* x, double* x64, dou
     c.res_seq = 1;
   }
   a.seq0 = c.res_seq;
-  launch(c, "pcg_res_clear", dim3(1), dim3(64), 0, k_res_clear, a.quit, c.scal);
+  launch(c, "pcg_res_clear", dim3(1), dim3(64), 0, k_res_clear, a.quit, c.res_raise_quit ? 1u : 0u, c.scal);
+  c.res_raise_quit = false;
   OpArgs oc = o;
   SolveScalars* sc = c.scal;
   void* args[] = {(void*)&oc, (void*)&a, (void*)&b, (void*)&x, (void*)&x64, (void*)&sc, (void*)&tol, (void*)&cap,

@@ -1075,6 +1075,10 @@ mpf_status mpf_step(mpf_ctx* ctx, int32_t frame, mpf_step_info* info) {
   return pst;
 }
 
+// For tests, not in mpflip.h: the next resident pressure solve finds the flag
+// raised with which a block that waited too long leaves.
+void mpf_internal_raise_quit(mpf_ctx* ctx) { ctx->c.res_raise_quit = true; }
+
 mpf_status mpf_set_kernel_timing(mpf_ctx* ctx, int32_t on) {
   if (!ctx) return MPF_INVALID_ARG;
   ctx->c.flush_timing();

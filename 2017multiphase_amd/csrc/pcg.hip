@@ -2037,10 +2037,16 @@ __global__ void __launch_bounds__(PB) k_true_resid(OpArgs o, Launch L, const B* 
 }
 
 // Sum of the S partials into sc->rr_true (one block).
-__global__ void __launch_bounds__(PB) k_collect_rr(const double* __restrict__ S, int nb, SolveScalars* sc) {
+// quit: the resident solve's flag (null: another solve).  Raised, some block
+// left without its part of the result, whatever the others recorded.
+__global__ void __launch_bounds__(PB) k_collect_rr(const double* __restrict__ S, int nb, SolveScalars* sc,
+                                                   const uint32_t* __restrict__ quit) {
   double t[1];
   read_partials<1>(S, nb, t);
-  if (threadIdx.x == 0) sc->rr_true = t[0];
+  if (threadIdx.x == 0) {
+    sc->rr_true = t[0];
+    if (quit && *quit) sc->done = 0;
+  }
 }
 
 // r.r of a residual pass with four sums per block (the single-kernel form).
@@ -2185,13 +2191,13 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
     return converged ? MPF_OK : MPF_NO_CONVERGENCE;
   };
   // |b - A x|^2 in FP64 for the report
-  auto true_rr = [&]() -> bool {
+  auto true_rr = [&](const uint32_t* quit) -> bool {
     if (mixed)
       launch(c, "pcg_true_resid", dim3(L.nblk), dim3(PB), 0, k_true_resid<OPk, V, double>, o, L, b,
              (const double*)x64, P);
     else
       launch(c, "pcg_true_resid", dim3(L.nblk), dim3(PB), 0, k_true_resid<OPk, V, V>, o, L, b, (const V*)x, P);
-    launch(c, "pcg_collect", dim3(1), dim3(PB), 0, k_collect_rr, (const double*)P.S, L.nblk, c.scal);
+    launch(c, "pcg_collect", dim3(1), dim3(PB), 0, k_collect_rr, (const double*)P.S, L.nblk, c.scal, quit);
     return read_scalars(c);
   };
   if constexpr (OPk != OP_HEAT) {
@@ -2204,7 +2210,7 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
       queued = resident_launch<V, false>(c, o, b, x, nullptr, ref ? eps_abs : -1.0, tol, cap, R, bc);
     }
     if (queued) {
-      if (!true_rr()) return MPF_HIP_ERROR;
+      if (!true_rr(resident_quit(c))) return MPF_HIP_ERROR;
       c.res_seq = c.scal_host->done ? c.scal_host->res_seq : 0;
       if (c.scal_host->done) return report(c.scal_host->res_missed != 0, c.scal_host->res_restarts);
       // a block waited too long for the others: the launch form solves it
@@ -2427,7 +2433,7 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
   }
   if (mixed)
     launch(c, "pcg_fold", dim3(L.nblk), dim3(PB), 0, k_final_fold, L, G, (const uint8_t*)c.nbm, (float*)x, x64);
-  if (!true_rr()) return MPF_HIP_ERROR;
+  if (!true_rr(nullptr)) return MPF_HIP_ERROR;
   return report(true_missed, restarts);
 }
 
