@@ -21,9 +21,14 @@
 // number: a block writes for meeting s + 2 only after meeting s + 1, which no
 // block joins before it has read all of meeting s.  The block sums are added
 // by every block in the same fixed order, so all derive the same scalars bit
-// for bit.  Polls are bounded in time; a block that gives up raises a flag on
-// which all leave, and the host solves with the launch-per-iteration kernels.
-// The launch is cooperative: every block is resident before any polls.
+// for bit.  The launch is cooperative: every block is resident before any polls.
+// Polls are bounded in time; a block that gives up raises a flag (quit) on
+// which all leave.  In the last meeting no later one waits for a block that
+// gave up, and the others may end the solve without its tile: the flag outlives
+// the launch, and a result counts only while it is down (k_collect_rr).
+// Otherwise the launch-per-iteration kernels solve, then and in that context
+// from then on: blocks that cannot all run at once (two processes on one GPU,
+// half of each one's blocks running) would cost every solve the wait.
 //
 // Measured per iteration (one MI355X, launch form -> this one): FP32 with an
 // air ball 23.0 -> 4.8 us at 64^3, FP32 28.8 -> 9.5 us at 128^3 and 40.7 -> 19.2
@@ -802,12 +807,13 @@ ResKernel<V, MIX> resident_kernel(int m) {
 inline uint32_t* resident_quit(Ctx& c) { return (uint32_t*)(c.res_buf + 2 * RG * RWORDS); }
 
 // Queues a resident solve (after the masks).  False when it cannot run: the
-// grid does not fit, or the device cannot hold all blocks at once.
+// grid does not fit, the device cannot hold all blocks at once, or an earlier
+// one of this context was left by a block that waited too long.
 template <class V, bool MIX>
 bool resident_launch(Ctx& c, const OpArgs& o, const V* b, V* x, double* x64, double eps_abs, double tol, int cap, int R,
                      double bc) {
   ResArgs<V> a;
-  if (!c.res_buf || !resident_tile(c.g, c.res_blocks, (int)sizeof(V), MIX, a.t)) return false;
+  if (!c.res_buf || c.res_off || !resident_tile(c.g, c.res_blocks, (int)sizeof(V), MIX, a.t)) return false;
   const int64_t n = (int64_t)a.t.nblk * a.t.cells;
   if (n > c.res_cells) return false;
   // records, quit word, then q halos (two buffers of two planes), r and x64 halos

@@ -191,6 +191,7 @@ struct Ctx {
   int64_t res_cells = 0;
   int res_blocks = 0;
   uint32_t res_seq = 0;
+  bool res_off = false;         // a resident solve was left by a block that waited too long: none is tried again
   bool res_raise_quit = false;  // the next resident solve finds its quit flag raised (for tests)
   SolveScalars* scal = nullptr;
   SolveScalars* scal_host = nullptr;  // pinned

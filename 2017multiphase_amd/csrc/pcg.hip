@@ -2213,7 +2213,9 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
       if (!true_rr(resident_quit(c))) return MPF_HIP_ERROR;
       c.res_seq = c.scal_host->done ? c.scal_host->res_seq : 0;
       if (c.scal_host->done) return report(c.scal_host->res_missed != 0, c.scal_host->res_restarts);
-      // a block waited too long for the others: the launch form solves it
+      // a block waited too long for the others: the launch form solves it, and
+      // what follows (the GPU is shared, and each try would cost that wait)
+      c.res_off = true;
     }
   }
   // slow rows: list in cell order (positions from a scan into the cell-count scratch)

@@ -35,3 +35,26 @@ def test_result_of_a_solve_that_was_left_is_not_taken(pkg, precision):
         for f in ["PRESSURE"] + FACE:
             e = rel_l2(sim.get_field(f), want.get_field(f))
             assert e <= ((2e-3 if f == "PRESSURE" else 2e-4) if precision == pkg.FP32 else 2e-5), (f, e)
+
+
+def test_no_further_wait_after_a_solve_that_was_left(pkg):
+    """A context whose resident solve was left solves launch by launch from then
+    on, with the bits of the solve that took over; another context is not touched."""
+    say("solves after one with a raised flag")
+    cfg, fields = _system(pkg, (40, 44, 52), pkg.MIXED, True)
+    sim, other = pkg.Simulator(cfg), pkg.Simulator(cfg)
+    got = []
+    for turn in range(3):
+        if turn == 0:
+            sim.L.mpf_internal_raise_quit(sim.h)
+        sim.set_kernel_timing(True)
+        sim.reset_kernel_times()
+        assert _project(sim, fields)["converged"] == 1
+        assert ("pcg_resident" in sim.kernel_times()) == (turn == 0)
+        got.append([sim.get_field(f) for f in ["PRESSURE"] + FACE])
+    for later in got[1:]:
+        for a, b in zip(later, got[0]):
+            assert (a == b).all()
+    other.set_kernel_timing(True)
+    assert _project(other, fields)["converged"] == 1
+    assert "pcg_resident" in other.kernel_times()
