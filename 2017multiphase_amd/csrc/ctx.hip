@@ -11,6 +11,7 @@
 #include <new>
 
 #include "mpf_internal.h"
+#include "tiling.h"
 
 namespace mpf {
 
@@ -192,8 +193,8 @@ bool alloc_all(Ctx& c) {
   ok = ok && dalloc(c, dd, G); c.vq2 = dd;
   ok = ok && dalloc(c, dd, G); c.vp3 = dd;
   ok = ok && dalloc(c, c.nbm, G) && dalloc(c, c.dslow, G);
-  c.npart = 1024 * 48;  // solver partial sums (pcg.hip lays out regions of 1024-block slots)
-  ok = ok && dalloc(c, c.partials, c.npart) && dalloc(c, c.scal, 1) && dalloc(c, c.counters, NCOUNTERS);
+  c.part_blocks = tiling_region_blocks(c.g.nx, c.g.ny, c.g.nz);
+  ok = ok && dalloc(c, c.partials, 48 * (size_t)c.part_blocks) && dalloc(c, c.scal, 1) && dalloc(c, c.counters, NCOUNTERS);
   if (ok) {  // one block per CU
     int cus = 0, coop = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device) == hipSuccess &&

@@ -182,8 +182,8 @@ struct Ctx {
   uint8_t* nbm = nullptr;  // per-cell neighbour mask of the current solve
   double* dslow = nullptr;  // 1/diag of the current solve's slow rows (flags-dependent)
   double* vx64 = nullptr;
-  double* partials = nullptr;
-  int npart = 0;
+  double* partials = nullptr;  // solver partial sums: regions of part_blocks blocks (pcg.hip)
+  int part_blocks = 0;
   // resident solve (null when the grid does not fit): records, then six halo
   // arrays of res_cells words; res_blocks blocks can be resident together;
   // number of the next meeting (0: clear the words first)

@@ -31,6 +31,7 @@
 // Streaming kernels walk contiguous cell chunks, mapped so each XCD (blocks
 // are dispatched round-robin over the 8 XCDs) walks one contiguous slab.
 #include "mpf_internal.h"
+#include "tiling.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -40,7 +41,6 @@ namespace mpf {
 namespace {
 
 constexpr int PB = 512;        // threads per block
-constexpr int MAX_BLK = 1024;  // blocks per solver launch
 constexpr int MAX_RESTARTS = 50;  // MIXED: restarts from the FP64 true residual per solve
 constexpr int OP_UNIT = 0, OP_VARDENS = 1, OP_HEAT = 2;
 constexpr uint8_t NB_UNKNOWN = 64, NB_SLOW = 128;
@@ -437,21 +437,12 @@ __global__ void __launch_bounds__(PB) k_init(OpArgs o, Launch L, const V* __rest
   }
 }
 
-// ---- spmv tiling ----
-// (j, k) column tiles of TCELLS / TK rows of TK cells, TK = 128 or 64 by the
-// grid (make_tiling), with a one-cell ring in LDS.
-constexpr int TCELLS = 1024;                  // cells of a tile's plane
-constexpr int TK_WIDE = 128, TK_NARROW = 64;
+// ---- spmv tiling (tiling.h) ----
 constexpr int ST = 512;                       // threads per spmv block
 constexpr int RPT = TCELLS / ST;              // tile rows per thread (2)
 static_assert(2 * TK_WIDE + 2 * (TCELLS / TK_WIDE) <= ST && 2 * TK_NARROW + 2 * (TCELLS / TK_NARROW) <= ST,
               "one ring cell per thread");
 
-struct Tiling {
-  int ntj, ntk, seg, nblk;
-  int tk;   // cells of a tile along k (TK)
-  int ns5;  // single-kernel iteration: blocks of slow-row partials after the nblk tile blocks
-};
 // Block -> tile run.  Blocks are dispatched round-robin over the 8 XCDs, so
 // each XCD takes a contiguous run of tiles (its L2 sees neighbouring tiles);
 // inside a run the second half swaps neighbouring tiles, so the two blocks a
@@ -2080,39 +2071,8 @@ Launch make_launch(int64_t G) {
   return L;
 }
 
-// spmv tiles: TJ x TK (j, k) columns, planes split along i into runs so the
-// launch has about `blocks` blocks: one resident round on 256 CUs, i.e. as
-// many 512-thread blocks as fit a CU at the kernel's register use (three for
-// FP32 vectors without slow rows, two otherwise).
-Tiling make_tiling(const Grid& g, int blocks, int tk) {
-  Tiling t;
-  t.tk = tk;
-  t.ns5 = 0;
-  const int tj = TCELLS / tk;
-  t.ntj = (g.ny + tj - 1) / tj;
-  t.ntk = (g.nz + tk - 1) / tk;
-  const int tiles = t.ntj * t.ntk;
-  int nseg = blocks / tiles;
-  if (nseg < 1) nseg = 1;
-  if (nseg > g.nx) nseg = g.nx;
-  // a run's planes as FP64 values stay within 32-bit byte offsets
-  const int64_t most = std::max<int64_t>(1, 0xfffffff0ll / (8 * (int64_t)g.ny * g.nz) - 6);
-  if (nseg < (g.nx + most - 1) / most) nseg = (int)((g.nx + most - 1) / most);
-  t.seg = (g.nx + nseg - 1) / nseg;
-  nseg = (g.nx + t.seg - 1) / t.seg;
-  t.nblk = tiles * nseg;
-  return t;
-}
-
-// Wide tiles read whole 512-byte rows and fewer ring cells per plane; narrow
-// ones pad less where nz ends early in the last wide tile.  A launch costs
-// about (seg + 3) plane steps (three fill the pipeline), a narrow step up to
-// 8/7 of a wide one (105 us a narrow launch against 94 at 256^3, where both
-// run 32 planes; 56 against 64 at 192^3, 14 planes against 20, before the
-// plane loop lost its branches).
-Tiling make_tiling(const Grid& g, int blocks) {
-  const Tiling w = make_tiling(g, blocks, TK_WIDE), n = make_tiling(g, blocks, TK_NARROW);
-  return 8 * (n.seg + 3) < 7 * (w.seg + 3) ? n : w;
+Tiling make_tiling(const Grid& g, int blocks, bool by_offset) {
+  return mpf::make_tiling(g.nx, g.ny, g.nz, blocks, by_offset);
 }
 
 OpArgs make_op(Ctx& c, int precond, int opk) {
@@ -2165,7 +2125,8 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
   V* r = (V*)c.vr;
   V* pbuf[2] = {(V*)c.vp, (V*)c.vp2};
   V* q = (V*)c.vq;
-  Parts P{c.partials, c.partials + 2 * MAX_BLK, c.partials + 4 * MAX_BLK, c.partials + 6 * MAX_BLK};
+  const int RB = c.part_blocks;
+  Parts P{c.partials, c.partials + 2 * RB, c.partials + 4 * RB, c.partials + 6 * RB};
   const double eps_abs = 1e-2 * (double)G;
   const int R = c.cfg.refine_every > 0 ? c.cfg.refine_every : 20;
   int check = mixed ? R : c.cfg.check_every;
@@ -2234,7 +2195,7 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
            (const uint32_t*)slow_list, nslow, slow_b);
   // slow-row blocks: grid-stride over the list, at most MAX_BLK of them (the
   // single-kernel iteration sums their partials after its tile blocks, in a
-  // region that holds 2 * MAX_BLK blocks)
+  // region that holds 2 * RB blocks)
   int nsb = (int)((nslow + PB - 1) / PB);
   if (nsb > MAX_BLK) nsb = MAX_BLK;
     // the MIXED form without slow rows runs one kernel per iteration (k_cgf)
@@ -2242,7 +2203,9 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
   // without slow rows the fused iteration can form q_{k-1} again instead of
   // storing q (k_cgq, one 1024-thread block per CU; cfg.pcg_recompute_q)
   const bool qfree = fused && nslow == 0 && c.cfg.pcg_recompute_q;
-  Tiling T = qfree ? make_tiling(c.g, 256, TK_WIDE) : make_tiling(c.g, fused ? 512 : ((sizeof(V) == 4 && nslow == 0) ? 768 : 512));
+  Tiling T = qfree   ? mpf::make_tiling(c.g.nx, c.g.ny, c.g.nz, 256, TK_WIDE, false)
+             : fused ? make_tiling(c.g, FUSED_BLOCKS, true)
+                     : make_tiling(c.g, (sizeof(V) == 4 && nslow == 0) ? 768 : 512, false);
   T.ns5 = fused ? nsb : 0;
   const bool wide = T.tk == TK_WIDE;
   auto spmv = nslow > 0 ? (wide ? k_spmv<V, Dacc, OPk, true, TK_WIDE> : k_spmv<V, Dacc, OPk, true, TK_NARROW>)
@@ -2251,13 +2214,13 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
                            : (wide ? k_resid64<OPk, 0, TK_WIDE> : k_resid64<OPk, 0, TK_NARROW>);
   // the true-residual pass keeps two 512-thread blocks per CU (its own
   // tiling when k_cgq runs one block per CU); its partial count is Tr.nblk
-  Tiling Tr = qfree ? make_tiling(c.g, 512, TK_WIDE) : T;
+  Tiling Tr = qfree ? mpf::make_tiling(c.g.nx, c.g.ny, c.g.nz, 512, TK_WIDE, false) : T;
   Tr.ns5 = T.ns5;
   // U-slot partials: update and init write L.nblk, the residual pass T.nblk;
   // both pad to npad, the count the spmv sums
   int npad = L.nblk > T.nblk ? L.nblk : T.nblk;
   if (Tr.nblk > npad) npad = Tr.nblk;
-  if (npad > MAX_BLK) {
+  if (npad > RB) {
     c.err = "grid too large for the solver's reduction buffers";
     return MPF_INVALID_ARG;
   }
@@ -2278,8 +2241,8 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
       // p_k in pf[(k + 1) % 3]: a launch reads p_k-1 and p_k-2 and writes p_k
       float* pf[3] = {(float*)c.vp, (float*)c.vp2, (float*)c.vp3};
       // partial sums: per launch T.nblk tile blocks then T.ns5 slow-row blocks
-      double* S7[2] = {c.partials + 8 * MAX_BLK, c.partials + 22 * MAX_BLK};
-      double* Rs = c.partials + 36 * MAX_BLK;
+      double* S7[2] = {c.partials + 8 * RB, c.partials + 22 * RB};
+      double* Rs = c.partials + 36 * RB;
       // x advances every other launch (modes 2 and 3 of k_cgf), and fully
       // before each true-residual pass
       struct Iter {

@@ -18,3 +18,12 @@ def test_fastdiv_matches_integer_division(tmp_path):
                     "-I/opt/rocm/include"], check=True, capture_output=True)
     out = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0, out.stdout + out.stderr
+
+
+@pytest.mark.skipif(not shutil.which("g++"), reason="g++ not available")
+def test_solver_tiling_of_every_grid(tmp_path):
+    src = os.path.join(ROOT, "tests", "native", "tiling_check.cpp")
+    exe = str(tmp_path / "tiling_check")
+    subprocess.run(["g++", "-O2", "-std=c++17", src, "-o", exe], check=True, capture_output=True)
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout + out.stderr
