@@ -717,11 +717,11 @@ __global__ void k_zero6(Grid g, Grads6 gr) {
   const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (f < face_n(g, blockIdx.y % 3)) gr.out[blockIdx.y][f] = 0.0;
 }
-// g_uold = -alpha g_u
+// g_uold = -alpha g_u (nothing with alpha = 0, also of an infinite g_u)
 __global__ void k_adj_uold(Grid g, Grads6 gr, double alpha) {
   const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int q = blockIdx.y;
-  if (f < face_n(g, q % 3)) gr.out[q][f] = 0.0 - alpha * gr.in[q][f];
+  if (f < face_n(g, q % 3)) gr.out[q][f] = alpha != 0.0 ? 0.0 - alpha * gr.in[q][f] : 0.0;
 }
 
 __global__ void k_fill_d(int64_t n, double* __restrict__ a, double v) {
