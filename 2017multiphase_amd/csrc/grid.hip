@@ -1805,12 +1805,8 @@ __global__ void k_mc_density(McGrid m, Grid g2, const f3* __restrict__ pos, cons
 }  // namespace
 
 // ================= host stage drivers =================
-// n two-buffer passes, ping-ponging between phi and the scratch field (one
-// copy at the end when n is odd).
-// n passes ending in phi; the initial field is in c.ctmp when in_tmp (the
-// preparing kernel wrote it there, so an odd n needs no final copy)
-// n passes (odd) over one field or two: from tmp into phi and back, the last
-// into phi.  flags: two sets of tile flags.
+// N two-buffer passes over one field or two: from tmp into phi and back, an odd
+// number so that the last is into phi.  flags: two sets of tile flags.
 struct SweepJob {
   float* phi;
   float* tmp;
@@ -1818,19 +1814,21 @@ struct SweepJob {
   int typeflag;
   uint8_t* flags;
 };
-static void sweep_n(Ctx& c, const SweepJob* jobs, int njobs, int n) {
+template <int N>
+static void sweep_n(Ctx& c, const SweepJob* jobs, int njobs) {
+  static_assert(N % 2 == 1, "the last pass writes phi");
   const uint32_t ntj = (uint32_t)((c.g.ny + SW_J - 1) / SW_J), ntk = (uint32_t)((c.g.nz + SW_K - 1) / SW_K);
   const int64_t nt = sweep_tiles(c.g);
   const int64_t nwaves = (nt + SW_L - 1) / SW_L;
-  for (int it = 0; it < n; ++it) {
+  for (int it = 0; it < N; ++it) {
     SweepPass p[2];
     for (int q = 0; q < 2; ++q) {
       const SweepJob& j = jobs[q < njobs ? q : 0];
       p[q] = SweepPass{(it & 1) ? j.phi : j.tmp, (it & 1) ? j.tmp : j.phi, j.mark, j.typeflag,
                        it == 0 ? nullptr : j.flags + ((it - 1) & 1) * nt, j.flags + (it & 1) * nt};
     }
-    launch(c, "sweep", dim3((unsigned)((nwaves + 3) / 4), njobs), dim3(256), 0, k_sweep, c.g, p[0], p[1], ntj, ntk,
-           (uint32_t)nt);
+    launch(c, njobs == 1 ? "sweep_one" : "sweep", dim3((unsigned)((nwaves + 3) / 4), njobs), dim3(256), 0, k_sweep,
+           c.g, p[0], p[1], ntj, ntk, (uint32_t)nt);
   }
 }
 
@@ -1844,9 +1842,9 @@ static void redistance(Ctx& c) {
   const SweepJob jobs[2] = {{c.lsfluid, c.ctmp, c.mark, FLUID, c.sflag},
                             {c.lsair, c.ftmp[0], mark2, FLUID, c.sflag + 2 * sweep_tiles(c.g)}};
   launch(c, "ls_prepare", dim3(nblocks(G, 256), 2), dim3(256), 0, k_ls_prepare<false>, G, p, c.g.h);
-  sweep_n(c, jobs, 2, 5);
+  sweep_n<5>(c, jobs, 2);
   launch(c, "ls_prepare", dim3(nblocks(G, 256), 2), dim3(256), 0, k_ls_prepare<true>, G, p, c.g.h);
-  sweep_n(c, jobs, 2, 5);
+  sweep_n<5>(c, jobs, 2);
 }
 
 // Brick summary of the occupancy masks (after every change of the masks).
@@ -1948,7 +1946,7 @@ void run_solid_phi_and_velocity(Ctx& c) {
   launch(c, "init_solid_phi", dim3(nblocks(G, 256)), dim3(256), 0, k_init_solid_phi, G, (const uint8_t*)c.cmask,
          c.ctmp, (float)(3 * c.g.nx));
   const SweepJob job{c.phisolid, c.ctmp, c.mark, -1, c.sflag};
-  sweep_n(c, &job, 1, 3);
+  sweep_n<3>(c, &job, 1);
   // solid velocity only where the collision response can read it
   p2g_liquid(c, c.su, nullptr, c.phisolid, (float)(3 * c.g.nx));
 }
@@ -1964,7 +1962,7 @@ void run_extrapolate_bc(Ctx& c, bool recompute_phi) {
            tmp2, (int8_t)FLUID, (float)(c.g.nx * 3));
     const SweepJob jobs[2] = {{c.phiair, c.ctmp, c.mark, AIR, c.sflag},
                               {c.phifluid, tmp2, c.mark, FLUID, c.sflag + 2 * sweep_tiles(c.g)}};
-    sweep_n(c, jobs, 2, 3);
+    sweep_n<3>(c, jobs, 2);
   }
   // Two passes: u -> scratch, scratch -> u; the first records per-tile changes
   // (a flag set per field), the second skips the tiles they leave unchanged.

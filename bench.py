@@ -69,6 +69,8 @@ KERNEL_BYTES = {
     "correct_pos": (0, 0, 25),
     # sweep of two fields: each 4 read, mark 1, 4 written
     "sweep": (18, 0, 0),
+    # the same of one field (solid distance)
+    "sweep_one": (9, 0, 0),
     # extrapolation pass of six face fields: each u 4, out 4, ls 2x4, mark 2
     "sweep_u": (108, 0, 0),
 }
