@@ -30,14 +30,23 @@
 // from then on: blocks that cannot all run at once (two processes on one GPU,
 // half of each one's blocks running) would cost every solve the wait.
 //
-// Measured per iteration (one MI355X, launch form -> this one): FP32 with an
-// air ball 23.0 -> 4.8 us at 64^3, FP32 28.8 -> 9.5 us at 128^3 and 40.7 -> 19.2
-// at 144^3; FP64 with six air balls 46.1 -> 12.7 us at 96^3, without 44.3 -> 25.0
-// at 128^3; MIXED 20.9 -> 6.0 us at 64^3, 23.1 -> 12.4 at 128^3 and 33.0 -> 26.9
-// at 132^3, true residuals included.  About 4.5 us is the meeting (two trips through memory, the sums
-// and the scalars; 32 or 200 blocks differ by 0.4 us), the rest grows with the
-// cells per thread and is vector arithmetic and LDS.  Every grid that fits
-// gained, so the rule is that it fits (resident_tile).
+// Measured per iteration (one MI355X, whole solves to 1e-6, launch form -> this
+// one; true residuals included; in brackets with six air balls):
+//   FP32   64^3 16.0 -> 4.3 us (19.8 -> 4.5), 128^3 26.2 -> 9.2 (29.4 -> 13.0),
+//          144^3 40.0 -> 21.4 (43.2 -> 27.7)
+//   FP64   64^3 17.3 -> 6.4 (23.8 -> 6.4), 96^3 25.6 -> 11.0 (33.5 -> 12.5),
+//          128^3 36.4 -> 25.0 (45.9 -> 31.5)
+//   MIXED  64^3 12.7 -> 5.4 (18.4 -> 5.6), 128^3 20.7 -> 12.0 (27.0 -> 17.7),
+//          130^3 29.9 -> 19.3 (37.0 -> 28.2), 133^3 29.9 -> 26.2 (36.6 -> 36.0),
+//          120 x 128 x 150 27.2 -> 26.2 (33.9 -> 36.4)
+// About 4.5 us is the meeting (two trips through memory, the sums and the
+// scalars; 32 or 200 blocks differ by 0.4 us), the rest grows with the cells
+// per thread and is vector arithmetic, LDS and, in the larger columns, spilled
+// registers (RES_M).  So the rule is that the grid fits (resident_tile).  At
+// its upper end, 12 cells a thread in the MIXED form (131^3 to 133^3 and
+// ragged grids of as many cells), the two forms are about equal: this one takes
+// 3 to 15% less without air, 2% less to 7% more with it, and which of them a
+// solve is shows only after the form is chosen.
 
 constexpr int RT = 1024;  // threads per block
 constexpr int RG = 256;   // most blocks
@@ -231,14 +240,14 @@ __device__ __forceinline__ bool grid_meet(const double (&v)[8], uint32_t seq, ui
 // the criterion (FP32 and FP64 forms), or of the FP64 true residual of x
 // (MIXED form).
 // Registers are what a larger column runs out of: the FP64 form keeps 1/diag
-// in LDS where there is room (T.dl, T.dr) and looks it up by the open faces of
-// a cell, or in memory for a slow row, elsewhere, and x lives in LDS (XL) in
-// the larger columns, where x64 of the MIXED form (always in LDS) leaves the
-// room.  The face weights of a slow row are read res_nbf at a time: one by one
-// they were a chain of up to six round trips (FP64 at 96^3 with bubbles 15.7 us
-// an iteration, 12.9 so, 12.7 with 1/diag in LDS, which at 112^3 takes 23.9 to
-// 20.9; MIXED at 128^3 with bubbles 25.4 -> 17.8); all six at once spill in the
-// larger columns.
+// in LDS where there is room (T.dl, T.dr; up to six cells) and looks it up by
+// the open faces of a cell, or in memory for a slow row, elsewhere, and x lives
+// in LDS (XL) in the larger columns, where x64 of the MIXED form (always in
+// LDS) leaves the room.  The face weights of a slow row are read res_nbf at a
+// time: one by one they were a chain of up to six round trips (FP64 at 96^3
+// with bubbles 15.7 us an iteration, 12.9 so, 12.7 with 1/diag in LDS, which at
+// 112^3 takes 23.9 to 20.9; MIXED at 128^3 with bubbles 25.4 -> 17.8); all six
+// at once spill more in the larger columns (FP64 128^3 24.4 -> 32.3 us).
 constexpr bool res_xl(int m, bool d64, bool mix) { return d64 ? m >= 3 : mix ? m == 8 : m >= 8; }
 constexpr int res_nbf(int m, bool d64, bool mix) { return m <= (d64 ? 4 : mix ? 6 : 8) ? 6 : 3; }
 template <class V, bool MIX, int M, int MJ>
@@ -732,8 +741,14 @@ __global__ void k_res_words(uint64_t* w, int64_t n) {  // no word carries a meet
   for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) w[q] = 0;
 }
 
-// Compiled sizes: cells and j ring cells per thread.  The register file holds
-// 12 FP32 or 8 FP64 cells (r, q, x, p, 1/diag) per thread at 1024 threads per CU.
+// Compiled sizes: cells and j ring cells per thread.  1024 threads a CU have
+// 128 vector registers each.  r, q, p and, in FP32 and MIXED, 1/diag are in
+// registers, x too where it is not in LDS (res_xl); what does not fit goes
+// through scratch memory in every iteration.  The compiler spills, at 3, 4, 6,
+// 8, 10 and 12 cells, 0, 0, 9, 28, 174 and 234 registers (FP32; up to 204
+// bytes a lane), 4, 8, 65, 72, 199 and 278 (MIXED; up to 332 bytes) and 4, 18,
+// 80 and 141 (FP64; up to 224 bytes): part of the step from 12.0 to 19.3 us
+// between 128^3 and 130^3 in the MIXED form (8 and 10 cells).
 constexpr int RES_NM = 8;
 constexpr int RES_M[RES_NM] = {1, 2, 3, 4, 6, 8, 10, 12}, RES_MJ[RES_NM] = {1, 1, 2, 2, 3, 3, 4, 4};
 constexpr int RES_NM64 = 6;

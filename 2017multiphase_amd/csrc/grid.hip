@@ -1424,8 +1424,8 @@ __global__ void k_heat_code(Grid g, const int8_t* __restrict__ mark, uint16_t* _
 }
 
 // One Jacobi pass: the diagonal h^2/(alpha_m dt) + 6, less one per Neumann
-// neighbour (each subtraction of 1 is exact, so the count is subtracted at
-// once); x of the open neighbours added to b in face order.  Four cells per
+// neighbour (subtracted at once: below 2^53 every subtraction of 1 is exact);
+// x of the open neighbours added to b in face order.  Four cells per
 // thread, their loads in flight together, and the six diagonals from the host:
 // 256^3 72 -> 59 us a pass, where every block of 256 cells had formed a
 // table of them.

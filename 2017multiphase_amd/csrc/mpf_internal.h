@@ -159,7 +159,7 @@ struct Ctx {
   bool own_sort = false;
 
   // cells
-  uint32_t* count = nullptr;  // per-cell counts, then scatter cursors
+  uint32_t* count = nullptr;  // per-cell counts; positions of scanned cell flags (slow rows, nucleation)
   uint32_t* cstart = nullptr;
   uint32_t* cend = nullptr;
   uint8_t* cmask = nullptr;
@@ -171,7 +171,7 @@ struct Ctx {
   float* ctmp = nullptr;  // scratch cell field for two-buffer sweeps
   float* sf = nullptr;    // surface tension force per cell
   uint8_t* sflag = nullptr;  // per-tile change flags: 2 x sweep_tiles (eikonal passes), then face_tiles of
-                             // each axis (first extrapolation pass)
+                             // each axis and phase (first extrapolation pass; eikonal passes of a second field)
   void* div = nullptr;    // float, or double under MPF_FP64
   void* press = nullptr;  // float under MPF_FP32, else double
   float *tp = nullptr, *tpchange = nullptr, *tsave = nullptr;

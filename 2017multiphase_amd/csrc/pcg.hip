@@ -9,8 +9,8 @@
 // Two kernels per iteration, both HBM-bound:
 //   spmv   : p_k = z_k + beta p_{k-1} (z = r * diag^-1), written to the other
 //            p buffer; q = A p_k; p.q                       -> alpha
-//            2.5-D tiling: a block owns a 16 x 64 (j, k) column tile over a
-//            run of planes along i; each p_k is formed once, the current
+//            2.5-D tiling: a block owns a (j, k) column tile (8 x 128 or
+//            16 x 64 cells, tiling.h) over a run of planes along i; each p_k is formed once, the current
 //            plane (with a one-cell ring) sits in LDS for the j/k
 //            neighbours and the i neighbours stay in registers.
 //   update : x += alpha p_k ; r -= alpha q ; r.z ; r.r   -> beta, convergence
@@ -1287,7 +1287,7 @@ __device__ __forceinline__ CgScalars cg_scalars(CgSums& s, int first, const doub
   return CgScalars{ald, be, stop, nonfin, zero_pq};
 }
 
-// ---- single-kernel iteration (MIXED form, solves without slow rows) ----
+// ---- single-kernel iteration (MIXED form) ----
 // One launch per iteration k does what update(k-1) and spmv(k) do: with
 // alpha_{k-1} = (r.z)_{k-1} / (p.q)_{k-1} it forms r_k = r_{k-1} - alpha q_{k-1},
 // advances x by alpha p_{k-1}, and forms p_k = z_k + beta p_{k-1} and
@@ -2198,7 +2198,8 @@ int cg_solve(Ctx& c, const V* b, V* x, double* x64, bool ref, int precond, int c
   // region that holds 2 * RB blocks)
   int nsb = (int)((nslow + PB - 1) / PB);
   if (nsb > MAX_BLK) nsb = MAX_BLK;
-    // the MIXED form without slow rows runs one kernel per iteration (k_cgf)
+  // the MIXED form runs one kernel per iteration (k_cgf), and a second one over
+  // the slow rows where there are any
   const bool fused = std::is_same<V, float>::value && OPk != OP_HEAT && mixed && !ref;
   // without slow rows the fused iteration can form q_{k-1} again instead of
   // storing q (k_cgq, one 1024-thread block per CU; cfg.pcg_recompute_q)

@@ -17,7 +17,7 @@
 //  3. scatter: cell start plus rank (without a context, which has no room for
 //     the ranks: one more atomic per run);
 //  4. per-cell segment sort of the permutation (runs from different waves can
-//     interleave within a cell): a register sorting network for <=16 entries;
+//     interleave within a cell): a register sorting network for <=32 entries;
 //  5. gather of the 45-byte particle record into the other buffer.
 #include <mutex>
 
@@ -343,8 +343,11 @@ __global__ void k_scan_blocks(uint32_t* blk, int64_t nb) {
   if (threadIdx.x == 0) blk[nb] = carry;
 }
 
-// 23.0 us with one against 25.2 with four at 200k particles, 44.3 and 44.5 at
-// 1.2M, 75.2 and 74.7 at 2.9M, 988 and 895 at 45M (the sort without a context).
+// The whole sort without a context: 23.0 us with one against 25.2 with four at
+// 200k particles, 44.3 and 44.5 at 1.2M, 75.2 and 74.7 at 2.9M, 988 and 895 at
+// 45M.  The count with ranks of the sort with one: 6.4 and 7.4 us at 170k, 16.3
+// and 17.4 at 1.4M, 27.8 and 28.0 at 2.7M, 49.3 and 46.6 at 4.7M, 413 and 347
+// at 44M.
 constexpr int64_t HC_MANY = 2500000;
 
 // The exclusive scan of in, tile by tile.  blk: the tiles' exclusive prefixes

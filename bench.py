@@ -44,7 +44,7 @@ KERNEL_BYTES = {
     "pcg_update": (1, 20, 0),
     # mask 1 per cell; b 4, x64 8, x 4 read, r 4 written per unknown
     "pcg_resid64": (1, 20, 0),
-    # one-kernel iteration (MIXED form without slow rows): mask 1 per cell;
+    # one-kernel iteration (MIXED form; slow rows by a kernel of their own): mask 1 per cell;
     # per unknown r, q, p_k-1 read and r, q, p_k written (24), and x advanced
     # every other launch (read, written, p_k-2 read: 12), fully before each
     # true residual (x 8) and folded into x64 after it (x64 16 more): over a
